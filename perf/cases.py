@@ -426,11 +426,11 @@ def work(case):
         return dict(bytes=49.0 * sites + 8.0 * pairs, flops=(100.0 + MLP_FLOPS) * pairs)
     if kind == "table":
         # (7,5) and (8,6) tubes of 10 unit cells; per atom pair the distance, its inverse root
-        # and a complex multiply-add for each of about eight momenta
-        atoms = [2180.0, 2960.0]
+        # and a complex multiply-add for each of about five momenta
+        atoms = [2180.0, 1480.0]
         nodes = case["n_theta"] * case["n_z"] * case["n_a1"] * case["n_a2"]
         return dict(bytes=8.0 * nodes + 160.0 * sum(atoms),
-                    flops=nodes * atoms[case["donor"]] * atoms[case["acceptor"]] * (16 + 4 * 8))
+                    flops=nodes * atoms[case["donor"]] * atoms[case["acceptor"]] * (16 + 4 * 5))
     steps = case["epochs"] * (case["rows"] // case["batch"])
     rows = steps * case["batch"]
     return dict(bytes=68.0 * case["rows"] + 36.0 * rows + steps * 51_841 * 24.0,
