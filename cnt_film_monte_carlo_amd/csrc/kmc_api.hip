@@ -75,6 +75,7 @@ struct kmc_ctx {
   kmc_config cfg{};
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  int n_cu = 1;  // compute units of the device
   std::string err;
 
   // sites
@@ -485,6 +486,8 @@ int kmc_create(const kmc_config* cfg, kmc_ctx** out) {
   c->cfg = *cfg;
   hipError_t e = hipSetDevice(cfg->device);
   if (e == hipSuccess) e = scratch_setup(cfg->device);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, cfg->device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&c->ev0);
   if (e == hipSuccess) e = hipEventCreate(&c->ev1);
@@ -1269,7 +1272,11 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
       }
       KMC_HIP(c, hipEventRecord(c->hop_ev[2 * launches], c->stream));
     }
-    KMC_HIP(c, launch_hop(a, count, sample, trace, fly, c->stream));
+    if (!fly && hop_rows_pays(movable, c->n_cu))
+      KMC_HIP(c, launch_hop_rows(a, movable, (uint32_t)(c->n_units / ROW_UNITS), c->n_cu, count,
+                                 sample, trace, c->stream));
+    else
+      KMC_HIP(c, launch_hop(a, count, sample, trace, fly, c->stream));
     if (c->time_hops) KMC_HIP(c, hipEventRecord(c->hop_ev[2 * launches + 1], c->stream));
     done += sub;
     ++launches;

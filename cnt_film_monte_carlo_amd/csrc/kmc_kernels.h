@@ -118,6 +118,8 @@ struct hop_args {
   // k_hop: positions [0, *n_alive) of perm (the idle excitons sorted after them are left out);
   // null: all v.x.n
   const uint32_t* n_alive;
+  // k_hop_rows: block lines counted in a workgroup's LDS window (32-bit counters), out of n_lines
+  uint32_t win_lines, n_lines;
 };
 
 struct ens_args {
@@ -218,6 +220,11 @@ hipError_t launch_mask_count(int64_t nnz, const uint8_t* cls, const uint8_t* mas
                              hipStream_t st);
 hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bool fly,
                       hipStream_t st);
+// The hop loop for launches of few excitons (k_hop_rows).  `movable`, the excitons expected to
+// move, decides and sizes the grid; any number is handled.  n_lines = block lines of the film.
+bool hop_rows_pays(int64_t movable, int n_cu);
+hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
+                           bool sample, bool trace, hipStream_t st);
 // links[i] = {line of left | drain bit, line of right | drain bit}, LINK_NONE for a tube end
 hipError_t launch_links(int64_t n, const int32_t* left, const int32_t* right, const uint8_t* flags,
                         const int64_t* roff, const site_hdr* hdr, uint2* links, hipStream_t st);

@@ -12,6 +12,9 @@
 // it bit for bit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <utility>
+
 #include "kmc_internal.h"
 #include "kmc_kernels.h"
 #include "philox.h"
@@ -1246,6 +1249,375 @@ __global__ __launch_bounds__(256, 4) void k_hop(hop_args a) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Few excitons (k_hop_rows).  With less than a wave per SIMD, k_hop's iteration takes its own
+// latency: LDS round trips, lane exchanges, ten Philox rounds and a logarithm one after another
+// in a single wave, ~3,500 cycles per hop, of which the row load itself is hidden; the chip is
+// idle.  What bounds this form is the same chain, shortened: ~1,300 cycles per hop, a quarter of
+// them the row's L2 latency (1,000 excitons on 5,000 sites, 1,250 hops: 2.19 -> 0.74 ms; 16,384
+// excitons on 76,543 sites: 2.03 -> 0.94 ms).  Each
+// exciton has a row of 16 lanes, four excitons to a wave.  The lanes hold the exciton's 128-byte
+// block line between them (8 bytes each), so a selection is a comparison per lane and a count of
+// the ballot's bits, with DPP row broadcasts instead of LDS staging.  Only the chain that leads
+// from row to row runs hop by hop; a batch of ROW_BATCH = 16 hops then has its draws, dwells and
+// displacements computed side by side, lane j for hop j, and folded into the exciton's sums in
+// hop order (the operations and their order are those of hop_wave, so are the bits).  Hops
+// selected past t_max are dropped when the batch is folded.
+constexpr uint32_t ROW_BATCH = 16;
+
+struct __align__(16) batch_lds {
+  uint4 reached[4][ROW_BATCH][2];  // per exciton and hop: {n, site, Gamma}, {x, y, z, -} of the row
+  double inc[4][ROW_BATCH][4];     // dwell, displacement x, y, z of the hop
+};
+
+// Value of lane L of the lane's row of 16 (v_mov_b32 with row_newbcast).
+template <int L>
+__device__ __forceinline__ uint32_t row_bcast(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + L, 0xF, 0xF, true);
+}
+template <int L>
+__device__ __forceinline__ double row_bcast(double x) {
+  return __hiloint2double((int)row_bcast<L>((uint32_t)__double2hiint(x)),
+                          (int)row_bcast<L>((uint32_t)__double2loint(x)));
+}
+
+// LDS written by some lanes of the wave and read by others: in order within the wave, which
+// the compiler must keep.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The chain of one batch.
+struct row_chain {
+  uint2 raw;        // the lane's 8 bytes of the current row's first line
+  uint2 more;       // and of its second line, for a row word with TGT_WIDE_BIT
+  uint32_t W;       // its row word
+  uint32_t cnt;     // hops selected in this batch
+  bool run;
+  uint32_t my_tg, my_W;  // lane j: target word and departure row word of hop j
+};
+
+// The lines of row word c.W, 8 bytes per lane.
+__device__ __forceinline__ void load_lines(const net_view& v, row_chain& c, uint32_t l) {
+  const uint32_t off = (c.W & TGT_LINE_MASK) * (uint32_t)(16u * ROW_UNITS) + 8u * l;
+  const char* b = reinterpret_cast<const char*>(v.blocks);
+  c.raw = *reinterpret_cast<const uint2*>(b + off);
+  if (c.W & TGT_WIDE_BIT) c.more = *reinterpret_cast<const uint2*>(b + off + 16u * ROW_UNITS);
+}
+
+template <int J>
+__device__ __forceinline__ void row_step(const net_view& v, row_chain& c, uint32_t e, uint64_t h0,
+                                         uint32_t left, double r_sel, uint32_t l, uint32_t g,
+                                         batch_lds* s) {
+#pragma clang fp contract(off)
+  if (J > 0) {
+    // the row that hop J - 1 reached: header and position (lanes 0, 1, 14, 15)
+    if (l < 2u || l >= 14u) reinterpret_cast<uint2*>(&s->reached[g][J > 0 ? J - 1 : 0][0])[l & 3u] = c.raw;
+  }
+  const uint32_t n = row_bcast<0>(c.raw.x);
+  const double mine = __hiloint2double((int)c.raw.y, (int)c.raw.x);
+  const double gamma = row_bcast<1>(mine);
+  const bool can = c.run && (uint32_t)J < left && !trapped(n, gamma);
+  // the lanes 2..9 hold the inline cumulative rates: their count <= dice is the selected entry
+  const double dice = div_rand_max(gamma * row_bcast<J>(r_sel));
+  const uint64_t le = __ballot(mine <= dice);
+  uint32_t idx = (uint32_t)__popc((uint32_t)(le >> (16u * g)) & 0x3FCu);
+  // targets 0..7 sit two to a lane in the lanes 10..13
+  const int src = (int)(4u * (16u * g + 10u + ((idx & 7u) >> 1)));
+  const uint32_t t0 = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)c.raw.x);
+  const uint32_t t1 = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)c.raw.y);
+  uint32_t tg = (idx & 1u) ? t1 : t0;
+  const bool wide = can && idx >= ROW_INLINE;
+  if (__ballot(wide) != 0ull) {
+    // the continuation line came with the first one: cum[8..n), then tgt[8..n), of a row with up
+    // to 18 entries
+    const uint32_t m = n - ROW_INLINE;
+    const bool one = m <= 10u;
+    const uint64_t lw = __ballot(wide && one && l + 1u < m &&
+                                 __hiloint2double((int)c.more.y, (int)c.more.x) <= dice);
+    const uint32_t word = 2u * m + (uint32_t)__popc((uint32_t)(lw >> (16u * g)) & 0xFFFFu);
+    const int at = (int)(4u * (16u * g + ((word >> 1) & 15u)));
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)c.more.x);
+    const uint32_t w1 = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)c.more.y);
+    if (wide) tg = (word & 1u) ? w1 : w0;
+    // longer rows sixteen entries at a time
+    const char* ce = reinterpret_cast<const char*>(v.blocks) +
+                     ((size_t)(c.W & TGT_LINE_MASK) + 1u) * (16u * ROW_UNITS);
+    bool left_over = wide && !one;
+    for (uint32_t q = 0; __ballot(left_over) != 0ull; q += 16u) {
+      const uint32_t k = q + l;
+      double ck = INFINITY;
+      uint32_t tk = 0u;
+      if (left_over && k < m) {
+        if (k + 1u < m) ck = *reinterpret_cast<const double*>(ce + 8u * (size_t)k);
+        tk = *reinterpret_cast<const uint32_t*>(ce + 8u * (size_t)m + 4u * (size_t)k);
+      }
+      const uint64_t lk = __ballot(ck <= dice);
+      const uint32_t add = (uint32_t)__popc((uint32_t)(lk >> (16u * g)) & 0xFFFFu);
+      const uint32_t tw =
+          (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4u * (16u * g + (add & 15u))), (int)tk);
+      if (left_over && add < 16u) {
+        tg = tw;
+        left_over = false;
+      }
+    }
+  }
+  uint32_t Wn = tg & ~EDGE_DRAIN_BIT;
+  if (can && (tg & EDGE_DRAIN_BIT))
+    Wn = v.src_roff[r31(draw4(v.seed, e, h0 + (uint32_t)J, STREAM_REINJECT).v[0]) % v.n_src];
+  if (l == (uint32_t)J) {
+    c.my_tg = tg;
+    c.my_W = c.W;
+  }
+  c.run = can;
+  if (can) {
+    c.W = Wn;
+    ++c.cnt;
+    load_lines(v, c, l);
+  }
+}
+
+template <int... J>
+__device__ __forceinline__ void row_steps(std::integer_sequence<int, J...>, const net_view& v,
+                                          row_chain& c, uint32_t e, uint64_t h0, uint32_t left,
+                                          double r_sel, uint32_t l, uint32_t g, batch_lds* s) {
+  (row_step<J>(v, c, e, h0, left, r_sel, l, g, s), ...);
+}
+
+// Visit hash over the sites the batch's hops reached, in hop order (none of them a drain).
+template <int... J>
+__device__ __forceinline__ uint64_t row_hash(std::integer_sequence<int, J...>, uint64_t hs,
+                                             uint32_t site, uint32_t cnt) {
+  ((hs = (uint32_t)J < cnt ? (hs ^ (uint64_t)row_bcast<J>(site)) * FNV_PRIME : hs), ...);
+  return hs;
+}
+
+template <bool COUNT, bool SAMPLE, bool TRACE>
+__device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool valid,
+                                         uint64_t hop_budget, double t_max, const trace_view& tv,
+                                         batch_lds* s, uint32_t lane, uint32_t* win,
+                                         uint32_t win_base, uint32_t win_lines) {
+#pragma clang fp contract(off)
+  using hops16 = std::make_integer_sequence<int, (int)ROW_BATCH>;
+  const uint32_t l = lane & 15u, g = lane >> 4;
+  // the exciton's state, the same in its 16 lanes
+  double t = INFINITY, dx = 0.0, dy = 0.0, dz = 0.0;
+  uint64_t h = 0, hs = 0;
+  uint32_t nd = 0, k = 0;
+  int64_t tr = 0;
+  row_chain c{};
+  if (valid) {
+    t = v.x.t_next[e];
+    h = v.x.hops[e];
+    dx = v.x.dx[e];
+    dy = v.x.dy[e];
+    dz = v.x.dz[e];
+    nd = v.x.drains[e];
+    hs = v.x.hash[e];
+    if (SAMPLE) k = v.x.k_rec[e];
+    if (TRACE && e < tv.n_trace) tr = tv.tr_n[e];
+    const uint32_t R0 = (uint32_t)v.roff[v.x.site[e]];
+    c.W = row_word(R0, v.blocks[(size_t)ROW_UNITS * R0].x);
+  }
+  load_lines(v, c, l);
+  uint32_t n = row_bcast<0>(c.raw.x), site = row_bcast<0>(c.raw.y);
+  double gamma = row_bcast<1>(__hiloint2double((int)c.raw.y, (int)c.raw.x));
+  float px = __uint_as_float(row_bcast<14>(c.raw.x)), py = __uint_as_float(row_bcast<14>(c.raw.y)),
+        pz = __uint_as_float(row_bcast<15>(c.raw.x));
+  const uint64_t h_end = h + hop_budget;
+  const size_t E = v.x.n;
+  double t_rec = INFINITY;
+  if (SAMPLE && k < (uint32_t)v.n_bins) t_rec = (double)(k + 1u) * v.dt_sample;
+  uint32_t* cbase = COUNT ? v.site_count + (size_t)xcd_id() * v.count_stride : nullptr;
+  // the MSD records that fall due before the pending hop at t
+  auto records = [&]() {
+    while (t_rec < t) {
+      const size_t r = (size_t)(k - (uint32_t)v.bin0) * E + e;
+      if (l == 0u) {
+        v.rec_dx[r] = dx;
+        v.rec_dy[r] = dy;
+        v.rec_dz[r] = dz;
+        v.rec_drain[r] = nd;
+      }
+      ++k;
+      t_rec = k < (uint32_t)v.n_bins ? (double)(k + 1u) * v.dt_sample : INFINITY;
+    }
+  };
+  if (SAMPLE && valid) records();
+  bool active = valid && h < h_end && t <= t_max && !trapped(n, gamma);
+
+  while (__ballot(active) != 0ull) {
+    // lane j's draws for hop h + j (one Philox call holds the words of two hops)
+    const uint64_t hj = h + l;
+    const u32x4 w = draw4(v.seed, e, hj >> 1, STREAM_HOP);
+    const bool odd = (hj & 1u) != 0u;
+    const double r_sel = (double)r31(odd ? w.v[2] : w.v[0]);
+    const uint32_t r_dw = nonzero_draw1(odd ? w.v[3] : w.v[1], v.seed, e, hj, STREAM_HOP_REDRAW);
+    const uint64_t left = active ? h_end - h : 0u;
+    c.cnt = 0u;
+    c.run = active;
+    row_steps(hops16{}, v, c, e, h, left < ROW_BATCH ? (uint32_t)left : ROW_BATCH, r_sel, l, g, s);
+    if (l < 2u || l >= 14u) reinterpret_cast<uint2*>(&s->reached[g][ROW_BATCH - 1][0])[l & 3u] = c.raw;
+    wave_lds_fence();
+    // lane j: hop j's dwell at the site reached and its displacement
+    const bool made = l < c.cnt;
+    const uint4 q0 = s->reached[g][l][0], q1 = s->reached[g][l][1];
+    const uint4 p1 = s->reached[g][l > 0u ? l - 1u : 0u][1];
+    const float fx = l > 0u ? __uint_as_float(p1.x) : px, fy = l > 0u ? __uint_as_float(p1.y) : py,
+                fz = l > 0u ? __uint_as_float(p1.z) : pz;
+    const bool drained = made && (c.my_tg & EDGE_DRAIN_BIT);
+    uint4 hd = q0, pd = q1;  // the hop's target: the row reached, or the drain site it re-injected from
+    if (drained) {
+      const uint4* bd = v.blocks + (size_t)ROW_UNITS * (c.my_tg & TGT_LINE_MASK);
+      hd = bd[0];
+      pd = bd[7];
+    }
+    double i_t = 0.0, i_x = 0.0, i_y = 0.0, i_z = 0.0;
+    if (made) {
+      i_t = dwell_time(hd.x, __hiloint2double((int)hd.w, (int)hd.z), r_dw);
+      i_x = min_image((double)__uint_as_float(pd.x) - (double)fx, v.half_per[0]);
+      i_y = min_image((double)__uint_as_float(pd.y) - (double)fy, v.half_per[1]);
+      i_z = min_image((double)__uint_as_float(pd.z) - (double)fz, v.half_per[2]);
+    }
+    s->inc[g][l][0] = i_t;
+    s->inc[g][l][1] = i_x;
+    s->inc[g][l][2] = i_y;
+    s->inc[g][l][3] = i_z;
+    wave_lds_fence();
+    // the sums in hop order: lane q of each four takes quantity q (an addition of zero for the
+    // hops not made changes nothing)
+    const uint32_t q = l & 3u;
+    double acc = q == 0u ? t : q == 1u ? dx : q == 2u ? dy : dz;
+#pragma unroll
+    for (uint32_t j = 0; j < ROW_BATCH; ++j) acc = acc + s->inc[g][j][q];
+    const double t_end = row_bcast<0>(acc);
+    const uint64_t drain_mask = __ballot(drained);
+    // no record falls due and no hop passes t_max before the batch's end, and nobody drained
+    const bool plain = !TRACE && !(t_rec < t_end) && t_end <= t_max;
+    uint32_t done = c.cnt;
+    if (__ballot(active && !plain) == 0ull && drain_mask == 0ull) {
+      t = t_end;
+      dx = row_bcast<1>(acc);
+      dy = row_bcast<2>(acc);
+      dz = row_bcast<3>(acc);
+      hs = row_hash(hops16{}, hs, q0.y, c.cnt);
+    } else {
+      done = 0u;
+      while (true) {
+        const bool go = done < c.cnt && t <= t_max;
+        if (__ballot(go) == 0ull) break;
+        if (go) {
+          const double* inc = s->inc[g][done];
+          const uint32_t at = 16u * g + done;
+          const uint32_t tg = (uint32_t)__shfl((int)c.my_tg, (int)at, 64);
+          const uint32_t to = (uint32_t)__shfl((int)hd.y, (int)at, 64);
+          const uint32_t reached = s->reached[g][done][0].y;
+          const double t_hop = t;
+          dx = dx + inc[1];
+          dy = dy + inc[2];
+          dz = dz + inc[3];
+          hs = (hs ^ (uint64_t)to) * FNV_PRIME;
+          t = t + inc[0];
+          if (tg & EDGE_DRAIN_BIT) {
+            ++nd;
+            hs = (hs ^ ((uint64_t)reached | (1ull << 32))) * FNV_PRIME;
+          }
+          if (TRACE && e < tv.n_trace && tr < tv.tr_max) {
+            if (l == 0u) {
+              tv.tr_site[(size_t)e * tv.tr_max + tr] = (int32_t)reached;
+              tv.tr_time[(size_t)e * tv.tr_max + tr] = t_hop;
+            }
+            ++tr;
+          }
+          ++done;
+          if (SAMPLE) records();
+        }
+      }
+    }
+    if (COUNT && l < done) {
+      const uint32_t line = c.my_W & TGT_LINE_MASK, off = line - win_base;
+      if (off < win_lines) atomicAdd(win + off, 1u);
+      else atomicAdd(cbase + count_slot(line, v.count_stride), 1u);
+    }
+    if (done > 0u) {
+      const uint4 r0 = s->reached[g][done - 1u][0], r1 = s->reached[g][done - 1u][1];
+      n = r0.x;
+      site = r0.y;
+      gamma = __hiloint2double((int)r0.w, (int)r0.z);
+      px = __uint_as_float(r1.x);
+      py = __uint_as_float(r1.y);
+      pz = __uint_as_float(r1.z);
+    }
+    h += done;
+    active = active && done == ROW_BATCH && h < h_end && t <= t_max && !trapped(n, gamma);
+    wave_lds_fence();
+  }
+  if (v.live) {
+    // excitons that a further launch could move (the budget aside)
+    const uint64_t b = __ballot(valid && l == 0u && !trapped(n, gamma) && t <= t_max);
+    if (lane == 0u && b != 0ull) atomicAdd(v.live, (uint32_t)__popcll(b));
+  }
+  if (!valid || l != 0u) return;
+  v.x.site[e] = (int32_t)site;
+  v.x.t_next[e] = t;
+  v.x.hops[e] = h;
+  v.x.dx[e] = dx;
+  v.x.dy[e] = dy;
+  v.x.dz[e] = dz;
+  v.x.drains[e] = nd;
+  v.x.hash[e] = hs;
+  if (SAMPLE) v.x.k_rec[e] = k;
+  if (TRACE && e < tv.n_trace) tv.tr_n[e] = tr;
+}
+
+// Positions as in k_hop, blockDim.x / 16 excitons to a workgroup; the workgroups of an XCD walk
+// its eighth of the order.  The departure counts of the lines around the workgroup's first
+// exciton -- all lines of a small film -- go to a window of 32-bit LDS counters (a launch's hops
+// cannot wrap one: at most 2^32 departures per copy), the others to the XCD's copy.
+template <bool COUNT, bool SAMPLE, bool TRACE>
+__global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
+  extern __shared__ uint4 rows_lds[];
+  const uint32_t waves = blockDim.x >> 6, per_group = blockDim.x >> 4;
+  batch_lds* s = reinterpret_cast<batch_lds*>(rows_lds) +
+                 __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t* win = reinterpret_cast<uint32_t*>(reinterpret_cast<batch_lds*>(rows_lds) + waves);
+  const uint32_t n = a.n_alive ? *a.n_alive : (uint32_t)a.v.x.n;
+  const uint32_t groups = (n + per_group - 1u) / per_group;
+  const uint32_t per_xcd = (groups + KMC_COUNT_COPIES - 1u) / KMC_COUNT_COPIES;
+  const uint32_t lane = threadIdx.x & 63u;
+  for (uint32_t rank = blockIdx.x / KMC_COUNT_COPIES; rank < per_xcd;
+       rank += gridDim.x / KMC_COUNT_COPIES) {
+    const uint32_t p0 = ((blockIdx.x % KMC_COUNT_COPIES) * per_xcd + rank) * per_group;
+    if (p0 >= n) break;
+    const uint32_t pos = p0 + (threadIdx.x >> 4);
+    const bool valid = pos < n;
+    const uint32_t e = valid ? (a.perm ? a.perm[pos] : pos) : 0u;
+    uint32_t base = 0u;
+    if constexpr (COUNT) {
+      for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) win[i] = 0u;
+      if (a.win_lines < a.n_lines) {
+        const uint32_t L0 = (uint32_t)a.v.roff[a.v.x.site[a.perm ? a.perm[p0] : p0]];
+        base = L0 > a.win_lines / 2u ? L0 - a.win_lines / 2u : 0u;
+        base = min(base, a.n_lines - a.win_lines);
+      }
+      __syncthreads();
+    }
+    hop_rows<COUNT, SAMPLE, TRACE>(a.v, e, valid, a.hop_budget, a.t_max, a.tv, s, lane, win, base,
+                                   a.win_lines);
+    if constexpr (COUNT) {
+      __syncthreads();
+      uint32_t* cbase = a.v.site_count + (size_t)xcd_id() * a.v.count_stride;
+      for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) {
+        const uint32_t cnt = win[i];
+        if (cnt) atomicAdd(cbase + count_slot(base + i, a.v.count_stride), cnt);
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // The same with drift along the tubes (v > 0).
 template <bool COUNT, bool SAMPLE, bool TRACE>
 __global__ __launch_bounds__(256) void k_hop_fly(hop_args a) {
@@ -1364,6 +1736,42 @@ hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bo
   KMC_HOP_CASE(false, true, true)
   KMC_HOP_CASE(true, true, true)
 #undef KMC_HOP_CASE
+  return hipErrorInvalidValue;
+}
+
+constexpr int64_t CU_LDS = 160 * 1024;
+
+// A row of lanes per exciton pays up to 128 excitons per CU: 1,250 hops on 76,543 sites take
+// 0.72 / 0.94 / 1.53 / 1.91 / 3.3 ms at 1,000 / 16,384 / 24,576 / 32,768 / 50,000 excitons (a wave
+// round per 16,384), k_hop's lane per exciton 1.93 / 2.03 / 2.07 / 2.10 / 2.14 ms.
+bool hop_rows_pays(int64_t movable, int n_cu) { return movable <= (int64_t)128 * n_cu; }
+
+hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
+                           bool sample, bool trace, hipStream_t st) {
+  int bs = 64;
+  while (bs < 256 && movable * 16 > (int64_t)bs * n_cu) bs *= 2;
+  const int64_t groups = (movable * 16 + bs - 1) / bs;
+  const int64_t grid = (groups + KMC_COUNT_COPIES - 1) / KMC_COUNT_COPIES * KMC_COUNT_COPIES;
+  // the window takes what the workgroups that share a CU leave of its LDS
+  const int64_t share = CU_LDS / std::max<int64_t>(1, std::min<int64_t>(8, (grid + n_cu - 1) / n_cu)) - 1024;
+  const int64_t batches = (int64_t)(bs / 64) * (int64_t)sizeof(batch_lds);
+  a.n_lines = n_lines;
+  a.win_lines = count ? (uint32_t)std::max<int64_t>(0, std::min<int64_t>(n_lines, (share - batches) / 4)) : 0u;
+  const size_t lds = (size_t)(batches + 4ll * a.win_lines);
+#define KMC_ROWS_CASE(C, S, T)                                                                 \
+  if (count == C && sample == S && trace == T) {                                               \
+    hipLaunchKernelGGL((k_hop_rows<C, S, T>), dim3((unsigned)grid), dim3(bs), lds, st, a);     \
+    return hipGetLastError();                                                                  \
+  }
+  KMC_ROWS_CASE(false, false, false)
+  KMC_ROWS_CASE(true, false, false)
+  KMC_ROWS_CASE(false, true, false)
+  KMC_ROWS_CASE(true, true, false)
+  KMC_ROWS_CASE(false, false, true)
+  KMC_ROWS_CASE(true, false, true)
+  KMC_ROWS_CASE(false, true, true)
+  KMC_ROWS_CASE(true, true, true)
+#undef KMC_ROWS_CASE
   return hipErrorInvalidValue;
 }
 
