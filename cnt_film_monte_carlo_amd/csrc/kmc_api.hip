@@ -17,6 +17,7 @@
 #include "kmc_internal.h"
 #include "kmc_kernels.h"
 #include "kmc_mlp.h"
+#include "kmc_transfer.h"
 
 #include <hipcub/device/device_radix_sort.hpp>
 #include <hipcub/device/device_reduce.hpp>
@@ -864,6 +865,31 @@ int kmc_pair_classes(kmc_ctx* c, int32_t n_chir, int64_t* class_start, const int
   return KMC_OK;
 }
 
+// Exact rates of the entries sel[start[k] .. start[k + 1]) by transfers[k] for every class k (none
+// for a null transfer), all classes in flight together: a class of the surrogate's fallback has a
+// few hundred geometries, too few to fill the GPU alone.
+static int exact_classes(kmc_ctx* c, int n_classes, kmc_transfer* const* transfers,
+                         const int64_t* start, const int64_t* sel, const char* who) {
+  int st = KMC_OK;
+  std::vector<kmc_transfer*> busy;
+  for (int k = 0; k < n_classes && st == KMC_OK; ++k) {
+    const int64_t n = start[k + 1] - start[k];
+    if (n == 0 || !transfers[k]) continue;
+    st = transfer_launch(transfers[k], n, c->d_geo[0].p, c->d_geo[1].p, c->d_geo[2].p,
+                         c->d_geo[3].p, sel + start[k], c->d_pair_rates.p);
+    busy.push_back(transfers[k]);
+  }
+  std::string why = st == KMC_OK ? "" : kmc_transfer_last_error();
+  for (kmc_transfer* t : busy) {
+    const int s = transfer_wait(t);
+    if (st == KMC_OK && s != KMC_OK) {
+      st = s;
+      why = kmc_transfer_last_error();
+    }
+  }
+  return st == KMC_OK ? KMC_OK : fail(c, st, std::string(who) + ": " + why);
+}
+
 int kmc_build_rates_exact(kmc_ctx* c, int32_t n_chir, kmc_transfer* const* transfers,
                           double* elapsed_ms) {
   if (!c || !transfers) return fail(c, KMC_ERR_ARG, "kmc_build_rates_exact: null argument");
@@ -876,14 +902,7 @@ int kmc_build_rates_exact(kmc_ctx* c, int32_t n_chir, kmc_transfer* const* trans
   KMC_TRY(dalloc(c, c->d_pair_rates, std::max<int64_t>(c->nnz, 1)));
   KMC_HIP(c, hipMemsetAsync(c->d_pair_rates.p, 0, c->nnz * sizeof(double), c->stream));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
-  for (int k = 0; k < n_chir * n_chir; ++k) {
-    const int64_t n = start[k + 1] - start[k];
-    if (n == 0 || !transfers[k]) continue;
-    const int s = kmc_transfer_rates_device(transfers[k], n, c->d_geo[0].p, c->d_geo[1].p,
-                                            c->d_geo[2].p, c->d_geo[3].p, sel + start[k],
-                                            c->d_pair_rates.p);
-    if (s != KMC_OK) return fail(c, s, std::string("kmc_build_rates_exact: ") + kmc_transfer_last_error());
-  }
+  KMC_TRY(exact_classes(c, n_chir * n_chir, transfers, start.data(), sel, "kmc_build_rates_exact"));
   KMC_TRY(kmc_set_pair_rates_device(c, c->d_pair_rates.p));
   if (elapsed_ms)
     *elapsed_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -930,13 +949,7 @@ int kmc_build_rates_mlp(kmc_ctx* c, kmc_mlp* mlp, int32_t n_chir, const int32_t*
     KMC_HIP(c, launch_pair_scatter(c->nnz, c->d_cls.p, c->d_mlp_flag.p, c->d_cls_start.p,
                                    c->d_cls_count.p, c->d_sel.p, c->stream));
     KMC_HIP(c, hipStreamSynchronize(c->stream));
-    for (int k = 0; k < nc; ++k) {
-      if (!cnt[k]) continue;
-      const int s = kmc_transfer_rates_device(transfers[k], cnt[k], c->d_geo[0].p, c->d_geo[1].p,
-                                              c->d_geo[2].p, c->d_geo[3].p, c->d_sel.p + start[k],
-                                              c->d_pair_rates.p);
-      if (s != KMC_OK) return fail(c, s, std::string("kmc_build_rates_mlp: ") + kmc_transfer_last_error());
-    }
+    KMC_TRY(exact_classes(c, nc, transfers, start.data(), c->d_sel.p, "kmc_build_rates_mlp"));
   }
   KMC_TRY(kmc_set_pair_rates_device(c, c->d_pair_rates.p));
   if (n_fallback) *n_fallback = start[nc];

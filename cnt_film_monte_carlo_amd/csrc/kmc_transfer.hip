@@ -23,21 +23,25 @@
 
 #include "../../include/cntkmc.h"
 #include "cnt_model.h"
+#include "kmc_transfer.h"
 
 using namespace cntkmc;
 
 
 namespace {
 
-constexpr int CHUNK = 16;     // acceptor momenta per kernel pass (W_b held in registers)
-constexpr int MAXTERMS = 256; // nonzero C_ab terms per pass (one owning thread each)
+constexpr int CHUNK = 16;     // acceptor momenta per group of the term limit
+constexpr int GROUP_TERMS = 256;  // nonzero C_ab terms accepted within one such group
+constexpr int MAXK = 8;       // nonzero |k_b| per kernel pass (their sums are held in registers)
+constexpr int MAXTERMS = 512; // folded terms of one pass
 constexpr int GEOM_BATCH = 65536;  // geometries per launch (one workgroup each)
 // Launches of fewer geometries than this (the surrogate's exact fallback, single-geometry calls)
-// give each (geometry, 256-atom donor chunk) its own workgroup, so that the GPU holds enough waves
-// to cover the scalar-load latency; the chunks' shares of J go through PART_CAP entries of device
-// memory and a finishing kernel.
+// give each (geometry, 64-atom donor chunk) its own workgroup, so that a few geometries still fill
+// the GPU; the chunks' shares of J go through PART_CAP entries of device memory and a finishing
+// kernel.
 constexpr int64_t SPLIT_BELOW = 4096;
 constexpr size_t PART_CAP = size_t(1) << 21;
+constexpr int DONORS = 64;    // donor atoms per chunk: one per lane, the same in the four waves
 
 struct ex_state {
   int ik_cm_idx, n;
@@ -102,15 +106,22 @@ void tube_atoms(const cnt_model& c, std::vector<double>& r3, std::vector<vec2>& 
 // device: one workgroup per geometry
 // ---------------------------------------------------------------------------------------------
 struct exact_args {
-  int32_t na, nb;                 // atoms per tube
-  int32_t nmb;                    // acceptor momenta of this pass (the kernel's NMB)
-  int32_t n_terms;                // nonzero (a, b) terms of this pass
+  int32_t na;                     // donor atoms
+  int32_t nu;                     // acceptor atoms of one unit cell
+  int32_t half, odd;              // pairs of acceptor cells at +-m about the tube's centre; 1: a
+                                  // cell at the centre too
+  int32_t nk;                     // nonzero |k_b| of this pass (the kernel's NK)
+  int32_t n_terms;                // folded (a, b) terms of this pass
   int32_t accumulate;             // 0: out = pass sum; 1: out += pass sum
   const double4* donor;           // [na] centred positions (w unused)
   const double2* u;               // [nma][na]  exp(-i k_a . r)
-  const double* rec;              // acceptor records of this pass: 4 + nb (2 nmb + 4) doubles
+  const double* rec;              // per unit-cell atom: x, y at the tube's centre, z, 0, then the
+                                  // pass's NK phases exp(i k_b . r) there
+  const double* cell;             // per pair of cells: their distance m from the centre in cells,
+                                  // then cos and sin of each k_b's phase over it
+  double period;                  // length T of a cell
   const int32_t* term_a;          // [n_terms] donor momentum slot
-  const int32_t* term_b;          // [n_terms] acceptor momentum slot within the pass
+  const int32_t* term_b;          // [n_terms] 0: k_b = 0, else 1 + the |k_b|'s place in the pass
   const double* term_c;           // [n_terms] C_ab
   int64_t n_geom;
   const double *theta, *z, *a1, *a2;
@@ -132,19 +143,13 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
   return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// Wave-wide sum; every lane ends with the same value.
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
-
-// rate = sum over terms of C_ab |J_ab|^2 (thread t < n_terms holds term t's J), written or added
-// to out[e] by thread 0.  Products are written as explicit FMAs here and in the J sums, so that
-// every kernel that shares this arithmetic rounds it the same way.
-__device__ __forceinline__ void finish_rate(const exact_args& a, int64_t e, bool owner, double jr,
-                                            double ji, double* s_red, int tid) {
-  double part = owner ? a.term_c[tid] * fma(ji, ji, jr * jr) : 0.0;
+// rate = sum over terms of C_ab |J_ab|^2 (thread t holds the J of terms t and t + 256), written or
+// added to out[e] by thread 0.  Products are written as explicit FMAs here and in the J sums, so
+// that every kernel that shares this arithmetic rounds it the same way.
+__device__ __forceinline__ void finish_rate(const exact_args& a, int64_t e, const double (&jr)[2],
+                                            const double (&ji)[2], double* s_red, int tid) {
+  double part = tid < a.n_terms ? a.term_c[tid] * fma(ji[0], ji[0], jr[0] * jr[0]) : 0.0;
+  if (tid + 256 < a.n_terms) part += a.term_c[tid + 256] * fma(ji[1], ji[1], jr[1] * jr[1]);
   for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
   if ((tid & 63) == 0) s_red[tid >> 6] = part;
   __syncthreads();
@@ -155,103 +160,189 @@ __device__ __forceinline__ void finish_rate(const exact_args& a, int64_t e, bool
   __syncthreads();
 }
 
-// One workgroup of 256 threads per geometry.  Donor atoms go in chunks of 256 (one per thread).
-// make_Ru_3d places the acceptor at R_j = Rz(theta) (b_j + s2 y) + z_s z and the donor at
-// r_i + s1 y; since Rz leaves z and lengths alone, |R_i - R_j| = |q_i - b_j| with the donor atom
-// taken into the acceptor's frame, q_i = Rz(-theta) (r_i + s1 y - z_s z) - s2 y.  The acceptor
-// records (b_j and v_b(j) of the pass's momenta) are then the same for every geometry and are
-// read with wave-uniform addresses (scalar loads): nothing is staged in LDS and the per-pair cost
-// is the distance, one reciprocal square root and 2 NMB FMAs on the VALU.  For its atom i a
-// thread accumulates W_b(i) = sum_j v_b(j) / |q_i - b_j|; the chunk's share of
-// J_ab = sum_i u_a(i) W_b(i) is then summed per term across each wave and the four wave sums
-// are added by the term's owning thread (t < n_terms).  Split launches run one chunk per workgroup
-// and leave each chunk's four-wave sum in part[] for k_exact_finish, which adds the chunks in the
-// same order, so both launch shapes give the same bits.
-template <int NMB>
+// One step of a wave sum of several values at once: the lanes below 32 (or of the even rows of
+// 16) go on with x, the others with y, each having taken the partner lane's part of its value.
+template <int W>
+__device__ __forceinline__ double fold_pair(double x, double y) {
+  const auto swap = [](uint32_t p, uint32_t q) {
+    if constexpr (W == 32) return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    else return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+  };
+  const auto lo = swap((uint32_t)__double2loint(x), (uint32_t)__double2loint(y));
+  const auto hi = swap((uint32_t)__double2hiint(x), (uint32_t)__double2hiint(y));
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// x plus its value in another lane of the row of 16 (a DPP control word).
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, true);
+  return x + __hiloint2double(hi, lo);
+}
+
+// The wave sums of four complex values at once, 34 VALU instructions where eight separate
+// butterflies take 144.  The row r = lane / 16 ends with component r / 2 (the lanes 0..31 re,
+// 32..63 im) of value (r & 1) in its lanes 0..7 and of value 2 + (r & 1) in its lanes 8..15.
+__device__ __forceinline__ double wave_sum4(const double2 (&v)[4], uint32_t lane) {
+  double c[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) c[k] = fold_pair<32>(v[k].x, v[k].y);
+  const double p = fold_pair<16>(c[0], c[1]), q = fold_pair<16>(c[2], c[3]);
+  const bool up = (lane & 8u) != 0u;
+  const double keep = up ? q : p, give = up ? p : q;
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(give), 0x128, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(give), 0x128, 0xF, 0xF, true);
+  double s = keep + __hiloint2double(hi, lo);  // row_ror:8
+  s = add_dpp<0x141>(s);                       // row_half_mirror: lane 7 - i of the half row
+  s = add_dpp<0x4E>(s);                        // quad_perm [2,3,0,1]
+  return add_dpp<0xB1>(s);                     // quad_perm [1,0,3,2]
+}
+
+// One workgroup of 256 threads per geometry.  make_Ru_3d places the acceptor at
+// R_j = Rz(theta) (b_j + s2 y) + z_s z and the donor at r_i + s1 y; since Rz leaves z and lengths
+// alone, |R_i - R_j| = |q_i - b_j| with the donor atom taken into the acceptor's frame,
+// q_i = Rz(-theta) (r_i + s1 y - z_s z) - s2 y, so the acceptor's data are the same for every
+// geometry and are read with wave-uniform addresses (scalar loads).
+//
+// The FP64 VALU bounds the sums W_b(i) = sum_j v_b(j) / |q_i - b_j|; three properties cut them:
+//  * W of -k_b is the conjugate of W of k_b (distances are real): only the |k_b| are summed.
+//  * The acceptor is a unit cell repeated along y: for one of its atoms the part of the distance
+//    across the tube is computed once for all cells.
+//  * The cells lie in pairs at +-m about the tube's centre, where the phase of k_b is that of the
+//    centre times exp(+-i k_b m): their inverse distances enter as sum and difference, with one
+//    FMA each per k_b, and the centre's phase is applied once per atom.
+// Per atom pair at NK = 2 (the momenta 0, +-1, +-2) that is ~16 issue slots (4 of them the
+// hardware root) against 28 for the plain sum over atoms and momenta: 27,951 geometries of
+// (8,6) -> (7,5) at 300 K take 63.3 -> 39.5 ms
+// (the nine tables of three chiralities 1,416 -> 791 ms), one geometry 0.27 -> 0.036 ms.  Errors
+// against an 80-bit evaluation of the same sum stay at rounding, 2e-16 to 4e-16 on average.
+//
+// Donor atoms go in chunks of 64, one per lane; the four waves take a quarter of the unit cell's
+// atoms each and add their sums through LDS.  The chunk's share of J_ab = sum_i u_a(i) W_b(i) is
+// then summed over the lanes, four terms at a time, the waves taking turns.  Split launches run
+// one chunk per workgroup and leave its share in part[] for k_exact_finish, which adds the chunks
+// in the same order, so both launch shapes give the same bits.
+template <int NK, int HALF>
 __global__ __launch_bounds__(256) void k_exact_rate(exact_args a, const double* __restrict__ rec,
+                                                    const double* __restrict__ cell,
                                                     const int32_t* __restrict__ term_a,
                                                     const int32_t* __restrict__ term_b) {
-  constexpr int S = 4 + 2 * NMB;   // doubles per acceptor record: (Re, Im) v_b, next x, y, z, 0
-  __shared__ double2 s_part[4][MAXTERMS];
+  constexpr int S = 4 + 2 * NK;    // doubles per unit-cell atom
+  constexpr int CS = 1 + 2 * NK;   // doubles per pair of cells
+  constexpr int NB = 1 + 2 * NK;   // sums per donor: W_0, then (Re, Im) W_b
+  __shared__ double s_w[4][NB][DONORS];
+  __shared__ double2 s_j[MAXTERMS];
   __shared__ double s_red[4];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const double period = a.period;
+  const int c_lo = a.nu * wave / 4, c_hi = a.nu * (wave + 1) / 4;
   for (int64_t g = blockIdx.x; g < a.n_geom; g += gridDim.x) {
     const int64_t e = a.sel ? a.sel[g] : g;
     const double zs = fmin(fmax(a.z[e], a.clamp_lo[0]), a.clamp_hi[0]);
     const double s1 = fmin(fmax(a.a1[e], a.clamp_lo[1]), a.clamp_hi[1]);
     const double s2 = fmin(fmax(a.a2[e], a.clamp_lo[2]), a.clamp_hi[2]);
     const double cth = a.trig[g].x, sth = a.trig[g].y;
-    const bool owner = tid < a.n_terms;
-    double jr = 0.0, ji = 0.0;
-    const int i_lo = a.split ? 256 * (int)blockIdx.y : 0;
-    const int i_hi = a.split ? min(a.na, i_lo + 256) : a.na;
-    for (int i0 = i_lo; i0 < i_hi; i0 += 256) {
-      const int i = i0 + tid;
+    double jr[2] = {0.0, 0.0}, ji[2] = {0.0, 0.0};
+    const int i_lo = a.split ? DONORS * (int)blockIdx.y : 0;
+    const int i_hi = a.split ? min(a.na, i_lo + DONORS) : a.na;
+    for (int i0 = i_lo; i0 < i_hi; i0 += DONORS) {
+      const int i = i0 + lane;
       const bool live = i < a.na;
       const double4 ri = live ? a.donor[i] : make_double4(0, 0, 0, 0);
       const double ry = ri.y + s1;
       const double qx = cth * ri.x + sth * ry;
       const double qy = cth * ry - sth * ri.x - s2;
       const double qz = ri.z - zs;
-      double wr[NMB], wi[NMB];
+      double w[NB];
 #pragma unroll
-      for (int q = 0; q < NMB; q++) wr[q] = wi[q] = 0.0;
-      // record j carries v_b(j) and the position of atom j + 1 (the first position leads the
-      // array), so each pair's scalar loads are issued together and waited on once
-      double bx = rec[0], by = rec[1], bz = rec[2];
-      asm volatile("" : "+s"(bx), "+s"(by), "+s"(bz));  // loaded before the loop, not pending in it
-      const double* b = rec + 4;
-      for (int j = 0; j < a.nb; j++) {
-        // the record's loads go out first and the distance and square root cover them (a
-        // scheduling fence keeps them there, a second one keeps the position hand-over after
-        // the FMAs so that the loads are waited on only there)
-        double v[2 * NMB];
+      for (int b = 0; b < NB; ++b) w[b] = 0.0;
+      const double* at = rec + (size_t)c_lo * S;
+      for (int c = c_lo; c < c_hi; ++c, at += S) {
+        const double dx = qx - at[0], dy = qy - at[1], dz = qz - at[2];
+        const double across = fma(dz, dz, dx * dx);
+        double z0 = 0.0, cs[NK > 0 ? NK : 1], sn[NK > 0 ? NK : 1];
 #pragma unroll
-        for (int k = 0; k < 2 * NMB; k++) v[k] = b[k];
-        const double nx = b[2 * NMB], ny = b[2 * NMB + 1], nz = b[2 * NMB + 2];
-        __builtin_amdgcn_sched_barrier(0);
-        const double dx = qx - bx, dy = qy - by, dz = qz - bz;
-        const double r = rsqrt_f64(fma(dz, dz, fma(dy, dy, dx * dx)));
+        for (int b = 0; b < NK; ++b) cs[b] = sn[b] = 0.0;
+        const auto pair_of_cells = [&](const double* t) {
+          // one rounding each (m T as a number of its own would move a whole cell by its rounding)
+          const double yp = fma(-t[0], period, dy), ym = fma(t[0], period, dy);
+          const double rp = rsqrt_f64(fma(yp, yp, across)), rm = rsqrt_f64(fma(ym, ym, across));
+          const double sum = rp + rm, dif = rp - rm;
+          z0 += sum;
 #pragma unroll
-        for (int q = 0; q < NMB; q++) {
-          wr[q] += v[2 * q] * r;
-          wi[q] += v[2 * q + 1] * r;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        bx = nx;
-        by = ny;
-        bz = nz;
-        // carry the next position in SGPRs (the compiler would otherwise reload it at the top
-        // of the next pair)
-        asm volatile("" : "+s"(bx), "+s"(by), "+s"(bz));
-        b += S;
-      }
-      // this chunk's u_a(i) W_b(i), summed over the wave for every term (a, b)
+          for (int b = 0; b < NK; ++b) {
+            cs[b] = fma(t[1 + 2 * b], sum, cs[b]);
+            sn[b] = fma(t[2 + 2 * b], dif, sn[b]);
+          }
+        };
+        if constexpr (HALF > 0) {
+          // read again for every atom (scalar loads that hit the cache): kept over the loop, the
+          // table would spill from scalar to vector registers
+          int t = 0;
+          if constexpr (NK > 2) asm volatile("" : "+s"(t));
 #pragma unroll
-      for (int q = 0; q < NMB; q++) {
-        const double w_r = live ? wr[q] : 0.0, w_i = live ? wi[q] : 0.0;
-        for (int t = 0; t < a.n_terms; t++) {
-          if (term_b[t] != q) continue;
-          const double2 u = live ? a.u[(size_t)term_a[t] * a.na + i] : make_double2(0, 0);
-          const double pr = wave_sum(fma(u.x, w_r, -(u.y * w_i)));
-          const double pi = wave_sum(fma(u.x, w_i, u.y * w_r));
-          if (lane == 0) s_part[wave][t] = make_double2(pr, pi);
-        }
-      }
-      __syncthreads();
-      if (owner) {
-        const double pr = (s_part[0][tid].x + s_part[1][tid].x) + (s_part[2][tid].x + s_part[3][tid].x);
-        const double pi = (s_part[0][tid].y + s_part[1][tid].y) + (s_part[2][tid].y + s_part[3][tid].y);
-        if (a.split) {
-          a.part[((size_t)g * gridDim.y + blockIdx.y) * a.n_terms + tid] = make_double2(pr, pi);
+          for (int p = 0; p < HALF; ++p) pair_of_cells(cell + t + p * CS);
         } else {
-          jr += pr;
-          ji += pi;
+          for (int p = 0; p < a.half; ++p) pair_of_cells(cell + p * CS);
+          if (a.odd) {
+            const double r = rsqrt_f64(fma(dy, dy, across));
+            z0 += r;
+#pragma unroll
+            for (int b = 0; b < NK; ++b) cs[b] += r;
+          }
+        }
+        w[0] += z0;
+#pragma unroll
+        for (int b = 0; b < NK; ++b) {
+          const double pr = at[4 + 2 * b], pi = at[5 + 2 * b];
+          w[1 + 2 * b] = fma(pr, cs[b], fma(-pi, sn[b], w[1 + 2 * b]));
+          w[2 + 2 * b] = fma(pr, sn[b], fma(pi, cs[b], w[2 + 2 * b]));
         }
       }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) s_w[wave][b][lane] = live ? w[b] : 0.0;
       __syncthreads();
+      for (int k = tid; k < NB * DONORS; k += 256) {
+        double* p = &s_w[0][0][0] + k;
+        p[0] = (p[0] + p[NB * DONORS]) + (p[2 * NB * DONORS] + p[3 * NB * DONORS]);
+      }
+      __syncthreads();
+      for (int t0 = 4 * wave; t0 < a.n_terms; t0 += 16) {
+        double2 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int t = t0 + k;
+          v[k] = make_double2(0.0, 0.0);
+          if (t < a.n_terms && live) {
+            const double2 u = a.u[(size_t)term_a[t] * a.na + i];
+            const int b = term_b[t];
+            const double wr = s_w[0][b == 0 ? 0 : 2 * b - 1][lane];
+            const double wi = b == 0 ? 0.0 : s_w[0][2 * b][lane];
+            v[k] = make_double2(fma(u.x, wr, -(u.y * wi)), fma(u.x, wi, u.y * wr));
+          }
+        }
+        const double s = wave_sum4(v, (uint32_t)lane);
+        const int t = t0 + ((lane >> 4) & 1) + 2 * ((lane >> 3) & 1);
+        if ((lane & 7) == 0 && t < a.n_terms)
+          reinterpret_cast<double*>(&s_j[t])[lane >> 5] = s;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int t = tid + 256 * h;
+        if (t < a.n_terms) {
+          if (a.split) {
+            a.part[((size_t)g * gridDim.y + blockIdx.y) * a.n_terms + t] = s_j[t];
+          } else {
+            jr[h] += s_j[t].x;
+            ji[h] += s_j[t].y;
+          }
+        }
+      }
     }
-    if (!a.split) finish_rate(a, e, owner, jr, ji, s_red, tid);
+    if (!a.split) finish_rate(a, e, jr, ji, s_red, tid);
   }
 }
 
@@ -261,19 +352,22 @@ __global__ __launch_bounds__(256) void k_exact_finish(exact_args a, int n_chunks
   const int tid = threadIdx.x;
   for (int64_t g = blockIdx.x; g < a.n_geom; g += gridDim.x) {
     const int64_t e = a.sel ? a.sel[g] : g;
-    const bool owner = tid < a.n_terms;
-    double jr = 0.0, ji = 0.0;
-    if (owner)
-      for (int c = 0; c < n_chunks; c++) {
-        const double2 p = a.part[((size_t)g * n_chunks + c) * a.n_terms + tid];
-        jr += p.x;
-        ji += p.y;
-      }
-    finish_rate(a, e, owner, jr, ji, s_red, tid);
+    double jr[2] = {0.0, 0.0}, ji[2] = {0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int t = tid + 256 * h;
+      if (t < a.n_terms)
+        for (int c = 0; c < n_chunks; c++) {
+          const double2 p = a.part[((size_t)g * n_chunks + c) * a.n_terms + t];
+          jr[h] += p.x;
+          ji[h] += p.y;
+        }
+    }
+    finish_rate(a, e, jr, ji, s_red, tid);
   }
 }
 
-int pass_width(int nmb) { return std::max(1, std::min(nmb, CHUNK)); }
+int n_chunks(int32_t na) { return (na + DONORS - 1) / DONORS; }
 
 // cos and sin of each geometry's theta, ahead of the rate passes (sincos' argument reduction would
 // otherwise set the register budget, and with it the occupancy, of every rate kernel).
@@ -291,24 +385,36 @@ __global__ void k_zero_rates(int64_t n, const int64_t* sel, double* out) {
   if (g < n) out[sel ? sel[g] : g] = 0.0;
 }
 
-// One pass over a chunk of at most 16 acceptor momenta.
+// One pass over at most MAXK nonzero |k_b| (and k_b = 0).  Tubes of 10 unit cells, the length
+// every table of the reference is made for, take the unrolled cell loop.
+template <int NK>
+void launch_width(const exact_args& a, dim3 g, hipStream_t st) {
+  if (a.half == 5 && !a.odd)
+    hipLaunchKernelGGL((k_exact_rate<NK, 5>), g, dim3(256), 0, st, a, a.rec, a.cell, a.term_a, a.term_b);
+  else
+    hipLaunchKernelGGL((k_exact_rate<NK, 0>), g, dim3(256), 0, st, a, a.rec, a.cell, a.term_a, a.term_b);
+}
+
 hipError_t launch_pass(const exact_args& a, hipStream_t st) {
   const unsigned grid = (unsigned)std::min<int64_t>(a.n_geom, GEOM_BATCH);
-  const int chunks = (a.na + 255) / 256;
-  const dim3 g(grid, a.split ? chunks : 1), b(256);
-  switch (a.nmb) {
-#define EXACT_CASE(n) \
-  case n: hipLaunchKernelGGL(k_exact_rate<n>, g, b, 0, st, a, a.rec, a.term_a, a.term_b); break;
-    EXACT_CASE(1) EXACT_CASE(2) EXACT_CASE(3) EXACT_CASE(4) EXACT_CASE(5) EXACT_CASE(6)
-    EXACT_CASE(7) EXACT_CASE(8) EXACT_CASE(9) EXACT_CASE(10) EXACT_CASE(11) EXACT_CASE(12)
-    EXACT_CASE(13) EXACT_CASE(14) EXACT_CASE(15) EXACT_CASE(16)
-#undef EXACT_CASE
+  const int chunks = n_chunks(a.na);
+  const dim3 g(grid, a.split ? chunks : 1);
+  switch (a.nk) {
+    case 0: launch_width<0>(a, g, st); break;
+    case 1: launch_width<1>(a, g, st); break;
+    case 2: launch_width<2>(a, g, st); break;
+    case 3: launch_width<3>(a, g, st); break;
+    case 4: launch_width<4>(a, g, st); break;
+    case 5: launch_width<5>(a, g, st); break;
+    case 6: launch_width<6>(a, g, st); break;
+    case 7: launch_width<7>(a, g, st); break;
+    case 8: launch_width<8>(a, g, st); break;
     default: return hipErrorInvalidValue;
   }
   if (a.split) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_exact_finish, dim3(grid), b, 0, st, a, chunks);
+    hipLaunchKernelGGL(k_exact_finish, dim3(grid), dim3(256), 0, st, a, chunks);
   }
   return hipGetLastError();
 }
@@ -329,14 +435,19 @@ struct kmc_transfer {
   std::vector<int> mom_a, mom_b;            // ik_cm of each momentum slot
   std::vector<int32_t> term_a, term_b;      // nonzero terms
   std::vector<double> term_c;
-  // acceptor slots [b0, b0 + 16), terms [t0, t0 + nt), records at h_rec[rec0]
-  struct pass { int b0, width, t0, nt; size_t rec0; };
+  // a pass sums nk nonzero |k_b|; folded terms [t0, t0 + nt), records at h_rec[rec0], cells at
+  // h_rec[cell0]
+  struct pass { int nk, t0, nt; size_t rec0, cell0; };
   std::vector<pass> passes;
+  std::vector<int32_t> fold_a, fold_b;      // the device's terms: (k_a, k_b) and (-k_a, -k_b), whose
+  std::vector<double> fold_c;               // J are conjugates, are one term
+  int nu = 0, length = 0;                   // acceptor: unit-cell atoms and cells
+  double period = 0.0;                      // and the length of a cell
   double clamp_lo[3] = {-1e300, -1e300, -1e300}, clamp_hi[3] = {1e300, 1e300, 1e300};
-  std::vector<double> h_donor, h_acc;
-  std::vector<vec2> r2d, r2a;
+  std::vector<double> h_donor;
+  std::vector<vec2> r2d;
   std::vector<cplx> h_u;
-  std::vector<double> h_rec;                // per pass: 4 + nb (2 width + 4) doubles of acceptor records
+  std::vector<double> h_rec;                // per pass: unit-cell atoms, then pairs of cells
   bool on_device = false;
   double4* d_donor = nullptr;
   double2* d_u = nullptr;
@@ -370,9 +481,9 @@ int upload(kmc_transfer* t) {
   if (e == hipSuccess) e = put(&t->d_rec, t->h_rec);
   if (e == hipSuccess) e = hipMalloc((void**)&t->d_trig, GEOM_BATCH * sizeof(double2));
   if (e == hipSuccess) e = hipMalloc((void**)&t->d_part, PART_CAP * sizeof(double2));
-  if (e == hipSuccess) e = put(&t->d_ta, t->term_a);
-  if (e == hipSuccess) e = put(&t->d_tb, t->term_b);
-  if (e == hipSuccess) e = put(&t->d_tc, t->term_c);
+  if (e == hipSuccess) e = put(&t->d_ta, t->fold_a);
+  if (e == hipSuccess) e = put(&t->d_tb, t->fold_b);
+  if (e == hipSuccess) e = put(&t->d_tc, t->fold_c);
   if (e != hipSuccess)
     return tfail(e == hipErrorNoDevice ? KMC_ERR_NODEVICE : KMC_ERR_HIP,
                  std::string("kmc_transfer: device setup failed: ") + hipGetErrorString(e));
@@ -383,7 +494,10 @@ int upload(kmc_transfer* t) {
 exact_args args_of(const kmc_transfer* t) {
   exact_args a{};
   a.na = t->info.n_atoms_donor;
-  a.nb = t->info.n_atoms_acceptor;
+  a.nu = t->nu;
+  a.half = t->length / 2;
+  a.odd = t->length & 1;
+  a.period = t->period;
   a.donor = t->d_donor;
   a.u = t->d_u;
   a.trig = t->d_trig;
@@ -407,7 +521,7 @@ hipError_t launch_exact(const kmc_transfer* t, exact_args a, hipStream_t st) {
   }
   int max_terms = 1;
   for (const auto& p : t->passes) max_terms = std::max(max_terms, p.nt);
-  const size_t per_geom = (size_t)((a.na + 255) / 256) * max_terms;  // chunk shares per geometry
+  const size_t per_geom = (size_t)n_chunks(a.na) * max_terms;  // chunk shares per geometry
   a.split = a.n_geom < SPLIT_BELOW && per_geom <= PART_CAP;
   const int64_t batch = a.split ? std::min<int64_t>(GEOM_BATCH, (int64_t)(PART_CAP / per_geom))
                                 : GEOM_BATCH;
@@ -429,10 +543,11 @@ hipError_t launch_exact(const kmc_transfer* t, exact_args a, hipStream_t st) {
     e = hipGetLastError();
     for (size_t k = 0; k < t->passes.size() && e == hipSuccess; k++) {
       const auto& p = t->passes[k];
-      b.nmb = p.width;
+      b.nk = p.nk;
       b.n_terms = p.nt;
       b.accumulate = k > 0;
       b.rec = t->d_rec + p.rec0;
+      b.cell = t->d_rec + p.cell0;
       b.term_a = t->d_ta + p.t0;
       b.term_b = t->d_tb + p.t0;
       b.term_c = t->d_tc + p.t0;
@@ -443,6 +558,39 @@ hipError_t launch_exact(const kmc_transfer* t, exact_args a, hipStream_t st) {
 }
 
 }  // namespace
+
+namespace cntkmc {
+
+int transfer_launch(kmc_transfer* t, int64_t n, const double* d_theta, const double* d_z,
+                    const double* d_a1, const double* d_a2, const int64_t* d_sel, double* d_rate) {
+  if (!t || n < 0 || (n > 0 && (!d_theta || !d_z || !d_a1 || !d_a2 || !d_rate)))
+    return tfail(KMC_ERR_ARG, "kmc_transfer_rates_device: bad argument");
+  if (n == 0) return KMC_OK;
+  {
+    const int s = upload(t);
+    if (s != KMC_OK) return s;
+  }
+  exact_args a = args_of(t);
+  a.n_geom = n;
+  a.theta = d_theta;
+  a.z = d_z;
+  a.a1 = d_a1;
+  a.a2 = d_a2;
+  a.sel = d_sel;
+  a.out = d_rate;
+  hipError_t e = hipSetDevice(t->device);
+  if (e == hipSuccess) e = launch_exact(t, a, t->stream);
+  if (e != hipSuccess) return tfail(KMC_ERR_HIP, std::string("kmc_transfer_rates: ") + hipGetErrorString(e));
+  return KMC_OK;
+}
+
+int transfer_wait(kmc_transfer* t) {
+  const hipError_t e = hipStreamSynchronize(t->stream);
+  if (e != hipSuccess) return tfail(KMC_ERR_HIP, std::string("kmc_transfer_rates: ") + hipGetErrorString(e));
+  return KMC_OK;
+}
+
+}  // namespace cntkmc
 
 extern "C" {
 
@@ -500,25 +648,26 @@ int kmc_transfer_create(int32_t device, const kmc_cnt* donor, const kmc_cnt* acc
   if (t->mom_a.empty()) t->mom_a.push_back(0);
   if (t->mom_b.empty()) t->mom_b.push_back(0);
   const int nma = (int)t->mom_a.size(), nmb = (int)t->mom_b.size();
-  // terms ordered by (donor slot, acceptor slot) and grouped into passes of 16 acceptor slots
+  // terms ordered by (donor slot, acceptor slot) within groups of 16 acceptor slots
   std::sort(acc.begin(), acc.end(), [](const term& x, const term& y) {
     return x.q / CHUNK != y.q / CHUNK ? x.q / CHUNK < y.q / CHUNK : x.p != y.p ? x.p < y.p : x.q < y.q;
   });
+  int group = -1, in_group = 0;
   for (const term& x : acc) {
     if (x.c == 0.0) continue;
-    const int b0 = x.q / CHUNK * CHUNK;
-    if (t->passes.empty() || t->passes.back().b0 != b0)
-      t->passes.push_back({b0, pass_width(std::min(CHUNK, nmb - b0)), (int)t->term_c.size(), 0, 0});
-    if (++t->passes.back().nt > MAXTERMS) {
+    if (x.q / CHUNK != group) {
+      group = x.q / CHUNK;
+      in_group = 0;
+    }
+    if (++in_group > GROUP_TERMS) {
       delete t;
       return tfail(KMC_ERR_CAPACITY, "kmc_transfer_create: more than 256 momentum terms "
                                      "within 16 acceptor momenta");
     }
     t->term_a.push_back(x.p);
-    t->term_b.push_back(x.q - b0);
+    t->term_b.push_back(x.q);
     t->term_c.push_back(x.c);
   }
-  const int v_rows = t->passes.empty() ? 0 : t->passes.back().b0 + t->passes.back().width;
   kmc_transfer_info& in = t->info;
   in.n_donor_states = (int)ds.size();
   in.n_acceptor_states = (int)as.size();
@@ -532,37 +681,83 @@ int kmc_transfer_create(int32_t device, const kmc_cnt* donor, const kmc_cnt* acc
   in.min_energy = min_energy;
   // host copies of the device data; uploaded on the first rate call
   tube_atoms(D, t->h_donor, t->r2d);
-  tube_atoms(A, t->h_acc, t->r2a);
-  t->h_u.assign((size_t)nma * t->r2d.size(), cplx(0, 0));
-  std::vector<cplx> h_v((size_t)std::max(v_rows, nmb) * t->r2a.size(), cplx(0, 0));
-  for (int p = 0; p < nma; p++) {
-    const double kx = t->mom_a[p] * D.dk_l.x, ky = t->mom_a[p] * D.dk_l.y;
-    for (size_t i = 0; i < t->r2d.size(); i++)
-      t->h_u[p * t->r2d.size() + i] = std::exp(-cplx(0, 1) * (kx * t->r2d[i].x + ky * t->r2d[i].y));
-  }
-  for (int q = 0; q < nmb; q++) {
-    const double kx = t->mom_b[q] * A.dk_l.x, ky = t->mom_b[q] * A.dk_l.y;
-    for (size_t j = 0; j < t->r2a.size(); j++)
-      h_v[q * t->r2a.size() + j] = std::exp(+cplx(0, 1) * (kx * t->r2a[j].x + ky * t->r2a[j].y));
-  }
-  // acceptor records of each pass: the first atom's position (x, y, z, 0), then for every atom
-  // j its v_b(j) over the pass's momenta followed by the position of atom j + 1 (zeros after the
-  // last atom)
-  const size_t nb = t->r2a.size();
-  auto put_pos = [&](size_t j) {
-    for (int k = 0; k < 3; k++) t->h_rec.push_back(j < nb ? t->h_acc[4 * j + k] : 0.0);
-    t->h_rec.push_back(0.0);
-  };
-  for (auto& p : t->passes) {
-    p.rec0 = t->h_rec.size();
-    put_pos(0);
-    for (size_t j = 0; j < nb; j++) {
-      for (int q = 0; q < p.width; q++) {
-        t->h_rec.push_back(h_v[(size_t)(p.b0 + q) * nb + j].real());
-        t->h_rec.push_back(h_v[(size_t)(p.b0 + q) * nb + j].imag());
-      }
-      put_pos(j + 1);
+  t->nu = A.Nu;
+  t->length = A.length;
+  t->period = A.t_vec_3d.y;
+  const size_t na = t->r2d.size();
+  // fold the terms: J of (-k_a, -k_b) is the conjugate of J of (k_a, k_b), so k_b >= 0 (and
+  // k_a >= 0 where k_b = 0) stands for both
+  struct folded { int ka, kb; double c; };
+  std::vector<folded> fold;
+  for (size_t k = 0; k < t->term_c.size(); k++) {
+    int ka = t->mom_a[t->term_a[k]], kb = t->mom_b[t->term_b[k]];
+    if (kb < 0 || (kb == 0 && ka < 0)) {
+      ka = -ka;
+      kb = -kb;
     }
+    auto it = std::find_if(fold.begin(), fold.end(),
+                           [&](const folded& x) { return x.ka == ka && x.kb == kb; });
+    if (it == fold.end()) fold.push_back({ka, kb, t->term_c[k]});
+    else it->c += t->term_c[k];
+  }
+  std::sort(fold.begin(), fold.end(), [](const folded& x, const folded& y) {
+    return x.kb != y.kb ? x.kb < y.kb : x.ka < y.ka;
+  });
+  // passes of at most MAXK nonzero |k_b| (k_b = 0 goes with the first)
+  std::vector<int> ka_slots;
+  size_t next = 0;
+  while (next < fold.size()) {
+    kmc_transfer::pass p{0, (int)t->fold_c.size(), 0, 0, 0};
+    std::vector<int> ks;
+    for (; next < fold.size() && p.nt < MAXTERMS; ++next) {
+      const folded& x = fold[next];
+      if (x.kb != 0 && (ks.empty() || ks.back() != x.kb)) {
+        if ((int)ks.size() == MAXK) break;
+        ks.push_back(x.kb);
+      }
+      t->fold_a.push_back(slot(ka_slots, x.ka));
+      t->fold_b.push_back(x.kb == 0 ? 0 : (int)ks.size());
+      t->fold_c.push_back(x.c);
+      ++p.nt;
+    }
+    p.nk = (int)ks.size();
+    // unit-cell atoms at the middle of the tube (make_Ru_3d centres y between its lowest and
+    // highest atom: exciton_transfer.cpp:310-322), their phases exp(i k_b . r) there; in extended
+    // precision, since a cell's phase is shared by all of its atoms
+    typedef long double ext;
+    double ymin = A.pos_u_3d[0].y, ymax = ymin;
+    for (int c = 0; c < A.Nu; c++) {
+      ymin = std::min(ymin, A.pos_u_3d[c].y);
+      ymax = std::max(ymax, A.pos_u_3d[c].y);
+    }
+    const ext T = A.t_vec_3d.y, centre = (ext)0.5 * (A.length - 1);
+    const ext mid = (ymax + (A.length - 1) * T + ymin) / 2;
+    const auto put_phase = [&](ext arg) {
+      t->h_rec.push_back((double)std::cos(arg));
+      t->h_rec.push_back((double)std::sin(arg));
+    };
+    p.rec0 = t->h_rec.size();
+    for (int c = 0; c < A.Nu; c++) {
+      t->h_rec.insert(t->h_rec.end(), {A.pos_u_3d[c].x,
+                                       (double)(A.pos_u_3d[c].y + centre * T - mid),
+                                       A.pos_u_3d[c].z, 0.0});
+      const ext rx = A.pos_a[c].x + centre * A.t_vec.x, ry = A.pos_a[c].y + centre * A.t_vec.y;
+      for (int kb : ks) put_phase(kb * ((ext)A.dk_l.x * rx + (ext)A.dk_l.y * ry));
+    }
+    p.cell0 = t->h_rec.size();
+    for (int q = 0; q < A.length / 2; q++) {
+      const ext m = A.length & 1 ? q + (ext)1 : q + (ext)0.5;  // cells from the centre
+      t->h_rec.push_back((double)m);
+      for (int kb : ks)
+        put_phase(m * kb * ((ext)A.dk_l.x * A.t_vec.x + (ext)A.dk_l.y * A.t_vec.y));
+    }
+    t->passes.push_back(p);
+  }
+  t->h_u.assign(std::max<size_t>(1, ka_slots.size()) * na, cplx(0, 0));
+  for (size_t p = 0; p < ka_slots.size(); p++) {
+    const double kx = ka_slots[p] * D.dk_l.x, ky = ka_slots[p] * D.dk_l.y;
+    for (size_t i = 0; i < na; i++)
+      t->h_u[p * na + i] = std::exp(-cplx(0, 1) * (kx * t->r2d[i].x + ky * t->r2d[i].y));
   }
   *out = t;
   return KMC_OK;
@@ -614,26 +809,8 @@ int kmc_transfer_set_clamp(kmc_transfer* t, const double lo[3], const double hi[
 int kmc_transfer_rates_device(kmc_transfer* t, int64_t n, const double* d_theta, const double* d_z,
                               const double* d_a1, const double* d_a2, const int64_t* d_sel,
                               double* d_rate) {
-  if (!t || n < 0 || (n > 0 && (!d_theta || !d_z || !d_a1 || !d_a2 || !d_rate)))
-    return tfail(KMC_ERR_ARG, "kmc_transfer_rates_device: bad argument");
-  if (n == 0) return KMC_OK;
-  {
-    const int s = upload(t);
-    if (s != KMC_OK) return s;
-  }
-  exact_args a = args_of(t);
-  a.n_geom = n;
-  a.theta = d_theta;
-  a.z = d_z;
-  a.a1 = d_a1;
-  a.a2 = d_a2;
-  a.sel = d_sel;
-  a.out = d_rate;
-  hipError_t e = hipSetDevice(t->device);
-  if (e == hipSuccess) e = launch_exact(t, a, t->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
-  if (e != hipSuccess) return tfail(KMC_ERR_HIP, std::string("kmc_transfer_rates: ") + hipGetErrorString(e));
-  return KMC_OK;
+  const int s = transfer_launch(t, n, d_theta, d_z, d_a1, d_a2, d_sel, d_rate);
+  return s == KMC_OK && n > 0 ? transfer_wait(t) : s;
 }
 
 int kmc_transfer_rates(kmc_transfer* t, int64_t n, const double* theta, const double* z,
