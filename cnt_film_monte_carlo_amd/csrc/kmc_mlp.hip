@@ -6,13 +6,14 @@
 // log10 rate.  All products run on the CDNA4 matrix cores as v_mfma_f32_32x32x16_bf16 with BF16
 // operands and FP32 accumulation; master weights, biases and the output layer are FP32.
 //
-// Training (layer by layer, activations in HBM, L2-resident at these batch sizes):
-//   forward   Z_l = H_{l-1} W_l + b_l, H_l = bf16(silu(Z_l))         k_gemm<.., EPI_FWD>
-//   head      y = H_3 . w4 + b4, dy = 2 (y - t) / n,
-//             dZ_3 = bf16(dy w4 silu'(Z_3))                           k_head
-//   backward  dW_l = H_{l-1}^T dZ_l (split over the batch, summed in a fixed order),
-//             db_l = colsum(dZ_l), dZ_{l-1} = bf16((dZ_l W_l^T) silu'(Z_{l-1}))
-//   Adam on the FP32 masters, which refreshes both BF16 copies W_l and W_l^T.
+// A training step is three launches (activations and gradients of a tile stay on the chip):
+//   k_mlp_rows   32 rows per workgroup through the whole network and back:
+//                Z_l = H_{l-1} W_l + b_l, H_l = bf16(silu(Z_l)), y = H_3 . w4 + b4,
+//                dy = 2 (y - t) / n, dZ_3 = bf16(dy w4 silu'(Z_3)),
+//                dZ_{l-1} = bf16((dZ_l W_l^T) silu'(Z_{l-1})); leaves H_l and dZ_l, transposed
+//   k_mlp_grads  dW_l = H_{l-1}^T dZ_l in splits over the batch, db_l, dw4, db4 in row blocks
+//   k_mlp_update the splits' and blocks' sums in a fixed order, then Adam on the FP32 masters,
+//                which refreshes both BF16 copies W_l and W_l^T.
 // Inference: one fused kernel, one 32-pair tile per wave.  The BF16 weights (100 KB) sit in LDS,
 // pre-arranged as MFMA A fragments; activations never leave registers because the hidden units
 // of layers 1..3 are taken in the order in which the accumulator of the previous layer holds
@@ -23,7 +24,10 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/cntkmc.h"
@@ -113,130 +117,264 @@ __host__ __device__ inline int64_t bin_index(const int32_t* dims, int cd, int ca
 // ---------------------------------------------------------------------------------------------
 // training kernels
 // ---------------------------------------------------------------------------------------------
-enum { EPI_FWD = 0, EPI_DH = 1, EPI_PART = 2 };
+constexpr int TILE = 32;            // rows of one workgroup of k_mlp_rows
+constexpr int K_SPLIT = 512;        // batch rows per split of the weight-gradient products
+constexpr int LOSS_PARTS = 256;     // partial sums of the squared error
+constexpr int COL_BLOCKS = 64;      // row blocks of the bias and output-layer gradients
+constexpr int COLS = NH * WD + WD + 1;  // their columns: db_0..db_3, dw4, db4
+constexpr int XS = WD + 8;          // LDS row of one sample's activations (padded: no bank conflicts)
+constexpr int LEAVES = 72;          // LDS row of one sample's 64 products of the output unit
 
-struct gemm_args {
-  int M, N, K, k_split;
-  const bf16* A;  // element (m, k): AT ? A[k * lda + m] : A[m * lda + k]
-  int lda;
-  const bf16* B;  // element (n, k) of B^T: BT ? B[k * ldb + n] : B[n * ldb + k]
-  int ldb;
-  const float* bias;   // EPI_FWD: Z = C + bias[n], H = bf16(silu(Z))
-  float* Z;
-  bf16* H;
-  const float* Zprev;  // EPI_DH: dZ = bf16(C * silu'(Zprev))
-  bf16* dZ;
-  float* part;         // EPI_PART: part[blockIdx.z][M][N] = C over this block's K range
+struct rows_args {
+  int n_valid;            // rows beyond have no target
+  const int32_t* idx;     // optional: batch row r is row idx[r] of X and tgt
+  const bf16* X;          // [rows][IN]
+  const float* tgt;
+  float inv_n;
+  const bf16 *Wtb, *Wb;   // W_l^T and W_l
+  const float* prm;
+  int64_t ld;             // rows of the transposed arrays
+  bf16 *XT, *HT, *DT;     // X^T [IN][ld], H_l^T and dZ_l^T [NH][WD][ld]
+  float *y, *dy, *err;
 };
 
-// C[M][N] = A B^T with K a multiple of 16.  Four waves per workgroup, each a 32 x 32 tile of
-// one MFMA accumulator; rows/columns beyond M/N read zeros and are not stored.
-template <bool AT, bool BT, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(gemm_args g) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int h = lane >> 5, c = lane & 31;
-  const int m0 = blockIdx.y * 64 + (w >> 1) * 32, n0 = blockIdx.x * 64 + (w & 1) * 32;
-  if (m0 >= g.M || n0 >= g.N) return;
-  const int k_lo = blockIdx.z * g.k_split, k_hi = min(g.K, k_lo + g.k_split);
-  const int am = m0 + c, bn = n0 + c;
-  const bool a_ok = am < g.M, b_ok = bn < g.N;
-  f32x16 acc = {};
-  for (int k0 = k_lo; k0 < k_hi; k0 += 16) {
-    const int kk = k0 + 8 * h;
-    bf16x8 a = {}, b = {};
-    if (a_ok) {
-      if (AT) {
+__device__ __forceinline__ float lane_swap(float x) {  // the value of lane i ^ 1
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0xB1, 0xF, 0xF, true));
+}
+
+// One wave's 32 rows x 32 units as the accumulator holds them (register r of lane (h, c): row
+// 8 (r / 4) + 4 h + r % 4, unit n = 32 wave + c): to LDS for the next layer's A operand (a
+// sample's units side by side) and, transposed, to memory for the weight gradients.
+__device__ __forceinline__ void put_tile(const bf16 (&v)[16], bf16 (*xa)[XS], int n, int h,
+                                         bf16* __restrict__ T, int64_t ld, int64_t row0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) a[e] = g.A[(int64_t)(kk + e) * g.lda + am];
-      } else {
-        a = *reinterpret_cast<const bf16x8*>(g.A + (int64_t)am * g.lda + kk);
-      }
-    }
-    if (b_ok) {
-      if (BT) {
+  for (int q = 0; q < 4; ++q) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    bf16x4 p;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) b[e] = g.B[(int64_t)(kk + e) * g.ldb + bn];
-      } else {
-        b = *reinterpret_cast<const bf16x8*>(g.B + (int64_t)bn * g.ldb + kk);
-      }
+    for (int j = 0; j < 4; ++j) {
+      xa[8 * q + 4 * h + j][n] = v[4 * q + j];
+      p[j] = v[4 * q + j];
     }
-    acc = mfma32(a, b, acc);
+    if (T) *reinterpret_cast<bf16x4*>(T + (int64_t)n * ld + row0 + 8 * q + 4 * h) = p;
   }
+}
+
+__device__ __forceinline__ f32x16 layer_product(const bf16 (*xa)[XS], int c, int h,
+                                                const bf16x8 (&w)[8]) {
+  f32x16 acc = {};
+#pragma unroll
+  for (int kb = 0; kb < 8; ++kb)
+    acc = mfma32(*reinterpret_cast<const bf16x8*>(&xa[c][16 * kb + 8 * h]), w[kb], acc);
+  return acc;
+}
+
+// 32 rows per workgroup, 32 units of every layer per wave: the four waves exchange a layer's
+// activations through LDS, and each holds its weight fragments (read from L2 ahead of their use),
+// pre-activations and gradients in registers.  A batch of 8,192 rows is 256 workgroups, one per
+// CU; what bounds it is the chain of seven layers, each eight MFMAs, an LDS exchange and sixteen
+// SiLUs or their derivatives per lane.  The products run in the order of k (16 per MFMA) with the
+// samples as A operand, and the output unit's 128 products are added in the order of a butterfly
+// over 64 pairs of units, so that a batch's results do not depend on how it is tiled.
+template <bool GRAD>
+__global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
+  __shared__ __align__(16) bf16 xa[2][TILE][XS];
+  __shared__ float leaf[TILE][LEAVES];
+  __shared__ float s_d[TILE];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, h = lane >> 5, c = lane & 31;
+  const int n = 32 * wv + c;
+  const int64_t row0 = (int64_t)blockIdx.x * TILE, row = row0 + c;
+  const int64_t src = g.idx ? g.idx[row] : row;
+  const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(g.X + src * IN + 8 * h);
+  const bf16x8 w0 = *reinterpret_cast<const bf16x8*>(g.Wtb + (int64_t)n * IN + 8 * h);
+  bf16x8 wf[3][8];
+#pragma unroll
+  for (int l = 1; l < NH; ++l)
+#pragma unroll
+    for (int kb = 0; kb < 8; ++kb)
+      wf[l - 1][kb] = *reinterpret_cast<const bf16x8*>(g.Wtb + q_off(l) + (int64_t)n * WD + 16 * kb + 8 * h);
+  if (GRAD && wv == 0) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g.XT[(int64_t)(8 * h + e) * g.ld + row] = a0[e];
+  }
+  float z[NH][16];
+  bf16 v[16];
+  f32x16 acc = {};
+#pragma unroll
+  for (int l = 0; l < NH; ++l) {
+    if (l == 0) {
+      acc = mfma32(a0, w0, acc);
+    } else {
+      __syncthreads();
+      acc = layer_product(xa[(l - 1) & 1], c, h, wf[l - 1]);
+    }
+    const float bias = g.prm[b_off(l) + n];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      z[l][r] = acc[r] + bias;
+      v[r] = (bf16)silu_f(z[l][r]);
+    }
+    if (l + 1 < NH || GRAD)
+      put_tile(v, xa[l & 1], n, h, GRAD ? g.HT + (int64_t)l * WD * g.ld : nullptr, g.ld, row0);
+  }
+  // the weights of the way back, read while the output unit is summed
+  bf16x8 wb[3][8];
+  if (GRAD) {
+#pragma unroll
+    for (int l = 1; l < NH; ++l)
+#pragma unroll
+      for (int kb = 0; kb < 8; ++kb)
+        wb[l - 1][kb] = *reinterpret_cast<const bf16x8*>(g.Wb + q_off(l) + (int64_t)n * WD + 16 * kb + 8 * h);
+  }
+  const float wa = g.prm[W4_OFF + n], wo = lane_swap(wa);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    const int row = m0 + 8 * (r >> 2) + 4 * h + (r & 3), col = n0 + c;
-    if (row >= g.M || col >= g.N) continue;
-    const int64_t o = (int64_t)row * g.N + col;
-    if (EPI == EPI_FWD) {
-      const float v = acc[r] + g.bias[col];
-      g.Z[o] = v;
-      g.H[o] = (bf16)silu_f(v);
-    } else if (EPI == EPI_DH) {
-      g.dZ[o] = (bf16)(acc[r] * dsilu_f(g.Zprev[o]));
-    } else {
-      g.part[(int64_t)blockIdx.z * g.M * g.N + o] = acc[r];
-    }
+    const float hv = (float)v[r], ho = lane_swap(hv);
+    if (!(c & 1)) leaf[8 * (r >> 2) + 4 * h + (r & 3)][n >> 1] = fmaf(hv, wa, ho * wo);
   }
-}
-
-// y = h3 . w4 + b4 per row (one wave per row, the 128 products reduced by a butterfly).  With
-// targets: dy = 2 (y - t) / n_valid for rows < n_valid (0 beyond), dZ3 = bf16(dy w4 silu'(Z3)),
-// and loss_part[wave] = sum of (y - t)^2 over the wave's rows.
-__global__ __launch_bounds__(256) void k_head(int n, int n_valid, const bf16* __restrict__ H3,
-                                              const float* __restrict__ Z3, const float* __restrict__ prm,
-                                              const float* __restrict__ tgt, float inv_n, float* y,
-                                              float* dy, bf16* dZ3, double* loss_part) {
-  const int lane = threadIdx.x & 63;
-  const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int nw = (gridDim.x * blockDim.x) >> 6;
-  const float wa = prm[W4_OFF + 2 * lane], wb = prm[W4_OFF + 2 * lane + 1], b4 = prm[B4_OFF];
-  double lsum = 0.0;
-  for (int s = wave; s < n; s += nw) {
-    const bf16* hr = H3 + (int64_t)s * WD;
-    float p = (float)hr[2 * lane] * wa + (float)hr[2 * lane + 1] * wb;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) p += __shfl_xor(p, off, 64);
-    const float yy = p + b4;
-    if (lane == 0) y[s] = yy;
-    if (tgt) {
-      const float e = s < n_valid ? yy - tgt[s] : 0.0f;
-      const float d = 2.0f * e * inv_n;
-      if (lane == 0) {
-        dy[s] = d;
-        lsum += (double)e * (double)e;
-      }
-      const float* zr = Z3 + (int64_t)s * WD;
-      dZ3[(int64_t)s * WD + 2 * lane] = (bf16)(d * wa * dsilu_f(zr[2 * lane]));
-      dZ3[(int64_t)s * WD + 2 * lane + 1] = (bf16)(d * wb * dsilu_f(zr[2 * lane + 1]));
-    }
-  }
-  if (loss_part && lane == 0) loss_part[wave] = lsum;
-}
-
-// part[block][j] = sum over the block's rows r of (X ? X[r][j] : 1) * (w ? w[r] : 1), cols <= 128.
-__global__ __launch_bounds__(256) void k_colsum(int n, int cols, const bf16* __restrict__ X,
-                                                const float* __restrict__ w, int chunk, float* part) {
-  __shared__ float s[256];
-  const int t = threadIdx.x, j = t & 127, half = t >> 7;
-  const int r0 = blockIdx.x * chunk, r1 = min(n, r0 + chunk);
-  float acc = 0.0f;
-  if (j < cols)
-    for (int r = r0 + half; r < r1; r += 2) {
-      const float x = X ? (float)X[(int64_t)r * cols + j] : 1.0f;
-      acc += w ? x * w[r] : x;
-    }
-  s[t] = acc;
   __syncthreads();
-  if (t < cols) part[(int64_t)blockIdx.x * cols + t] = s[t] + s[t + 128];
+  {
+    const int s = threadIdx.x >> 3, p = threadIdx.x & 7;
+    float u[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) u[q] = leaf[s][8 * q + p];
+    float t = ((u[0] + u[4]) + (u[2] + u[6])) + ((u[1] + u[5]) + (u[3] + u[7]));
+    t += __shfl_xor(t, 4, 64);
+    t += __shfl_xor(t, 2, 64);
+    t += __shfl_xor(t, 1, 64);
+    const float yy = t + g.prm[B4_OFF];
+    if (p == 0) {
+      const int64_t q = row0 + s;
+      g.y[q] = yy;
+      if (GRAD) {
+        const float e = q < g.n_valid ? yy - g.tgt[g.idx ? g.idx[q] : q] : 0.0f;
+        const float d = 2.0f * e * g.inv_n;
+        g.dy[q] = d;
+        g.err[q] = e;
+        s_d[s] = d;
+      }
+    }
+  }
+  if (!GRAD) return;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    v[r] = (bf16)(s_d[8 * (r >> 2) + 4 * h + (r & 3)] * wa * dsilu_f(z[NH - 1][r]));
+  put_tile(v, xa[0], n, h, g.DT + (int64_t)(NH - 1) * WD * g.ld, g.ld, row0);
+#pragma unroll
+  for (int l = NH - 1; l >= 1; --l) {
+    __syncthreads();
+    acc = layer_product(xa[(NH - 1 - l) & 1], c, h, wb[l - 1]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = (bf16)(acc[r] * dsilu_f(z[l - 1][r]));
+    put_tile(v, xa[(NH - l) & 1], n, h, g.DT + (int64_t)(l - 1) * WD * g.ld, g.ld, row0);
+  }
 }
 
-// out[i] = sum_{z < nz} part[z][i], in order.
-__global__ void k_sum_parts(int64_t len, int nz, const float* __restrict__ part, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= len) return;
+struct grads_args {
+  int nb, nz;             // rows (a multiple of 128) and splits of K_SPLIT rows
+  int64_t ld;
+  const bf16 *XT, *HT, *DT;
+  const float *dy, *err;
+  float* part;            // weight layer l: nz q_off(l) + [nz][fan_in][WD]
+  float* cpart;           // [COL_BLOCKS][COLS]
+  double* lpart;          // [LOSS_PARTS]
+};
+
+// Blocks [0, 13 nz): dW tiles.  A wave takes 32 x 32 weights over one split's rows, 16 per MFMA in
+// row order, both operands 16 contiguous bytes of a transposed array per lane; layer 0 has one
+// 32-row tile (16 features), the others four.  Then 3 COL_BLOCKS blocks of column sums (a thread
+// per column, even and odd rows apart) and one block for the squared error.  832 waves and 192
+// small blocks at 8,192 rows: bound by the latency of a split's chain of 32 MFMAs and its loads.
+__global__ __launch_bounds__(256) void k_mlp_grads(grads_args g) {
+#pragma clang fp contract(off)
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, h = lane >> 5, c = lane & 31;
+  int b = blockIdx.x;
+  if (b < 13 * g.nz) {
+    const int zi = b / 13, x = b % 13;
+    const int l = x == 0 ? 0 : 1 + (x - 1) / 4, mt = x == 0 ? 0 : (x - 1) % 4;
+    const int m = 32 * mt + c, n = 32 * wv + c;
+    const bf16* A = (l == 0 ? g.XT : g.HT + (int64_t)(l - 1) * WD * g.ld) + (int64_t)m * g.ld;
+    const bf16* B = g.DT + ((int64_t)l * WD + n) * g.ld;
+    const bool a_ok = m < fan_in(l);
+    const int k_lo = zi * K_SPLIT, k_hi = min(g.nb, k_lo + K_SPLIT);
+    f32x16 acc = {};
+    for (int k0 = k_lo; k0 < k_hi; k0 += 128) {  // nb and K_SPLIT are multiples of 128
+      bf16x8 av[8], bv[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int k = k0 + 16 * q + 8 * h;
+        av[q] = bf16x8{};
+        if (a_ok) av[q] = *reinterpret_cast<const bf16x8*>(A + k);
+        bv[q] = *reinterpret_cast<const bf16x8*>(B + k);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc = mfma32(av[q], bv[q], acc);
+    }
+    float* out = g.part + (int64_t)g.nz * q_off(l) + (int64_t)zi * fan_in(l) * WD;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
+      if (row < fan_in(l)) out[(int64_t)row * WD + n] = acc[r];
+    }
+    return;
+  }
+  b -= 13 * g.nz;
+  if (b < 3 * COL_BLOCKS) {
+    const int blk = b / 3, col = 256 * (b % 3) + t;
+    if (col >= COLS) return;
+    const int chunk = (g.nb + COL_BLOCKS - 1) / COL_BLOCKS;  // even: nb is a multiple of 128
+    const int r0 = blk * chunk, r1 = min(g.nb, r0 + chunk);
+    float s0 = 0.0f, s1 = 0.0f;
+    const bf16* x = col < NH * WD ? g.DT + (int64_t)col * g.ld
+                                  : g.HT + ((int64_t)(NH - 1) * WD + (col - NH * WD)) * g.ld;
+    if (col < NH * WD) {
+      for (int r = r0; r < r1; r += 2) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 v = *reinterpret_cast<const bf16x2*>(x + r);
+        s0 = s0 + (float)v[0];
+        s1 = s1 + (float)v[1];
+      }
+    } else {
+      const bool last = col == COLS - 1;  // db4: the sum of dy
+      for (int r = r0; r < r1; r += 2) {
+        s0 = s0 + (last ? 1.0f : (float)x[r]) * g.dy[r];
+        s1 = s1 + (last ? 1.0f : (float)x[r + 1]) * g.dy[r + 1];
+      }
+    }
+    g.cpart[(int64_t)blk * COLS + col] = s0 + s1;
+    return;
+  }
+  double s = 0.0;
+  for (int r = t; r < g.nb; r += LOSS_PARTS) s = s + (double)g.err[r] * (double)g.err[r];
+  g.lpart[t] = s;
+}
+
+// Sum of parameter p's gradient over the splits or row blocks, in order.
+__device__ __forceinline__ float sum_parts(int64_t p, int nz, const float* __restrict__ part,
+                                           const float* __restrict__ cpart) {
   float a = 0.0f;
-  for (int z = 0; z < nz; ++z) a += part[(int64_t)z * len + i];
-  out[i] = a;
+  int col = -1;
+#pragma unroll
+  for (int l = 0; l < NH; ++l) {
+    if (p >= w_off(l) && p < b_off(l)) {
+      const int64_t len = (int64_t)fan_in(l) * WD;
+      const float* q = part + (int64_t)nz * q_off(l) + (p - w_off(l));
+      for (int z = 0; z < nz; ++z) a += q[z * len];
+      return a;
+    }
+    if (p >= b_off(l) && p < b_off(l) + WD) col = l * WD + (int)(p - b_off(l));
+  }
+  if (col < 0) col = NH * WD + (int)(p - W4_OFF);  // w4, then b4
+#pragma unroll 8
+  for (int z = 0; z < COL_BLOCKS; ++z) a += cpart[(int64_t)z * COLS + col];
+  return a;
+}
+
+__global__ void k_mlp_sum(int nz, const float* __restrict__ part, const float* __restrict__ cpart,
+                          float* __restrict__ grad) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < NP) grad[p] = sum_parts(p, nz, part, cpart);
 }
 
 __device__ __forceinline__ void write_copies(int64_t p, float w, bf16* Wb, bf16* Wtb) {
@@ -256,18 +394,31 @@ __global__ void k_refresh(const float* __restrict__ prm, bf16* Wb, bf16* Wtb) {
 }
 
 // Adam with bias corrections c1 = 1 / (1 - beta1^t), c2 = 1 / (1 - beta2^t).
-__global__ void k_adam(float* prm, const float* __restrict__ grad, float* m, float* v, float lr,
-                       float b1, float b2, float eps, float c1, float c2, bf16* Wb, bf16* Wtb) {
+struct adam_args {
+  float *prm, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+  bf16 *Wb, *Wtb;
+};
+
+__device__ __forceinline__ void adam_update(const adam_args& o, int64_t p, float g) {
+  const float mm = o.b1 * o.m[p] + (1.0f - o.b1) * g;
+  const float vv = o.b2 * o.v[p] + (1.0f - o.b2) * g * g;
+  o.m[p] = mm;
+  o.v[p] = vv;
+  const float w = o.prm[p] - o.lr * (mm * o.c1) / (sqrtf(vv * o.c2) + o.eps);
+  o.prm[p] = w;
+  write_copies(p, w, o.Wb, o.Wtb);
+}
+
+__global__ void k_adam(adam_args o, const float* __restrict__ grad) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= NP) return;
-  const float g = grad[p];
-  const float mm = b1 * m[p] + (1.0f - b1) * g;
-  const float vv = b2 * v[p] + (1.0f - b2) * g * g;
-  m[p] = mm;
-  v[p] = vv;
-  const float w = prm[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
-  prm[p] = w;
-  write_copies(p, w, Wb, Wtb);
+  if (p < NP) adam_update(o, p, grad[p]);
+}
+
+__global__ void k_mlp_update(adam_args o, int nz, const float* __restrict__ part,
+                             const float* __restrict__ cpart) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < NP) adam_update(o, p, sum_parts(p, nz, part, cpart));
 }
 
 __global__ void k_to_bf16(int64_t n, const float* __restrict__ x, bf16* y) {
@@ -275,17 +426,11 @@ __global__ void k_to_bf16(int64_t n, const float* __restrict__ x, bf16* y) {
   if (i < n) y[i] = (bf16)x[i];
 }
 
-// rows idx[r] of the data set into the batch
-__global__ void k_gather(int nb, const int32_t* __restrict__ idx, const bf16* __restrict__ dx,
-                         const float* __restrict__ dt, bf16* X, float* tgt) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nb) return;
-  const int64_t s = idx[r];
-  const bf16x8* src = reinterpret_cast<const bf16x8*>(dx + s * IN);
-  bf16x8* dst = reinterpret_cast<bf16x8*>(X + (int64_t)r * IN);
-  dst[0] = src[0];
-  dst[1] = src[1];
-  tgt[r] = dt[s];
+// An epoch's order of the rows: the shuffle pi applied to the order before it.
+__global__ void k_reorder(int64_t n, const int32_t* __restrict__ before, const int32_t* __restrict__ pi,
+                          int32_t* __restrict__ after) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) after[i] = before ? before[pi[i]] : pi[i];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -494,10 +639,8 @@ struct kmc_mlp {
   int64_t cap = 0;
   bf16* X = nullptr;
   float* tgt = nullptr;
-  float* Z[NH] = {};
-  bf16* H[NH] = {};
-  float *y = nullptr, *dy = nullptr;
-  bf16 *dZa = nullptr, *dZb = nullptr;
+  bf16 *XT = nullptr, *HT = nullptr, *DT = nullptr;
+  float *y = nullptr, *dy = nullptr, *err = nullptr;
   float *part = nullptr, *cpart = nullptr;
   double* lpart = nullptr;
   float* fstage = nullptr;  // FP32 staging of host feature rows
@@ -509,10 +652,6 @@ struct kmc_mlp {
 };
 
 namespace {
-
-constexpr int K_SPLIT = 512;    // batch rows per split of the weight-gradient products
-constexpr int HEAD_WAVES = 256; // waves of k_head (its loss_part length)
-constexpr int COL_BLOCKS = 64;  // row blocks of k_colsum
 
 #define MLP_HIP(call)                                                                      \
   do {                                                                                     \
@@ -536,111 +675,90 @@ int ensure_cap(kmc_mlp* m, int64_t rows) {
   if (rows <= m->cap) return KMC_OK;
   MLP_HIP(grow(&m->X, rows * IN));
   MLP_HIP(grow(&m->tgt, rows));
-  for (int l = 0; l < NH; ++l) {
-    MLP_HIP(grow(&m->Z[l], rows * WD));
-    MLP_HIP(grow(&m->H[l], rows * WD));
-  }
+  m->cap = 0;
+  MLP_HIP(grow(&m->XT, rows * IN));
+  MLP_HIP(grow(&m->HT, rows * WD * NH));
+  MLP_HIP(grow(&m->DT, rows * WD * NH));
   MLP_HIP(grow(&m->y, rows));
   MLP_HIP(grow(&m->dy, rows));
-  MLP_HIP(grow(&m->dZa, rows * WD));
-  MLP_HIP(grow(&m->dZb, rows * WD));
-  MLP_HIP(grow(&m->part, round_up(rows, K_SPLIT) / K_SPLIT * WD * WD));
+  MLP_HIP(grow(&m->err, rows));
+  MLP_HIP(grow(&m->part, round_up(rows, K_SPLIT) / K_SPLIT * NQ));
   MLP_HIP(grow(&m->fstage, rows * IN));
   m->cap = rows;
   return KMC_OK;
 }
 
-hipError_t launch_gemm(const gemm_args& g, bool at, bool bt, int epi, hipStream_t st) {
-  const int nz = (g.K + g.k_split - 1) / g.k_split;
-  const dim3 grid((g.N + 63) / 64, (g.M + 63) / 64, nz);
-  if (!at && !bt && epi == EPI_FWD) hipLaunchKernelGGL((k_gemm<false, false, EPI_FWD>), grid, dim3(256), 0, st, g);
-  else if (!at && !bt && epi == EPI_DH) hipLaunchKernelGGL((k_gemm<false, false, EPI_DH>), grid, dim3(256), 0, st, g);
-  else if (at && bt && epi == EPI_PART) hipLaunchKernelGGL((k_gemm<true, true, EPI_PART>), grid, dim3(256), 0, st, g);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
+int splits(int nb) { return (nb + K_SPLIT - 1) / K_SPLIT; }
 
-hipError_t colsum(kmc_mlp* m, int n, int cols, const bf16* X, const float* w, float* out) {
-  const int chunk = (n + COL_BLOCKS - 1) / COL_BLOCKS;
-  hipLaunchKernelGGL(k_colsum, dim3(COL_BLOCKS), dim3(256), 0, m->stream, n, cols, X, w, chunk, m->cpart);
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(128), 0, m->stream, (int64_t)cols, COL_BLOCKS, m->cpart, out);
-  return hipGetLastError();
-}
-
-// Forward over rows [0, nb) of m->X; with targets also the head gradient, backward and the
-// gradient in m->d_grad.  nb is a multiple of 128.
-hipError_t step(kmc_mlp* m, int nb, int n_valid, bool backward) {
+// Forward over nb rows (a multiple of 128) of X, or of the rows idx of X; with `backward` also
+// the parts of the gradient and the squared error's sums in lpart.
+hipError_t step(kmc_mlp* m, int nb, int n_valid, bool backward, const bf16* X, const float* tgt,
+                const int32_t* idx, double* lpart) {
   hipStream_t st = m->stream;
-  for (int l = 0; l < NH; ++l) {
-    gemm_args g{};
-    g.M = nb;
-    g.N = WD;
-    g.K = fan_in(l);
-    g.k_split = g.K;
-    g.A = l == 0 ? m->X : m->H[l - 1];
-    g.lda = fan_in(l);
-    g.B = m->d_wtb + q_off(l);
-    g.ldb = fan_in(l);
-    g.bias = m->d_prm + b_off(l);
-    g.Z = m->Z[l];
-    g.H = m->H[l];
-    hipError_t e = launch_gemm(g, false, false, EPI_FWD, st);
-    if (e != hipSuccess) return e;
+  rows_args g{};
+  g.n_valid = n_valid;
+  g.idx = idx;
+  g.X = X;
+  g.tgt = tgt;
+  g.inv_n = 1.0f / (float)std::max(n_valid, 1);
+  g.Wtb = m->d_wtb;
+  g.Wb = m->d_wb;
+  g.prm = m->d_prm;
+  g.ld = m->cap;
+  g.XT = m->XT;
+  g.HT = m->HT;
+  g.DT = m->DT;
+  g.y = m->y;
+  g.dy = m->dy;
+  g.err = m->err;
+  const dim3 grid((unsigned)(nb / TILE));
+  if (!backward) {
+    hipLaunchKernelGGL(k_mlp_rows<false>, grid, dim3(256), 0, st, g);
+    return hipGetLastError();
   }
-  hipLaunchKernelGGL(k_head, dim3(HEAD_WAVES / 4), dim3(256), 0, st, nb, n_valid, m->H[NH - 1],
-                     m->Z[NH - 1], m->d_prm, backward ? m->tgt : nullptr,
-                     1.0f / (float)std::max(n_valid, 1), m->y, m->dy, m->dZa,
-                     backward ? m->lpart : nullptr);
+  hipLaunchKernelGGL(k_mlp_rows<true>, grid, dim3(256), 0, st, g);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || !backward) return e;
-  e = colsum(m, nb, WD, m->H[NH - 1], m->dy, m->d_grad + W4_OFF);
-  if (e == hipSuccess) e = colsum(m, nb, 1, nullptr, m->dy, m->d_grad + B4_OFF);
-  bf16 *dz = m->dZa, *dz_next = m->dZb;
-  for (int l = NH - 1; l >= 0 && e == hipSuccess; --l) {
-    gemm_args g{};
-    g.M = fan_in(l);
-    g.N = WD;
-    g.K = nb;
-    g.k_split = K_SPLIT;
-    g.A = l == 0 ? m->X : m->H[l - 1];
-    g.lda = fan_in(l);
-    g.B = dz;
-    g.ldb = WD;
-    g.part = m->part;
-    e = launch_gemm(g, true, true, EPI_PART, st);
-    if (e != hipSuccess) break;
-    const int64_t len = (int64_t)fan_in(l) * WD;
-    const int nz = (nb + K_SPLIT - 1) / K_SPLIT;
-    hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, st, len, nz,
-                       m->part, m->d_grad + w_off(l));
-    e = colsum(m, nb, WD, dz, nullptr, m->d_grad + b_off(l));
-    if (e != hipSuccess || l == 0) break;
-    gemm_args d{};
-    d.M = nb;
-    d.N = fan_in(l);
-    d.K = WD;
-    d.k_split = WD;
-    d.A = dz;
-    d.lda = WD;
-    d.B = m->d_wb + q_off(l);
-    d.ldb = WD;
-    d.Zprev = m->Z[l - 1];
-    d.dZ = dz_next;
-    e = launch_gemm(d, false, false, EPI_DH, st);
-    std::swap(dz, dz_next);
-  }
-  return e;
+  if (e != hipSuccess) return e;
+  grads_args q{};
+  q.nb = nb;
+  q.nz = splits(nb);
+  q.ld = m->cap;
+  q.XT = m->XT;
+  q.HT = m->HT;
+  q.DT = m->DT;
+  q.dy = m->dy;
+  q.err = m->err;
+  q.part = m->part;
+  q.cpart = m->cpart;
+  q.lpart = lpart;
+  hipLaunchKernelGGL(k_mlp_grads, dim3((unsigned)(13 * q.nz + 3 * COL_BLOCKS + 1)), dim3(256), 0, st, q);
+  return hipGetLastError();
 }
 
-hipError_t adam(kmc_mlp* m, double lr, double b1, double b2, double eps) {
+constexpr unsigned PARAM_BLOCKS = (unsigned)((NP + 255) / 256);
+
+adam_args next_adam(kmc_mlp* m, double lr, double b1, double b2, double eps) {
   ++m->adam_t;
   const double c1 = 1.0 / (1.0 - std::pow(b1, (double)m->adam_t));
   const double c2 = 1.0 / (1.0 - std::pow(b2, (double)m->adam_t));
-  hipLaunchKernelGGL(k_adam, dim3((unsigned)((NP + 255) / 256)), dim3(256), 0, m->stream, m->d_prm,
-                     m->d_grad, m->d_m, m->d_v, (float)lr, (float)b1, (float)b2, (float)eps,
-                     (float)c1, (float)c2, m->d_wb, m->d_wtb);
   m->pk_dirty = true;
-  return hipGetLastError();
+  return adam_args{m->d_prm,  m->d_m,      m->d_v,    (float)lr, (float)b1, (float)b2,
+                   (float)eps, (float)c1, (float)c2, m->d_wb,   m->d_wtb};
+}
+
+// One epoch's Fisher-Yates shuffle as a permutation of [0, n): the n - 1 draws of the splitmix64
+// stream that start after `skip` draws.
+void shuffle(int64_t n, uint64_t seed, uint64_t skip, int32_t* pi) {
+  constexpr uint64_t STEP = 0x9E3779B97F4A7C15ull;
+  for (int64_t i = 0; i < n; ++i) pi[i] = (int32_t)i;
+  uint64_t rs = (seed ^ STEP) + skip * STEP;
+  for (int64_t i = n - 1; i > 0; --i) {
+    uint64_t z = (rs += STEP);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    std::swap(pi[i], pi[z % (uint64_t)(i + 1)]);
+  }
 }
 
 // feature rows (host FP32) -> m->X (BF16) with rows [n, nb) zero
@@ -788,8 +906,8 @@ int kmc_mlp_create(int32_t device, const kmc_mlp_domain* dom, kmc_mlp** out) {
   if (e == hipSuccess) e = grow(&m->d_wb, NQ);
   if (e == hipSuccess) e = grow(&m->d_wtb, NQ);
   if (e == hipSuccess) e = grow(&m->d_pk, NQ);
-  if (e == hipSuccess) e = grow(&m->cpart, COL_BLOCKS * WD);
-  if (e == hipSuccess) e = grow(&m->lpart, HEAD_WAVES);
+  if (e == hipSuccess) e = grow(&m->cpart, (size_t)COL_BLOCKS * COLS);
+  if (e == hipSuccess) e = grow(&m->lpart, LOSS_PARTS);
   for (float* b : {m->d_prm, m->d_grad, m->d_m, m->d_v})
     if (e == hipSuccess) e = hipMemsetAsync(b, 0, NP * sizeof(float), m->stream);
   if (e == hipSuccess) {
@@ -811,14 +929,11 @@ int kmc_mlp_destroy(kmc_mlp* m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   void* bufs[] = {m->d_prm, m->d_grad, m->d_m,  m->d_v,  m->d_wb,    m->d_wtb, m->d_pk,
-                  m->d_rmap, m->X,     m->tgt,  m->y,    m->dy,      m->dZa,   m->dZb,
-                  m->part,  m->cpart,  m->lpart, m->fstage, m->d_geo, m->d_rate, m->d_flag};
+                  m->d_rmap, m->X,     m->tgt,  m->y,    m->dy,      m->err,   m->XT,
+                  m->HT,    m->DT,     m->part, m->cpart, m->lpart,  m->fstage, m->d_geo,
+                  m->d_rate, m->d_flag};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
-  for (int l = 0; l < NH; ++l) {
-    if (m->Z[l]) (void)hipFree(m->Z[l]);
-    if (m->H[l]) (void)hipFree(m->H[l]);
-  }
   if (m->ev0) (void)hipEventDestroy(m->ev0);
   if (m->ev1) (void)hipEventDestroy(m->ev1);
   if (m->stream) (void)hipStreamDestroy(m->stream);
@@ -899,7 +1014,7 @@ int kmc_mlp_forward(kmc_mlp* m, int64_t n, const float* feat, float* y) {
     int st = ensure_cap(m, nb);
     if (st == KMC_OK) st = load_rows(m, k, nb, feat + s * IN, nullptr);
     if (st != KMC_OK) return st;
-    MLP_HIP(step(m, (int)nb, (int)k, false));
+    MLP_HIP(step(m, (int)nb, (int)k, false, m->X, nullptr, nullptr, nullptr));
     MLP_HIP(hipMemcpyAsync(y + s, m->y, k * sizeof(float), hipMemcpyDeviceToHost, m->stream));
     MLP_HIP(hipStreamSynchronize(m->stream));
   }
@@ -915,9 +1030,12 @@ int kmc_mlp_loss_grad(kmc_mlp* m, int64_t n, const float* feat, const float* tar
   int st = ensure_cap(m, nb);
   if (st == KMC_OK) st = load_rows(m, n, nb, feat, targets);
   if (st != KMC_OK) return st;
-  MLP_HIP(step(m, (int)nb, (int)n, true));
-  std::vector<double> lp(HEAD_WAVES);
-  MLP_HIP(hipMemcpyAsync(lp.data(), m->lpart, HEAD_WAVES * sizeof(double), hipMemcpyDeviceToHost, m->stream));
+  MLP_HIP(step(m, (int)nb, (int)n, true, m->X, m->tgt, nullptr, m->lpart));
+  hipLaunchKernelGGL(k_mlp_sum, dim3(PARAM_BLOCKS), dim3(256), 0, m->stream, splits((int)nb), m->part,
+                     m->cpart, m->d_grad);
+  MLP_HIP(hipGetLastError());
+  std::vector<double> lp(LOSS_PARTS);
+  MLP_HIP(hipMemcpyAsync(lp.data(), m->lpart, LOSS_PARTS * sizeof(double), hipMemcpyDeviceToHost, m->stream));
   if (grad) MLP_HIP(hipMemcpyAsync(grad, m->d_grad, NP * sizeof(float), hipMemcpyDeviceToHost, m->stream));
   MLP_HIP(hipStreamSynchronize(m->stream));
   if (loss) {
@@ -934,7 +1052,9 @@ int kmc_mlp_adam_step(kmc_mlp* m, const float* grad, double lr, double b1, doubl
   MLP_HIP(hipSetDevice(m->device));
   MLP_HIP(hipMemcpyAsync(m->d_grad, grad, NP * sizeof(float), hipMemcpyHostToDevice, m->stream));
   m->adam_t = step_no - 1;
-  MLP_HIP(adam(m, lr, b1, b2, eps));
+  hipLaunchKernelGGL(k_adam, dim3(PARAM_BLOCKS), dim3(256), 0, m->stream, next_adam(m, lr, b1, b2, eps),
+                     m->d_grad);
+  MLP_HIP(hipGetLastError());
   MLP_HIP(hipStreamSynchronize(m->stream));
   return KMC_OK;
 }
@@ -949,19 +1069,52 @@ int kmc_mlp_train(kmc_mlp* m, int64_t n, const float* feat, const float* targets
   MLP_HIP(hipSetDevice(m->device));
   int st = ensure_cap(m, batch);
   if (st != KMC_OK) return st;
-  // the data set on the device: BF16 rows, FP32 targets, per-epoch permutation
+  const int64_t per_epoch = n / batch;
+  const double total = (double)epochs * per_epoch;
+  const size_t n_lp = (size_t)LOSS_PARTS * per_epoch;
+  // The shuffles of the next epochs are drawn by threads of their own while the GPU works (an
+  // epoch's draws start at a known place of the stream, and its permutation is applied to the
+  // order before it on the device); at most 2^26 entries ahead.
+  const int ahead = (int)std::max<int64_t>(
+      1, std::min<int64_t>({(int64_t)epochs, 8, ((int64_t)1 << 26) / n,
+                            (int64_t)std::thread::hardware_concurrency() / 2}));
+  std::vector<std::vector<int32_t>> pis;
+  std::vector<std::thread> drawing;
+  try {
+    drawing.resize(ahead);
+    pis.assign(ahead, std::vector<int32_t>(n));
+  } catch (const std::bad_alloc&) {
+    return mfail(KMC_ERR_ALLOC, "kmc_mlp_train: no memory for the shuffles");
+  }
+  const auto draw_epoch = [&](int32_t ep) {
+    int32_t* pi = pis[ep % ahead].data();
+    const uint64_t skip = (uint64_t)ep * (uint64_t)(n - 1);
+    try {
+      drawing[ep % ahead] = std::thread([n, seed, skip, pi] { shuffle(n, seed, skip, pi); });
+    } catch (const std::system_error&) {  // no thread to be had: drawn here
+      shuffle(n, seed, skip, pi);
+    }
+  };
+  // the data set on the device: BF16 rows, FP32 targets, the rows' order (two, used in turn) and
+  // an epoch's shuffle; squared-error sums of two epochs, on the device and pinned
   float* d_f = nullptr;
   bf16* d_x = nullptr;
   float* d_t = nullptr;
   int32_t* d_idx = nullptr;
-  auto release = [&]() {
-    for (void* b : {(void*)d_f, (void*)d_x, (void*)d_t, (void*)d_idx})
-      if (b) (void)hipFree(b);
-  };
+  double* d_lp = nullptr;
+  double* h_lp = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr}, uploaded = nullptr;
   hipError_t e = hipMalloc((void**)&d_f, n * IN * sizeof(float));
   if (e == hipSuccess) e = hipMalloc((void**)&d_x, n * IN * sizeof(bf16));
   if (e == hipSuccess) e = hipMalloc((void**)&d_t, n * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc((void**)&d_idx, n * sizeof(int32_t));
+  if (e == hipSuccess) e = hipMalloc((void**)&d_idx, 3 * n * sizeof(int32_t));
+  if (e == hipSuccess) e = hipMalloc((void**)&d_lp, 2 * n_lp * sizeof(double));
+  if (e == hipSuccess) e = hipHostMalloc((void**)&h_lp, 2 * n_lp * sizeof(double));
+  for (hipEvent_t& ev : done)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&uploaded, hipEventDisableTiming);
+  if (e == hipSuccess)
+    for (int32_t ep = 0; ep < ahead; ++ep) draw_epoch(ep);
   if (e == hipSuccess) e = hipMemcpyAsync(d_f, feat, n * IN * sizeof(float), hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(d_t, targets, n * sizeof(float), hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) {
@@ -971,46 +1124,55 @@ int kmc_mlp_train(kmc_mlp* m, int64_t n, const float* feat, const float* targets
   }
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (d_f) (void)hipFree(d_f);
-  d_f = nullptr;
-  const int64_t per_epoch = n / batch;
-  const double total = (double)epochs * per_epoch;
-  std::vector<int32_t> perm(n);
-  for (int64_t i = 0; i < n; ++i) perm[i] = (int32_t)i;
-  uint64_t rs = seed ^ 0x9E3779B97F4A7C15ull;
-  auto next = [&]() {  // splitmix64
-    uint64_t z = (rs += 0x9E3779B97F4A7C15ull);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
+  // an epoch's mean loss, once its sums have arrived
+  const auto read_loss = [&](int32_t ep) {
+    const hipError_t w = hipEventSynchronize(done[ep & 1]);
+    if (w != hipSuccess || !epoch_loss) return w;
+    const double* lp = h_lp + (ep & 1) * n_lp;
+    double s = 0;
+    for (size_t k = 0; k < n_lp; ++k) s += lp[k];
+    epoch_loss[ep] = s / ((double)per_epoch * batch);
+    return w;
   };
-  std::vector<double> lp(HEAD_WAVES * per_epoch);
-  double* d_lp = nullptr;
-  if (e == hipSuccess) e = hipMalloc((void**)&d_lp, lp.size() * sizeof(double));
   int64_t it = 0;
   for (int32_t ep = 0; ep < epochs && e == hipSuccess; ++ep) {
-    for (int64_t i = n - 1; i > 0; --i) std::swap(perm[i], perm[next() % (uint64_t)(i + 1)]);
-    e = hipMemcpyAsync(d_idx, perm.data(), n * sizeof(int32_t), hipMemcpyHostToDevice, m->stream);
+    if (drawing[ep % ahead].joinable()) drawing[ep % ahead].join();
+    int32_t* pi = d_idx + 2 * n;
+    int32_t* order = d_idx + (ep & 1) * n;
+    e = hipMemcpyAsync(pi, pis[ep % ahead].data(), n * sizeof(int32_t), hipMemcpyHostToDevice, m->stream);
+    if (e != hipSuccess) break;
+    hipLaunchKernelGGL(k_reorder, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, m->stream, n,
+                       ep > 0 ? d_idx + ((ep + 1) & 1) * n : nullptr, pi, order);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipEventRecord(uploaded, m->stream);
+    if (ep >= 2 && e == hipSuccess) e = read_loss(ep - 2);  // before its buffers are used again
+    double* lp = d_lp + (ep & 1) * n_lp;
     for (int64_t b = 0; b < per_epoch && e == hipSuccess; ++b, ++it) {
-      hipLaunchKernelGGL(k_gather, dim3((unsigned)((batch + 255) / 256)), dim3(256), 0, m->stream,
-                         batch, d_idx + b * batch, d_x, d_t, m->X, m->tgt);
-      double* keep = m->lpart;
-      m->lpart = d_lp + b * HEAD_WAVES;
-      e = step(m, batch, batch, true);
-      m->lpart = keep;
+      e = step(m, batch, batch, true, d_x, d_t, order + b * batch, lp + b * LOSS_PARTS);
       const double rate = lr_min + 0.5 * (lr - lr_min) * (1.0 + std::cos(M_PI * (double)it / total));
-      if (e == hipSuccess) e = adam(m, rate, 0.9, 0.999, 1e-8);
+      if (e != hipSuccess) break;
+      hipLaunchKernelGGL(k_mlp_update, dim3(PARAM_BLOCKS), dim3(256), 0, m->stream,
+                         next_adam(m, rate, 0.9, 0.999, 1e-8), splits(batch), m->part, m->cpart);
+      e = hipGetLastError();
     }
     if (e == hipSuccess)
-      e = hipMemcpyAsync(lp.data(), d_lp, lp.size() * sizeof(double), hipMemcpyDeviceToHost, m->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
-    if (e == hipSuccess && epoch_loss) {
-      double s = 0;
-      for (double v : lp) s += v;
-      epoch_loss[ep] = s / ((double)per_epoch * batch);
+      e = hipMemcpyAsync(h_lp + (ep & 1) * n_lp, lp, n_lp * sizeof(double), hipMemcpyDeviceToHost, m->stream);
+    if (e == hipSuccess) e = hipEventRecord(done[ep & 1], m->stream);
+    // the epoch's shuffle has been read: its buffer takes the next one to draw
+    if (ep + ahead < epochs && e == hipSuccess) {
+      e = hipEventSynchronize(uploaded);
+      if (e == hipSuccess) draw_epoch(ep + ahead);
     }
   }
-  if (d_lp) (void)hipFree(d_lp);
-  release();
+  for (std::thread& t : drawing)
+    if (t.joinable()) t.join();
+  for (int32_t ep = std::max(0, epochs - 2); ep < epochs && e == hipSuccess; ++ep) e = read_loss(ep);
+  (void)hipStreamSynchronize(m->stream);
+  for (void* b : {(void*)d_x, (void*)d_t, (void*)d_idx, (void*)d_lp})
+    if (b) (void)hipFree(b);
+  if (h_lp) (void)hipHostFree(h_lp);
+  for (hipEvent_t ev : {done[0], done[1], uploaded})
+    if (ev) (void)hipEventDestroy(ev);
   if (e != hipSuccess) return mfail(KMC_ERR_HIP, std::string("kmc_mlp_train: ") + hipGetErrorString(e));
   if (elapsed_ms)
     *elapsed_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
