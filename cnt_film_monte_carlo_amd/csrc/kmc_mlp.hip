@@ -133,10 +133,18 @@ struct rows_args {
   float inv_n;
   const bf16 *Wtb, *Wb;   // W_l^T and W_l
   const float* prm;
-  int64_t ld;             // rows of the transposed arrays
-  bf16 *XT, *HT, *DT;     // X^T [IN][ld], H_l^T and dZ_l^T [NH][WD][ld]
+  int64_t layer;          // elements of one layer of HT and DT
+  bf16 *XT, *HT, *DT;     // X^T, H_l^T and dZ_l^T by tiles of 32 rows: [tile][unit][32]
   float *y, *dy, *err;
 };
+
+// A workgroup barrier for data in LDS: unlike __syncthreads it does not wait for the wave's
+// global stores, which nothing in the kernel reads back.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 __device__ __forceinline__ float lane_swap(float x) {  // the value of lane i ^ 1
   return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0xB1, 0xF, 0xF, true));
@@ -146,7 +154,7 @@ __device__ __forceinline__ float lane_swap(float x) {  // the value of lane i ^ 
 // 8 (r / 4) + 4 h + r % 4, unit n = 32 wave + c): to LDS for the next layer's A operand (a
 // sample's units side by side) and, transposed, to memory for the weight gradients.
 __device__ __forceinline__ void put_tile(const bf16 (&v)[16], bf16 (*xa)[XS], int n, int h,
-                                         bf16* __restrict__ T, int64_t ld, int64_t row0) {
+                                         bf16* __restrict__ T) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -156,7 +164,7 @@ __device__ __forceinline__ void put_tile(const bf16 (&v)[16], bf16 (*xa)[XS], in
       xa[8 * q + 4 * h + j][n] = v[4 * q + j];
       p[j] = v[4 * q + j];
     }
-    if (T) *reinterpret_cast<bf16x4*>(T + (int64_t)n * ld + row0 + 8 * q + 4 * h) = p;
+    if (T) *reinterpret_cast<bf16x4*>(T + TILE * n + 8 * q + 4 * h) = p;
   }
 }
 
@@ -195,7 +203,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
       wf[l - 1][kb] = *reinterpret_cast<const bf16x8*>(g.Wtb + q_off(l) + (int64_t)n * WD + 16 * kb + 8 * h);
   if (GRAD && wv == 0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) g.XT[(int64_t)(8 * h + e) * g.ld + row] = a0[e];
+    for (int e = 0; e < 8; ++e) g.XT[row0 * IN + TILE * (8 * h + e) + c] = a0[e];
   }
   float z[NH][16];
   bf16 v[16];
@@ -205,7 +213,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
     if (l == 0) {
       acc = mfma32(a0, w0, acc);
     } else {
-      __syncthreads();
+      lds_barrier();
       acc = layer_product(xa[(l - 1) & 1], c, h, wf[l - 1]);
     }
     const float bias = g.prm[b_off(l) + n];
@@ -215,7 +223,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
       v[r] = (bf16)silu_f(z[l][r]);
     }
     if (l + 1 < NH || GRAD)
-      put_tile(v, xa[l & 1], n, h, GRAD ? g.HT + (int64_t)l * WD * g.ld : nullptr, g.ld, row0);
+      put_tile(v, xa[l & 1], n, h, GRAD ? g.HT + l * g.layer + row0 * WD : nullptr);
   }
   // the weights of the way back, read while the output unit is summed
   bf16x8 wb[3][8];
@@ -232,7 +240,7 @@ __global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
     const float hv = (float)v[r], ho = lane_swap(hv);
     if (!(c & 1)) leaf[8 * (r >> 2) + 4 * h + (r & 3)][n >> 1] = fmaf(hv, wa, ho * wo);
   }
-  __syncthreads();
+  lds_barrier();
   {
     const int s = threadIdx.x >> 3, p = threadIdx.x & 7;
     float u[8];
@@ -256,24 +264,24 @@ __global__ __launch_bounds__(256) void k_mlp_rows(rows_args g) {
     }
   }
   if (!GRAD) return;
-  __syncthreads();
+  lds_barrier();
 #pragma unroll
   for (int r = 0; r < 16; ++r)
     v[r] = (bf16)(s_d[8 * (r >> 2) + 4 * h + (r & 3)] * wa * dsilu_f(z[NH - 1][r]));
-  put_tile(v, xa[0], n, h, g.DT + (int64_t)(NH - 1) * WD * g.ld, g.ld, row0);
+  put_tile(v, xa[0], n, h, g.DT + (NH - 1) * g.layer + row0 * WD);
 #pragma unroll
   for (int l = NH - 1; l >= 1; --l) {
-    __syncthreads();
+    lds_barrier();
     acc = layer_product(xa[(NH - 1 - l) & 1], c, h, wb[l - 1]);
 #pragma unroll
     for (int r = 0; r < 16; ++r) v[r] = (bf16)(acc[r] * dsilu_f(z[l - 1][r]));
-    put_tile(v, xa[(NH - l) & 1], n, h, g.DT + (int64_t)(l - 1) * WD * g.ld, g.ld, row0);
+    put_tile(v, xa[(NH - l) & 1], n, h, g.DT + (l - 1) * g.layer + row0 * WD);
   }
 }
 
 struct grads_args {
   int nb, nz;             // rows (a multiple of 128) and splits of K_SPLIT rows
-  int64_t ld;
+  int64_t layer;
   const bf16 *XT, *HT, *DT;
   const float *dy, *err;
   float* part;            // weight layer l: nz q_off(l) + [nz][fan_in][WD]
@@ -294,28 +302,29 @@ __global__ __launch_bounds__(256) void k_mlp_grads(grads_args g) {
     const int zi = b / 13, x = b % 13;
     const int l = x == 0 ? 0 : 1 + (x - 1) / 4, mt = x == 0 ? 0 : (x - 1) % 4;
     const int m = 32 * mt + c, n = 32 * wv + c;
-    const bf16* A = (l == 0 ? g.XT : g.HT + (int64_t)(l - 1) * WD * g.ld) + (int64_t)m * g.ld;
-    const bf16* B = g.DT + ((int64_t)l * WD + n) * g.ld;
-    const bool a_ok = m < fan_in(l);
+    const int fan = fan_in(l);
+    const bf16* A = (l == 0 ? g.XT : g.HT + (l - 1) * g.layer) + TILE * m + 8 * h;
+    const bf16* B = g.DT + l * g.layer + TILE * n + 8 * h;
+    const bool a_ok = m < fan;
     const int k_lo = zi * K_SPLIT, k_hi = min(g.nb, k_lo + K_SPLIT);
     f32x16 acc = {};
     for (int k0 = k_lo; k0 < k_hi; k0 += 128) {  // nb and K_SPLIT are multiples of 128
       bf16x8 av[8], bv[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
-        const int k = k0 + 16 * q + 8 * h;
+        const int64_t k = k0 + 32 * (q >> 1);  // the tile's first row; its second sixteen for odd q
         av[q] = bf16x8{};
-        if (a_ok) av[q] = *reinterpret_cast<const bf16x8*>(A + k);
-        bv[q] = *reinterpret_cast<const bf16x8*>(B + k);
+        if (a_ok) av[q] = *reinterpret_cast<const bf16x8*>(A + k * fan + 16 * (q & 1));
+        bv[q] = *reinterpret_cast<const bf16x8*>(B + k * WD + 16 * (q & 1));
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc = mfma32(av[q], bv[q], acc);
     }
-    float* out = g.part + (int64_t)g.nz * q_off(l) + (int64_t)zi * fan_in(l) * WD;
+    float* out = g.part + (int64_t)g.nz * q_off(l) + (int64_t)zi * fan * WD;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = 32 * mt + 8 * (r >> 2) + 4 * h + (r & 3);
-      if (row < fan_in(l)) out[(int64_t)row * WD + n] = acc[r];
+      if (row < fan) out[(int64_t)row * WD + n] = acc[r];
     }
     return;
   }
@@ -326,20 +335,34 @@ __global__ __launch_bounds__(256) void k_mlp_grads(grads_args g) {
     const int chunk = (g.nb + COL_BLOCKS - 1) / COL_BLOCKS;  // even: nb is a multiple of 128
     const int r0 = blk * chunk, r1 = min(g.nb, r0 + chunk);
     float s0 = 0.0f, s1 = 0.0f;
-    const bf16* x = col < NH * WD ? g.DT + (int64_t)col * g.ld
-                                  : g.HT + ((int64_t)(NH - 1) * WD + (col - NH * WD)) * g.ld;
-    if (col < NH * WD) {
-      for (int r = r0; r < r1; r += 2) {
-        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-        const bf16x2 v = *reinterpret_cast<const bf16x2*>(x + r);
-        s0 = s0 + (float)v[0];
-        s1 = s1 + (float)v[1];
+    const bool plain = col < NH * WD, last = col == COLS - 1;  // last: db4, the sum of dy
+    const int unit = last ? 0 : col % WD;
+    const bf16* x = (plain ? g.DT + (col / WD) * g.layer : g.HT + (NH - 1) * g.layer) + TILE * unit;
+    if (chunk % TILE == 0) {
+      // whole tiles: 64 contiguous bytes each
+      for (int r = r0; r < r1; r += TILE) {
+        bf16x8 v[4];
+        float d[TILE];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const bf16x8*>(x + (int64_t)r * WD + 8 * q);
+        if (!plain) {
+#pragma unroll
+          for (int q = 0; q < TILE; ++q) d[q] = g.dy[r + q];
+        }
+#pragma unroll
+        for (int q = 0; q < TILE; q += 2) {
+          const float x0 = last ? 1.0f : (float)v[q >> 3][q & 7];
+          const float x1 = last ? 1.0f : (float)v[q >> 3][(q & 7) + 1];
+          s0 = s0 + (plain ? x0 : x0 * d[q]);
+          s1 = s1 + (plain ? x1 : x1 * d[q + 1]);
+        }
       }
     } else {
-      const bool last = col == COLS - 1;  // db4: the sum of dy
       for (int r = r0; r < r1; r += 2) {
-        s0 = s0 + (last ? 1.0f : (float)x[r]) * g.dy[r];
-        s1 = s1 + (last ? 1.0f : (float)x[r + 1]) * g.dy[r + 1];
+        const int64_t at = (int64_t)(r & ~(TILE - 1)) * WD + (r & (TILE - 1));
+        const float x0 = last ? 1.0f : (float)x[at], x1 = last ? 1.0f : (float)x[at + 1];
+        s0 = s0 + (plain ? x0 : x0 * g.dy[r]);
+        s1 = s1 + (plain ? x1 : x1 * g.dy[r + 1]);
       }
     }
     g.cpart[(int64_t)blk * COLS + col] = s0 + s1;
@@ -360,14 +383,25 @@ __device__ __forceinline__ float sum_parts(int64_t p, int nz, const float* __res
     if (p >= w_off(l) && p < b_off(l)) {
       const int64_t len = (int64_t)fan_in(l) * WD;
       const float* q = part + (int64_t)nz * q_off(l) + (p - w_off(l));
-      for (int z = 0; z < nz; ++z) a += q[z * len];
+      int z = 0;
+      for (; z + 16 <= nz; z += 16) {  // sixteen loads in flight
+        float v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = q[(z + k) * len];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) a += v[k];
+      }
+      for (; z < nz; ++z) a += q[z * len];
       return a;
     }
     if (p >= b_off(l) && p < b_off(l) + WD) col = l * WD + (int)(p - b_off(l));
   }
   if (col < 0) col = NH * WD + (int)(p - W4_OFF);  // w4, then b4
-#pragma unroll 8
-  for (int z = 0; z < COL_BLOCKS; ++z) a += cpart[(int64_t)z * COLS + col];
+  float v[COL_BLOCKS];
+#pragma unroll
+  for (int z = 0; z < COL_BLOCKS; ++z) v[z] = cpart[(int64_t)z * COLS + col];
+#pragma unroll
+  for (int z = 0; z < COL_BLOCKS; ++z) a += v[z];
   return a;
 }
 
@@ -704,7 +738,7 @@ hipError_t step(kmc_mlp* m, int nb, int n_valid, bool backward, const bf16* X, c
   g.Wtb = m->d_wtb;
   g.Wb = m->d_wb;
   g.prm = m->d_prm;
-  g.ld = m->cap;
+  g.layer = m->cap * WD;
   g.XT = m->XT;
   g.HT = m->HT;
   g.DT = m->DT;
@@ -722,7 +756,7 @@ hipError_t step(kmc_mlp* m, int nb, int n_valid, bool backward, const bf16* X, c
   grads_args q{};
   q.nb = nb;
   q.nz = splits(nb);
-  q.ld = m->cap;
+  q.layer = m->cap * WD;
   q.XT = m->XT;
   q.HT = m->HT;
   q.DT = m->DT;
