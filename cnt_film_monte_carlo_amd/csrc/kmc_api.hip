@@ -363,7 +363,9 @@ int copy_out(kmc_ctx* c, void* dst, const void* src, size_t bytes) {
 // Row blocks of the hop kernel from the finished CSR (hdr, cum, edge), plus the block offsets of
 // the source sites.  Blocks are laid out in cell-list order when the cell list is current, so
 // sites that are close in space are close in memory.
-int pack_rows(kmc_ctx* c) {
+// `who` (may be null) names a caller whose rates k_finish_pair_rates has just checked: the verdict
+// comes back with the line count.
+int pack_rows(kmc_ctx* c, const char* who = nullptr) {
   const int64_t n = c->n_sites;
   KMC_TRY(dalloc(c, c->d_units, n));
   KMC_TRY(dalloc(c, c->d_roff, n + 1));
@@ -376,10 +378,14 @@ int pack_rows(kmc_ctx* c) {
     KMC_TRY(dalloc(c, c->d_place, 2 * n));
     KMC_HIP(c, launch_morton_keys(n, c->d_cell_of.p, c->cells.nx, c->cells.ny, c->d_pkeys.p,
                                   c->d_place.p, c->stream));
+    // a cell coordinate below 2^b spreads over the key bits below 3 b
+    int bits = 1;
+    while (bits < 21 && (std::max({c->cells.nx, c->cells.ny, c->cells.nz}) - 1) >> bits) ++bits;
+    const int end_bit = std::min(64, 3 * bits);
     size_t need = 0;
     KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(nullptr, need, c->d_pkeys.p, c->d_pkeys.p + n,
-                                                  c->d_place.p, c->d_place.p + n, (int)n, 0, 64,
-                                                  c->stream));
+                                                  c->d_place.p, c->d_place.p + n, (int)n, 0,
+                                                  end_bit, c->stream));
     if (need > c->sort_tmp_bytes) {
       KMC_TRY(dalloc(c, c->d_sort_tmp, need));
       c->sort_tmp_bytes = need;
@@ -387,7 +393,8 @@ int pack_rows(kmc_ctx* c) {
     size_t have = c->sort_tmp_bytes;
     KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(c->d_sort_tmp.p, have, c->d_pkeys.p,
                                                   c->d_pkeys.p + n, c->d_place.p,
-                                                  c->d_place.p + n, (int)n, 0, 64, c->stream));
+                                                  c->d_place.p + n, (int)n, 0, end_bit,
+                                                  c->stream));
     order = c->d_place.p + n;
   }
   if (order) {
@@ -399,7 +406,11 @@ int pack_rows(kmc_ctx* c) {
     KMC_HIP(c, exclusive_scan(c->d_units.p, c->d_roff.p, n, c->d_scan_tmp.p, c->stream));
   }
   int64_t lines = 0;
+  int32_t bad = 0;
+  if (who)
+    KMC_HIP(c, hipMemcpyAsync(&bad, c->d_err.p, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
   KMC_TRY(copy_out(c, &lines, c->d_roff.p + n, sizeof(int64_t)));
+  if (bad) return fail(c, KMC_ERR_RATE, std::string(who) + ": negative, NaN or infinite rate");
   // the wave loop addresses the blocks with 32-bit byte offsets: at most 2^25 lines (4 GiB)
   if (lines > ((int64_t)1 << 25))
     return fail(c, KMC_ERR_CAPACITY, "pack_rows: row blocks beyond 4 GiB (2^25 lines of 128 B)");
@@ -416,13 +427,6 @@ int pack_rows(kmc_ctx* c) {
   KMC_HIP(c, launch_links(n, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p, c->d_hdr.p,
                           c->d_links.p, c->stream));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
-  return KMC_OK;
-}
-
-int check_err_flag(kmc_ctx* c, const char* what) {
-  int32_t h = 0;
-  KMC_TRY(copy_out(c, &h, c->d_err.p, sizeof(int32_t)));
-  if (h != 0) return fail(c, KMC_ERR_RATE, std::string(what) + ": negative, NaN or infinite rate");
   return KMC_OK;
 }
 
@@ -783,9 +787,9 @@ int kmc_build_rates(kmc_ctx* c, int32_t mode) {
   }
   KMC_HIP(c, hipMemsetAsync(c->d_err.p, 0, sizeof(int32_t), c->stream));
   KMC_HIP(c, launch_fill_pairs(mode, s, c->cells, c->d_cell_start.p, c->d_cell_sites.p,
-                               c->d_row_ptr.p, t, csr_of(c), geo, c->d_err.p, c->stream));
-  KMC_TRY(check_err_flag(c, "kmc_build_rates"));
-  if (mode == KMC_RATE_TABLE) KMC_TRY(pack_rows(c));
+                               c->d_row_ptr.p, nnz, t, csr_of(c), geo, c->d_err.p, c->stream));
+  if (mode == KMC_RATE_TABLE) KMC_TRY(pack_rows(c, "kmc_build_rates"));
+  else KMC_HIP(c, hipStreamSynchronize(c->stream));
   c->csr_state = (mode == KMC_RATE_TABLE) ? 2 : 1;
   reset_downstream(c, 2);
   return KMC_OK;
@@ -829,8 +833,7 @@ int kmc_set_pair_rates_device(kmc_ctx* c, const double* d_rates) {
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   KMC_HIP(c, hipMemsetAsync(c->d_err.p, 0, sizeof(int32_t), c->stream));
   KMC_HIP(c, launch_finish_pair_rates(c->n_sites, d_rates, csr_of(c), c->d_err.p, c->stream));
-  KMC_TRY(check_err_flag(c, "kmc_set_pair_rates"));
-  KMC_TRY(pack_rows(c));
+  KMC_TRY(pack_rows(c, "kmc_set_pair_rates"));
   c->csr_state = 2;
   reset_downstream(c, 2);
   return KMC_OK;

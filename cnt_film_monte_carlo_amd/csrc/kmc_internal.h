@@ -263,27 +263,18 @@ __host__ __device__ __forceinline__ int cell_coord(const cell_desc& c, int axis,
   return (int)((p - c.lo[axis]) / c.cell[axis]);
 }
 
-// The up to three stencil coordinates along one axis, in the order i-1, i, i+1 with
-// out-of-range cells dropped on open axes (monte_carlo.h:402-405) and wrapped (duplicates
-// dropped) on periodic axes.  Returns the count.
-__host__ __device__ __forceinline__ int stencil_axis(const cell_desc& c, int axis, int i,
-                                                     int out[3]) {
+// The k-th (0..2) stencil coordinate along one axis, or -1 when there are not so many: i-1, i, i+1
+// with out-of-range cells dropped on open axes (monte_carlo.h:402-405) and wrapped (duplicates
+// dropped) on periodic axes.
+__host__ __device__ __forceinline__ int stencil_cell(const cell_desc& c, int axis, int i, int k) {
   const int n = axis == 0 ? c.nx : (axis == 1 ? c.ny : c.nz);
-  int k = 0;
   if (c.periodic_mask & (1 << axis)) {
-    for (int d = -1; d <= 1; ++d) {
-      const int w = ((i + d) % n + n) % n;
-      bool dup = false;
-      for (int q = 0; q < k; ++q) dup = dup || (out[q] == w);
-      if (!dup) out[k++] = w;
-    }
-  } else {
-    for (int d = -1; d <= 1; ++d) {
-      const int w = i + d;
-      if (w > -1 && w < n) out[k++] = w;
-    }
+    if (k >= n) return -1;  // one or two cells: each once
+    const int w = i - 1 + k;
+    return w < 0 ? w + n : (w >= n ? w - n : w);
   }
-  return k;
+  const int w = (i > 0 ? i - 1 : i) + k;
+  return w <= i + 1 && w < n ? w : -1;
 }
 
 }  // namespace cntkmc

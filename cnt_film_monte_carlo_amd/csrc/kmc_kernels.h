@@ -157,8 +157,9 @@ hipError_t launch_count_pairs(const site_arrays& s, const cell_desc& c, const in
                               const int32_t* cell_sites, uint32_t* deg, hipStream_t st);
 hipError_t launch_fill_pairs(int mode, const site_arrays& s, const cell_desc& c,
                              const int64_t* cell_start, const int32_t* cell_sites,
-                             const int64_t* row_ptr, const table_desc& t, const csr_arrays& out,
-                             const pair_geom_arrays& geo, int32_t* err, hipStream_t st);
+                             const int64_t* row_ptr, int64_t nnz, const table_desc& t,
+                             const csr_arrays& out, const pair_geom_arrays& geo, int32_t* err,
+                             hipStream_t st);
 hipError_t launch_finish_pair_rates(int64_t n, const double* rates, const csr_arrays& out,
                                     int32_t* err, hipStream_t st);
 hipError_t launch_inject(const exciton_arrays& x, const uint4* blocks, const uint32_t* src_roff,

@@ -1,7 +1,7 @@
 // kmc_kernels.hip -- CDNA4 (gfx950) kernels of the KMC exciton-hopping path.
 //
 //   (a) cell list          k_cell_assign, k_cell_scatter, k_cell_sort
-//   (b) CSR out-rate table  k_count_pairs, k_fill_pairs, k_finish_pair_rates
+//   (b) CSR out-rate table  k_count_pairs, k_list_pairs, k_pair_values, k_finish_pair_rates
 //   (c) hop kernel          k_inject, k_hop
 //   (d) MSD/current reduce  k_reduce_samples
 // plus a three-phase exclusive scan used by (a) and (b).
@@ -167,109 +167,152 @@ __global__ __launch_bounds__(256) void k_cell_sort(int64_t n_cells,
 // (b) CSR build (find_neighbors + set_max_rate, src/monte_carlo/scatterer.cpp:34-83,
 //     src/monte_carlo/scatterer.h:89-93)
 // =============================================================================================
-// Visit every candidate of site i in the reference order and call f(j, image, distance)
-// for those inside (min_distance, cutoff).
+// A site has 32 lanes, one per cell of its stencil (27 of them used): lane 9 a + 3 b + e visits
+// the a-th, b-th, e-th valid cell along x, y, z, so that the lanes' order is the reference's
+// (x-outer, y, z-inner) and a lane's neighbours follow those of the lanes before it.  A thread per
+// site walked the 27 cells one after another, each a chain of dependent loads, with one lane of a
+// wave at a time in the pair arithmetic (50,101 sites and 0.22 M pairs: count 54, fill 455 us; now
+// count 21, list 39, values 12 us).
+constexpr uint32_t STENCIL_LANES = 32;
+
+// Calls f(j, image of j) for the neighbours of site i in the lane's cell, those inside
+// (min_distance, cutoff), ascending.
 template <typename F>
-__device__ __forceinline__ void for_each_neighbor(const site_arrays& s, const cell_desc& c,
-                                                  const int64_t* __restrict__ cell_start,
-                                                  const int32_t* __restrict__ cell_sites,
-                                                  int64_t i, F&& f) {
+__device__ __forceinline__ void cell_neighbors(const site_arrays& s, const cell_desc& c,
+                                               const int64_t* __restrict__ cell_start,
+                                               const int32_t* __restrict__ cell_sites, int64_t i,
+                                               uint32_t lane, F&& f) {
 #pragma clang fp contract(off)
   const double pix = s.px[i], piy = s.py[i], piz = s.pz[i];
-  int sx[3], sy[3], sz[3];
-  const int nsx = stencil_axis(c, 0, cell_coord(c, 0, pix), sx);
-  const int nsy = stencil_axis(c, 1, cell_coord(c, 1, piy), sy);
-  const int nsz = stencil_axis(c, 2, cell_coord(c, 2, piz), sz);
-  for (int a = 0; a < nsx; ++a) {
-    for (int b = 0; b < nsy; ++b) {
-      for (int d = 0; d < nsz; ++d) {
-        const int64_t cell = (int64_t)sx[a] + (int64_t)sy[b] * c.nx + (int64_t)sz[d] * c.nx * c.ny;
-        const int64_t beg = cell_start[cell], end = cell_start[cell + 1];
-        for (int64_t q = beg; q < end; ++q) {
-          const int32_t j = cell_sites[q];
-          double pjx = s.px[j], pjy = s.py[j], pjz = s.pz[j];
-          if (c.periodic_mask & 1) pjx = image_of(pix, pjx, c.period[0]);
-          if (c.periodic_mask & 2) pjy = image_of(piy, pjy, c.period[1]);
-          if (c.periodic_mask & 4) pjz = image_of(piz, pjz, c.period[2]);
-          const double dist = norm3(pix - pjx, piy - pjy, piz - pjz);
-          if ((dist < c.cutoff) && (dist > c.min_distance)) f(j, pjx, pjy, pjz);
-        }
-      }
-    }
+  const int x = stencil_cell(c, 0, cell_coord(c, 0, pix), (int)lane / 9);
+  const int y = stencil_cell(c, 1, cell_coord(c, 1, piy), (int)lane / 3 % 3);
+  const int z = stencil_cell(c, 2, cell_coord(c, 2, piz), (int)lane % 3);
+  if (lane >= 27u || x < 0 || y < 0 || z < 0) return;
+  const int64_t cell = (int64_t)x + (int64_t)y * c.nx + (int64_t)z * c.nx * c.ny;
+  const int64_t beg = cell_start[cell], end = cell_start[cell + 1];
+  for (int64_t q = beg; q < end; ++q) {
+    const int32_t j = cell_sites[q];
+    double pjx = s.px[j], pjy = s.py[j], pjz = s.pz[j];
+    if (c.periodic_mask & 1) pjx = image_of(pix, pjx, c.period[0]);
+    if (c.periodic_mask & 2) pjy = image_of(piy, pjy, c.period[1]);
+    if (c.periodic_mask & 4) pjz = image_of(piz, pjz, c.period[2]);
+    const double dist = norm3(pix - pjx, piy - pjy, piz - pjz);
+    if ((dist < c.cutoff) && (dist > c.min_distance)) f(j, pjx, pjy, pjz);
   }
 }
 
-__global__ __launch_bounds__(256) void k_count_pairs(site_arrays s, cell_desc c,
+// Neighbours of the lane's cell, and of the site's cells before it (exclusive) and altogether.
+__device__ __forceinline__ uint32_t stencil_count(const site_arrays& s, const cell_desc& c,
+                                                  const int64_t* __restrict__ cell_start,
+                                                  const int32_t* __restrict__ cell_sites, int64_t i,
+                                                  uint32_t lane, uint32_t* before) {
+  uint32_t count = 0;
+  if (i < s.n)
+    cell_neighbors(s, c, cell_start, cell_sites, i, lane,
+                   [&](int32_t, double, double, double) { ++count; });
+  uint32_t sum = count;
+#pragma unroll
+  for (int off = 1; off < (int)STENCIL_LANES; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)sum, off, (int)STENCIL_LANES);
+    if (lane >= (uint32_t)off) sum += y;
+  }
+  *before = sum - count;
+  return (uint32_t)__shfl((int)sum, (int)STENCIL_LANES - 1, (int)STENCIL_LANES);
+}
+
+__global__ __launch_bounds__(256) void k_count_pairs(int64_t i0, site_arrays s, cell_desc c,
                                                      const int64_t* __restrict__ cell_start,
                                                      const int32_t* __restrict__ cell_sites,
                                                      uint32_t* __restrict__ deg) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= s.n) return;
-  uint32_t count = 0;
-  for_each_neighbor(s, c, cell_start, cell_sites, i,
-                    [&](int32_t, double, double, double) { ++count; });
-  deg[i] = count;
+  const int64_t i = i0 + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / STENCIL_LANES;
+  const uint32_t lane = threadIdx.x % STENCIL_LANES;
+  uint32_t before;
+  const uint32_t n = stencil_count(s, c, cell_start, cell_sites, i, lane, &before);
+  if (lane == 0 && i < s.n) deg[i] = n;
 }
 
-// mode 0 (table): rate from the nearest-node table and the running FP64 prefix sum
-// (scatterer.cpp:63, 78-80).  mode 1 (pair): store the geometry for an external rate.
-template <int MODE>
-__global__ __launch_bounds__(256) void k_fill_pairs(site_arrays s, cell_desc c,
+// The pairs, row by row: target in edge[p].col, source in the bits of cum[p] (which k_pair_values
+// or k_finish_pair_rates overwrite).
+__global__ __launch_bounds__(256) void k_list_pairs(int64_t i0, site_arrays s, cell_desc c,
                                                     const int64_t* __restrict__ cell_start,
                                                     const int32_t* __restrict__ cell_sites,
                                                     const int64_t* __restrict__ row_ptr,
-                                                    table_desc t, csr_arrays out,
-                                                    pair_geom_arrays geo,
-                                                    int32_t* __restrict__ err) {
-#pragma clang fp contract(off)
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                                                    csr_arrays out) {
+  const int64_t i = i0 + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / STENCIL_LANES;
+  const uint32_t lane = threadIdx.x % STENCIL_LANES;
+  uint32_t before;
+  const uint32_t n = stencil_count(s, c, cell_start, cell_sites, i, lane, &before);
   if (i >= s.n) return;
-  const double pix = s.px[i], piy = s.py[i], piz = s.pz[i];
-  const double oix = s.ox[i], oiy = s.oy[i], oiz = s.oz[i];
-  const int ci = s.chir[i];
-  int64_t pos = row_ptr[i];
-  double cum = 0.0;
-  bool first = true;
-  for_each_neighbor(s, c, cell_start, cell_sites, i,
-                    [&](int32_t j, double pjx, double pjy, double pjz) {
-                      const pair_geom g = pair_geometry(pix, piy, piz, pjx, pjy, pjz, oix, oiy,
-                                                        oiz, s.ox[j], s.oy[j], s.oz[j]);
-                      edge_rec e;
-                      e.col = (uint32_t)j | ((s.flags[j] & 2u) ? EDGE_DRAIN_BIT : 0u);
-                      e.dx = (float)(pjx - pix);
-                      e.dy = (float)(pjy - piy);
-                      e.dz = (float)(pjz - piz);
-                      out.edge[pos] = e;
-                      if (MODE == 0) {
-                        const double r = table_rate(t, ci, s.chir[j], g);
-                        if (!(r >= 0.0) || isinf(r)) atomicOr(err, 1);
-                        cum = first ? r : cum + r;
-                        first = false;
-                        out.cum[pos] = cum;
-                      } else {
-                        geo.theta[pos] = g.theta;
-                        geo.z[pos] = g.z;
-                        geo.a1[pos] = g.a1;
-                        geo.a2[pos] = g.a2;
-                      }
-                      ++pos;
-                    });
-  site_hdr h;
-  h.rs = (uint32_t)row_ptr[i];
-  h.n = (uint32_t)(row_ptr[i + 1] - row_ptr[i]);
-  h.gamma = (MODE == 0 && h.n > 0) ? cum : 0.0;
-  out.hdr[i] = h;
+  const int64_t rs = row_ptr[i];
+  int64_t pos = rs + before;
+  cell_neighbors(s, c, cell_start, cell_sites, i, lane, [&](int32_t j, double, double, double) {
+    out.edge[pos].col = (uint32_t)j | ((s.flags[j] & 2u) ? EDGE_DRAIN_BIT : 0u);
+    out.cum[pos] = __longlong_as_double((long long)i);
+    ++pos;
+  });
+  if (lane == 0) {
+    site_hdr h;
+    h.rs = (uint32_t)rs;
+    h.n = n;
+    h.gamma = 0.0;
+    out.hdr[i] = h;
+  }
 }
 
-template __global__ void k_fill_pairs<0>(site_arrays, cell_desc, const int64_t*, const int32_t*,
-                                         const int64_t*, table_desc, csr_arrays, pair_geom_arrays,
-                                         int32_t*);
-template __global__ void k_fill_pairs<1>(site_arrays, cell_desc, const int64_t*, const int32_t*,
-                                         const int64_t*, table_desc, csr_arrays, pair_geom_arrays,
-                                         int32_t*);
+// Grid axes kept in LDS while the pairs look up their nodes; longer ones are read from memory.
+constexpr int GRID_LDS = 1024;
+
+// A thread per listed pair: displacement and geometry, then in mode 0 (table) the rate from the
+// nearest-node table into cum, which k_finish_pair_rates turns into the running FP64 prefix sum
+// (scatterer.cpp:63, 78-80), in mode 1 (pair) the geometry for an external rate.  Within the
+// search, where a few lanes of a wave hold a pair at a time, the ~600 instructions of geometry and
+// lookup took 192 us for 50,101 sites and 0.22 M pairs; here, with full waves, 12 us (list 39 us).
+template <int MODE>
+__global__ __launch_bounds__(256) void k_pair_values(int64_t p0, int64_t nnz, site_arrays s,
+                                                     cell_desc c, table_desc t, csr_arrays out,
+                                                     pair_geom_arrays geo) {
+#pragma clang fp contract(off)
+  __shared__ double grid[MODE == 0 ? GRID_LDS : 1];
+  if (MODE == 0) {
+    const int len = t.n_th + t.n_z + t.n_a1 + t.n_a2;  // the axes follow one another in memory
+    if (len <= GRID_LDS) {
+      for (int k = threadIdx.x; k < len; k += blockDim.x) grid[k] = t.th[k];
+      t.th = grid;
+      t.z = t.th + t.n_th;
+      t.a1 = t.z + t.n_z;
+      t.a2 = t.a1 + t.n_a1;
+    }
+    __syncthreads();
+  }
+  const int64_t p = p0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz) return;
+  const int64_t i = (int64_t)__double_as_longlong(out.cum[p]);
+  edge_rec e = out.edge[p];
+  const uint32_t j = e.col & EDGE_COL_MASK;
+  const double pix = s.px[i], piy = s.py[i], piz = s.pz[i];
+  double pjx = s.px[j], pjy = s.py[j], pjz = s.pz[j];
+  if (c.periodic_mask & 1) pjx = image_of(pix, pjx, c.period[0]);
+  if (c.periodic_mask & 2) pjy = image_of(piy, pjy, c.period[1]);
+  if (c.periodic_mask & 4) pjz = image_of(piz, pjz, c.period[2]);
+  const pair_geom g = pair_geometry(pix, piy, piz, pjx, pjy, pjz, s.ox[i], s.oy[i], s.oz[i],
+                                    s.ox[j], s.oy[j], s.oz[j]);
+  e.dx = (float)(pjx - pix);
+  e.dy = (float)(pjy - piy);
+  e.dz = (float)(pjz - piz);
+  out.edge[p] = e;
+  if (MODE == 0) {
+    out.cum[p] = table_rate(t, s.chir[i], s.chir[j], g);
+  } else {
+    geo.theta[p] = g.theta;
+    geo.z[p] = g.z;
+    geo.a1[p] = g.a1;
+    geo.a2[p] = g.a2;
+  }
+}
 
 // Sequential FP64 inclusive prefix sum per row from per-pair rates (scatterer.cpp:78-80).
-__global__ __launch_bounds__(256) void k_finish_pair_rates(int64_t n, const double* __restrict__ rates,
+// rates may be out.cum itself.
+__global__ __launch_bounds__(256) void k_finish_pair_rates(int64_t n, const double* rates,
                                                            csr_arrays out,
                                                            int32_t* __restrict__ err) {
 #pragma clang fp contract(off)
@@ -2203,27 +2246,40 @@ hipError_t launch_cell_sort(int64_t n_cells, const int64_t* cell_start, int32_t*
   return hipGetLastError();
 }
 
+// Sites of one launch of the pair search: its threads stay below 2^32.
+constexpr int64_t STENCIL_SITES = (int64_t)1 << 26;
+static dim3 stencil_grid(int64_t sites) {
+  return grid_for(std::min(sites, STENCIL_SITES) * (int64_t)STENCIL_LANES);
+}
+
 hipError_t launch_count_pairs(const site_arrays& s, const cell_desc& c, const int64_t* cell_start,
                               const int32_t* cell_sites, uint32_t* deg, hipStream_t st) {
   if (s.n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_count_pairs, grid_for(s.n), dim3(256), 0, st, s, c, cell_start,
-                     cell_sites, deg);
+  for (int64_t i0 = 0; i0 < s.n; i0 += STENCIL_SITES)
+    hipLaunchKernelGGL(k_count_pairs, stencil_grid(s.n - i0), dim3(256), 0, st, i0, s, c,
+                       cell_start, cell_sites, deg);
   return hipGetLastError();
 }
 
 hipError_t launch_fill_pairs(int mode, const site_arrays& s, const cell_desc& c,
                              const int64_t* cell_start, const int32_t* cell_sites,
-                             const int64_t* row_ptr, const table_desc& t, const csr_arrays& out,
-                             const pair_geom_arrays& geo, int32_t* err, hipStream_t st) {
+                             const int64_t* row_ptr, int64_t nnz, const table_desc& t,
+                             const csr_arrays& out, const pair_geom_arrays& geo, int32_t* err,
+                             hipStream_t st) {
   if (s.n == 0) return hipSuccess;
-  if (mode == 0) {
-    hipLaunchKernelGGL(k_fill_pairs<0>, grid_for(s.n), dim3(256), 0, st, s, c, cell_start,
-                       cell_sites, row_ptr, t, out, geo, err);
-  } else {
-    hipLaunchKernelGGL(k_fill_pairs<1>, grid_for(s.n), dim3(256), 0, st, s, c, cell_start,
-                       cell_sites, row_ptr, t, out, geo, err);
+  for (int64_t i0 = 0; i0 < s.n; i0 += STENCIL_SITES)
+    hipLaunchKernelGGL(k_list_pairs, stencil_grid(s.n - i0), dim3(256), 0, st, i0, s, c, cell_start,
+                       cell_sites, row_ptr, out);
+  constexpr int64_t SLICE = (int64_t)1 << 30;
+  for (int64_t p0 = 0; p0 < nnz; p0 += SLICE) {
+    const dim3 grid = grid_for(std::min(nnz - p0, SLICE));
+    if (mode == 0)
+      hipLaunchKernelGGL(k_pair_values<0>, grid, dim3(256), 0, st, p0, nnz, s, c, t, out, geo);
+    else
+      hipLaunchKernelGGL(k_pair_values<1>, grid, dim3(256), 0, st, p0, nnz, s, c, t, out, geo);
   }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || mode != 0 ? e : launch_finish_pair_rates(s.n, out.cum, out, err, st);
 }
 
 hipError_t launch_finish_pair_rates(int64_t n, const double* rates, const csr_arrays& out,
