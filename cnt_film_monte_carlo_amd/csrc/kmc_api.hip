@@ -129,6 +129,7 @@ struct kmc_ctx {
   dbuf<uint32_t> d_cls_count;
   dbuf<int64_t> d_cls_start, d_sel;
   dbuf<uint8_t> d_mlp_flag;  // surrogate flags of the last surrogate build
+  dbuf<uint8_t> d_read;      // read-backs: the caller's layout of one chunk
   // drift along the tubes (particle::fly): velocity [m/s], links as block lines, error word
   double velocity = 0.0;      // set by kmc_set_velocity
   double exc_velocity = 0.0;  // the velocity of the injected excitons (fixed by kmc_inject)
@@ -207,6 +208,9 @@ constexpr int CONTACT_EV_PAIRS = 64;
 // the live count after step k - CONTACT_LIVE_LAG bounds the slots step k's sort, step and
 // compaction cover; the host waits for it only that many steps back
 constexpr int CONTACT_LIVE_LAG = 2;
+
+// Sites or pairs that a read-back rearranges on the device at a time, 16 bytes each in d_read.
+constexpr int64_t READ_CHUNK = (int64_t)1 << 20;
 
 namespace {
 
@@ -353,10 +357,35 @@ int copy_in(kmc_ctx* c, void* dst, const void* src, size_t bytes) {
   return KMC_OK;
 }
 
+// A copy to the host that is complete after the stream's next synchronisation.
+int queue_out(kmc_ctx* c, void* dst, const void* src, size_t bytes) {
+  if (bytes == 0) return KMC_OK;
+  KMC_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+  return KMC_OK;
+}
+
 int copy_out(kmc_ctx* c, void* dst, const void* src, size_t bytes) {
   if (bytes == 0) return KMC_OK;
   KMC_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
+  return KMC_OK;
+}
+
+// d_read of at least `bytes` (grown, at most 16 READ_CHUNK).
+int read_scratch(kmc_ctx* c, int64_t bytes) {
+  return (int64_t)c->d_read.n >= bytes ? KMC_OK : dalloc(c, c->d_read, (size_t)bytes);
+}
+
+// queue_out of three arrays of n values, interleaved: dst[3 k + a].
+int queue_out3(kmc_ctx* c, double* dst, const double* x, const double* y, const double* z, int64_t n) {
+  constexpr int64_t CHUNK = READ_CHUNK * 16 / 24;
+  KMC_TRY(read_scratch(c, 24 * std::min(CHUNK, n)));
+  double* d = reinterpret_cast<double*>(c->d_read.p);
+  for (int64_t i = 0; i < n; i += CHUNK) {
+    const int64_t k = std::min(CHUNK, n - i);
+    KMC_HIP(c, launch_interleave3(k, x + i, y + i, z + i, d, c->stream));
+    KMC_TRY(queue_out(c, dst + 3 * i, d, 3 * k * sizeof(double)));
+  }
   return KMC_OK;
 }
 
@@ -525,7 +554,7 @@ int kmc_destroy(kmc_ctx* c) {
   dfree(c->d_units); dfree(c->d_src_roff); dfree(c->d_roff); dfree(c->d_blocks);
   dfree(c->d_first); dfree(c->d_keys); dfree(c->d_ids); dfree(c->d_sort_tmp);
   dfree(c->d_counts64); dfree(c->d_cls); dfree(c->d_cls_count); dfree(c->d_cls_start);
-  dfree(c->d_sel); dfree(c->d_mlp_flag);
+  dfree(c->d_sel); dfree(c->d_mlp_flag); dfree(c->d_read);
   dfree(c->d_err); dfree(c->x_site); dfree(c->x_t); dfree(c->x_dx); dfree(c->x_dy);
   dfree(c->x_dz); dfree(c->x_hops); dfree(c->x_hash); dfree(c->x_drains); dfree(c->x_krec);
   dfree(c->x_heading); dfree(c->x_soff); dfree(c->x_tlast); dfree(c->d_links); dfree(c->d_fly_err);
@@ -983,27 +1012,30 @@ int kmc_get_csr(kmc_ctx* c, int64_t* row_ptr, int32_t* col, double* cum, float* 
   if (c->csr_state != 2) return fail(c, KMC_ERR_STATE, "kmc_get_csr: CSR not complete");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   const int64_t n = c->n_sites, nnz = c->nnz;
-  std::vector<site_hdr> hdr(n);
-  KMC_TRY(copy_out(c, hdr.data(), c->d_hdr.p, n * sizeof(site_hdr)));
-  if (row_ptr) {
-    for (int64_t i = 0; i < n; ++i) row_ptr[i] = hdr[i].rs;
-    row_ptr[n] = nnz;
+  // unpacked on the device, `chunk` sites or pairs at a time, straight into the caller's arrays
+  const int64_t chunk = std::min(READ_CHUNK, std::max(n, nnz));
+  if (row_ptr || gamma || col || disp) KMC_TRY(read_scratch(c, 16 * chunk));
+  for (int64_t i = 0; (row_ptr || gamma) && i < n; i += chunk) {
+    const int64_t k = std::min<int64_t>(chunk, n - i);
+    int64_t* d_row = reinterpret_cast<int64_t*>(c->d_read.p);
+    double* d_gamma = reinterpret_cast<double*>(c->d_read.p + chunk * 8);
+    KMC_HIP(c, launch_unpack_rows(k, c->d_hdr.p + i, row_ptr ? d_row : nullptr,
+                                  gamma ? d_gamma : nullptr, c->stream));
+    if (row_ptr) KMC_TRY(queue_out(c, row_ptr + i, d_row, k * sizeof(int64_t)));
+    if (gamma) KMC_TRY(queue_out(c, gamma + i, d_gamma, k * sizeof(double)));
   }
-  if (gamma)
-    for (int64_t i = 0; i < n; ++i) gamma[i] = hdr[i].gamma;
-  if (cum) KMC_TRY(copy_out(c, cum, c->d_cum.p, nnz * sizeof(double)));
-  if (col || disp) {
-    std::vector<edge_rec> edge(nnz);
-    KMC_TRY(copy_out(c, edge.data(), c->d_edge.p, nnz * sizeof(edge_rec)));
-    for (int64_t p = 0; p < nnz; ++p) {
-      if (col) col[p] = (int32_t)(edge[p].col & EDGE_COL_MASK);
-      if (disp) {
-        disp[3 * p + 0] = edge[p].dx;
-        disp[3 * p + 1] = edge[p].dy;
-        disp[3 * p + 2] = edge[p].dz;
-      }
-    }
+  if (cum) KMC_TRY(queue_out(c, cum, c->d_cum.p, nnz * sizeof(double)));
+  for (int64_t p = 0; (col || disp) && p < nnz; p += chunk) {
+    const int64_t k = std::min<int64_t>(chunk, nnz - p);
+    int32_t* d_col = reinterpret_cast<int32_t*>(c->d_read.p);
+    float* d_disp = reinterpret_cast<float*>(c->d_read.p + chunk * 4);
+    KMC_HIP(c, launch_unpack_edges(k, c->d_edge.p + p, col ? d_col : nullptr,
+                                   disp ? d_disp : nullptr, c->stream));
+    if (col) KMC_TRY(queue_out(c, col + p, d_col, k * sizeof(int32_t)));
+    if (disp) KMC_TRY(queue_out(c, disp + 3 * p, d_disp, 3 * k * sizeof(float)));
   }
+  KMC_HIP(c, hipStreamSynchronize(c->stream));
+  if (row_ptr) row_ptr[n] = nnz;
   return KMC_OK;
 }
 
@@ -1393,19 +1425,13 @@ int kmc_get_excitons(kmc_ctx* c, int32_t* site, double* t_next, uint64_t* hops, 
   if (c->n_exc == 0) return fail(c, KMC_ERR_STATE, "kmc_get_excitons: no excitons");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   const int64_t E = c->n_exc;
-  if (site) KMC_TRY(copy_out(c, site, c->x_site.p, E * sizeof(int32_t)));
-  if (t_next) KMC_TRY(copy_out(c, t_next, c->x_t.p, E * sizeof(double)));
-  if (hops) KMC_TRY(copy_out(c, hops, c->x_hops.p, E * sizeof(uint64_t)));
-  if (drains) KMC_TRY(copy_out(c, drains, c->x_drains.p, E * sizeof(uint32_t)));
-  if (seq_hash) KMC_TRY(copy_out(c, seq_hash, c->x_hash.p, E * sizeof(uint64_t)));
-  if (disp) {
-    std::vector<double> v(E);
-    const dbuf<double>* src[3] = {&c->x_dx, &c->x_dy, &c->x_dz};
-    for (int a = 0; a < 3; ++a) {
-      KMC_TRY(copy_out(c, v.data(), src[a]->p, E * sizeof(double)));
-      for (int64_t e = 0; e < E; ++e) disp[3 * e + a] = v[e];
-    }
-  }
+  if (site) KMC_TRY(queue_out(c, site, c->x_site.p, E * sizeof(int32_t)));
+  if (t_next) KMC_TRY(queue_out(c, t_next, c->x_t.p, E * sizeof(double)));
+  if (hops) KMC_TRY(queue_out(c, hops, c->x_hops.p, E * sizeof(uint64_t)));
+  if (drains) KMC_TRY(queue_out(c, drains, c->x_drains.p, E * sizeof(uint32_t)));
+  if (seq_hash) KMC_TRY(queue_out(c, seq_hash, c->x_hash.p, E * sizeof(uint64_t)));
+  if (disp) KMC_TRY(queue_out3(c, disp, c->x_dx.p, c->x_dy.p, c->x_dz.p, E));
+  KMC_HIP(c, hipStreamSynchronize(c->stream));
   return KMC_OK;
 }
 
@@ -1442,17 +1468,12 @@ int kmc_get_run_stats(kmc_ctx* c, int64_t* launches, int64_t* live_excitons) {
 int kmc_get_samples(kmc_ctx* c, double* disp, uint32_t* drains, uint32_t* n_recorded) {
   if (!c) return fail(nullptr, KMC_ERR_ARG, "kmc_get_samples: null context");
   if (c->n_bins == 0) return fail(c, KMC_ERR_STATE, "kmc_get_samples: no sampling grid");
+  KMC_HIP(c, hipSetDevice(c->cfg.device));
   const size_t nrec = (size_t)window_bins(c) * c->n_exc;
-  if (disp) {
-    std::vector<double> v(nrec);
-    const dbuf<double>* src[3] = {&c->r_dx, &c->r_dy, &c->r_dz};
-    for (int a = 0; a < 3; ++a) {
-      KMC_TRY(copy_out(c, v.data(), src[a]->p, nrec * sizeof(double)));
-      for (size_t r = 0; r < nrec; ++r) disp[3 * r + a] = v[r];
-    }
-  }
-  if (drains) KMC_TRY(copy_out(c, drains, c->r_drain.p, nrec * sizeof(uint32_t)));
-  if (n_recorded) KMC_TRY(copy_out(c, n_recorded, c->x_krec.p, c->n_exc * sizeof(uint32_t)));
+  if (disp) KMC_TRY(queue_out3(c, disp, c->r_dx.p, c->r_dy.p, c->r_dz.p, (int64_t)nrec));
+  if (drains) KMC_TRY(queue_out(c, drains, c->r_drain.p, nrec * sizeof(uint32_t)));
+  if (n_recorded) KMC_TRY(queue_out(c, n_recorded, c->x_krec.p, c->n_exc * sizeof(uint32_t)));
+  KMC_HIP(c, hipStreamSynchronize(c->stream));
   return KMC_OK;
 }
 

@@ -160,6 +160,13 @@ hipError_t launch_fill_pairs(int mode, const site_arrays& s, const cell_desc& c,
                              const int64_t* row_ptr, int64_t nnz, const table_desc& t,
                              const csr_arrays& out, const pair_geom_arrays& geo, int32_t* err,
                              hipStream_t st);
+// read-back: the caller's layouts from the device's (null outputs are left out)
+hipError_t launch_unpack_edges(int64_t n, const edge_rec* edge, int32_t* col, float* disp,
+                               hipStream_t st);
+hipError_t launch_unpack_rows(int64_t n, const site_hdr* hdr, int64_t* row, double* gamma,
+                              hipStream_t st);
+hipError_t launch_interleave3(int64_t n, const double* x, const double* y, const double* z,
+                              double* out, hipStream_t st);
 hipError_t launch_finish_pair_rates(int64_t n, const double* rates, const csr_arrays& out,
                                     int32_t* err, hipStream_t st);
 hipError_t launch_inject(const exciton_arrays& x, const uint4* blocks, const uint32_t* src_roff,

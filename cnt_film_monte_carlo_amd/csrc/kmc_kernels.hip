@@ -310,6 +310,44 @@ __global__ __launch_bounds__(256) void k_pair_values(int64_t p0, int64_t nnz, si
   }
 }
 
+// Pairs [p0, p0 + n) as the caller's arrays hold them (col and disp optional).
+__global__ __launch_bounds__(256) void k_unpack_edges(int64_t n, const edge_rec* __restrict__ edge,
+                                                      int32_t* __restrict__ col,
+                                                      float* __restrict__ disp) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const edge_rec e = edge[p];
+  if (col) col[p] = (int32_t)(e.col & EDGE_COL_MASK);
+  if (disp) {
+    disp[3 * p] = e.dx;
+    disp[3 * p + 1] = e.dy;
+    disp[3 * p + 2] = e.dz;
+  }
+}
+
+// Row starts and total rates of n sites (either optional).
+__global__ __launch_bounds__(256) void k_unpack_rows(int64_t n, const site_hdr* __restrict__ hdr,
+                                                     int64_t* __restrict__ row,
+                                                     double* __restrict__ gamma) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const site_hdr h = hdr[i];
+  if (row) row[i] = h.rs;
+  if (gamma) gamma[i] = h.gamma;
+}
+
+// Three arrays of n values interleaved: out[3 k + a].
+__global__ __launch_bounds__(256) void k_interleave3(int64_t n, const double* __restrict__ x,
+                                                     const double* __restrict__ y,
+                                                     const double* __restrict__ z,
+                                                     double* __restrict__ out) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  out[3 * k] = x[k];
+  out[3 * k + 1] = y[k];
+  out[3 * k + 2] = z[k];
+}
+
 // Sequential FP64 inclusive prefix sum per row from per-pair rates (scatterer.cpp:78-80).
 // rates may be out.cum itself.
 __global__ __launch_bounds__(256) void k_finish_pair_rates(int64_t n, const double* rates,
@@ -2280,6 +2318,27 @@ hipError_t launch_fill_pairs(int mode, const site_arrays& s, const cell_desc& c,
   }
   const hipError_t e = hipGetLastError();
   return e != hipSuccess || mode != 0 ? e : launch_finish_pair_rates(s.n, out.cum, out, err, st);
+}
+
+hipError_t launch_unpack_edges(int64_t n, const edge_rec* edge, int32_t* col, float* disp,
+                               hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_unpack_edges, grid_for(n), dim3(256), 0, st, n, edge, col, disp);
+  return hipGetLastError();
+}
+
+hipError_t launch_unpack_rows(int64_t n, const site_hdr* hdr, int64_t* row, double* gamma,
+                              hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_unpack_rows, grid_for(n), dim3(256), 0, st, n, hdr, row, gamma);
+  return hipGetLastError();
+}
+
+hipError_t launch_interleave3(int64_t n, const double* x, const double* y, const double* z,
+                              double* out, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_interleave3, grid_for(n), dim3(256), 0, st, n, x, y, z, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_finish_pair_rates(int64_t n, const double* rates, const csr_arrays& out,
