@@ -187,7 +187,7 @@ struct kmc_ctx {
   dbuf<uint8_t> c_head[2];
   int c_buf = 0;                          // the buffer holding the live particles
   dbuf<uint32_t> c_keep;
-  dbuf<int64_t> c_off, c_scan_tmp, c_live, c_live_out;
+  dbuf<int64_t> c_off, c_scan_tmp, c_live, c_live_out, c_base;
   dbuf<uint64_t> c_next;
   dbuf<int32_t> c_err, c_pop_out, c_cur_out;
   dbuf<uint64_t> c_made;                  // hops made since kmc_contact_init
@@ -561,7 +561,7 @@ int kmc_destroy(kmc_ctx* c) {
   dfree(c->d_site_count); dfree(c->r_dx); dfree(c->r_dy); dfree(c->r_dz);
   dfree(c->d_reduced); dfree(c->r_drain); dfree(c->tr_site); dfree(c->tr_time); dfree(c->tr_n);
   dfree(c->d_min);
-  dfree(c->c_sites); dfree(c->c_keep); dfree(c->c_off); dfree(c->c_scan_tmp); dfree(c->c_live);
+  dfree(c->c_sites); dfree(c->c_keep); dfree(c->c_off); dfree(c->c_scan_tmp); dfree(c->c_live); dfree(c->c_base);
   dfree(c->c_live_out); dfree(c->c_next); dfree(c->c_err); dfree(c->c_pop_out); dfree(c->c_cur_out);
   dfree(c->c_made); dfree(c->c_skeys); dfree(c->c_sids); dfree(c->c_sort_tmp);
   for (hipEvent_t e : c->c_ev)
@@ -1946,33 +1946,32 @@ contact_slots contact_buf(kmc_ctx* c, int b) {
 
 // The order in which a step's threads take the live slots.  Slots sort by the eighth of the film
 // their site lies in (the eighths of the sorted slots go to the eight XCDs, so each XCD's L2
-// serves one compact region), then by the site's chirality, then by the site's row.  The
-// chirality sets the rates a particle meets along its tube, so the particles of one wave make
-// similar numbers of hops in a step and fewer of its lanes idle while its last particle hops.
-// A film whose keys would not fit 32 bits sorts by the row alone.
+// serves one compact region), then by the site's chirality, then by the site's row in the eighth,
+// to as many of the row's leading bits as the sort's last 8-bit pass has left.  The chirality sets
+// the rates a particle meets along its tube, so the particles of one wave make similar numbers of
+// hops in a step and fewer of its lanes idle while its last particle hops.  Finer rows gain
+// nothing: with 1 M particles on 625k sites of three chiralities the sort and the step kernel take
+// 73 + 655 us with 8 key bits, 124 + 685 with 16 and 178 + 687 with all 28; with one chirality
+// the kernel takes 6.5 ms at 8 bits, 6.9 at 11 and 7.0 at 16.
+// Dead slots follow the live ones in the sort's input and have the largest key, so its stability
+// leaves them last.
 contact_key_layout contact_key_layout_of(const kmc_ctx* c, uint32_t lines) {
-  const auto bits = [](uint64_t v) {  // bits that hold the values [0, v]
+  const auto bits = [](uint32_t v) {  // bits that hold the values [0, v]
     int b = 1;
-    while (b < 64 && (v >> b) != 0) ++b;
+    while (b < 32 && (v >> b) != 0) ++b;
     return b;
   };
+  static_assert(KMC_COUNT_COPIES == 8, "three key bits hold the eighth");
   contact_key_layout kl{};
   kl.lines = lines;
   uint8_t top = 0;
   for (const uint8_t ch : c->h_chir) top = std::max(top, ch);
   kl.chir_bits = top ? bits(top) : 0;
-  kl.row_bits = bits(lines - 1u);
-  if (4 + kl.chir_bits + kl.row_bits <= 32) {
-    kl.regions = 1;
-    kl.dead = (uint32_t)KMC_COUNT_COPIES << (kl.chir_bits + kl.row_bits);
-    kl.key_bits = 4 + kl.chir_bits + kl.row_bits;
-  } else {
-    kl.regions = 0;
-    kl.chir_bits = 0;
-    kl.dead = lines;
-    kl.key_bits = std::min(bits(lines), 32);
-    kl.row_bits = kl.key_bits;
-  }
+  const int row_bits = bits(lines / KMC_COUNT_COPIES + 1u);  // an eighth starts at a rounded line
+  kl.row_bits = std::min(row_bits, (3 + kl.chir_bits + 7) / 8 * 8 - (3 + kl.chir_bits));
+  kl.row_shift = row_bits - kl.row_bits;
+  kl.key_bits = 3 + kl.chir_bits + kl.row_bits;
+  kl.dead = (1u << kl.key_bits) - 1u;
   return kl;
 }
 
@@ -2130,7 +2129,9 @@ int kmc_contact_init(kmc_ctx* c, int32_t n_seg, int64_t c1_pop, int64_t c2_pop, 
     KMC_TRY(dalloc(c, c->c_tlast[b], capacity));
   }
   KMC_TRY(dalloc(c, c->c_keep, capacity));
-  KMC_TRY(dalloc(c, c->c_off, capacity + 1));
+  // scan offsets of the slots, or the two counts of every tile of them
+  KMC_TRY(dalloc(c, c->c_off, std::max(capacity + 1, 2 * scan_tmp_elems(capacity))));
+  KMC_TRY(dalloc(c, c->c_base, 3));
   KMC_TRY(dalloc(c, c->c_scan_tmp, scan_tmp_elems(capacity)));
   KMC_TRY(dalloc(c, c->c_live, 1));
   KMC_TRY(dalloc(c, c->c_next, 1));
@@ -2240,27 +2241,56 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
     c->c_time = a.t_end;  // _time += dt (monte_carlo.h:354)
     // repopulate_contacts (monte_carlo.h:443-491): contact 1, then contact n_seg; the kept
     // particles keep their order, the new ones follow them
-    int64_t n_side = bound;  // slots the live ones lie in: contact 1's injection may add some
-    for (int side = 0; side < 2; ++side) {
-      a.s = contact_buf(c, c->c_buf);
-      KMC_HIP(c, launch_contact_keep(a, n_side, c->c_rm_lo[side], c->c_rm_hi[side], c->c_keep.p,
-                                     c->stream));
-      KMC_HIP(c, exclusive_scan(c->c_keep.p, c->c_off.p, n_side, c->c_scan_tmp.p, c->stream));
-      KMC_HIP(c, launch_contact_compact(n_side, contact_buf(c, c->c_buf),
-                                        contact_buf(c, 1 - c->c_buf), c->c_keep.p, c->c_off.p,
-                                        c->stream));
-      c->c_buf = 1 - c->c_buf;
-      a.s = contact_buf(c, c->c_buf);
-      KMC_HIP(c, launch_contact_inject(a, c->c_off.p + n_side, c->c_pop[side],
-                                       c->c_sites.p + c->c_list_off[side], c->c_list_n[side],
-                                       c->c_next.p, c->c_time, c->c_live.p, c->stream));
-      n_side = std::min(cap, n_side + c->c_pop[side]);
-    }
-    KMC_HIP(c, hipMemcpyAsync(c->c_live_out.p + k, c->c_live.p, sizeof(int64_t),
-                              hipMemcpyDeviceToDevice, c->stream));
     const int slot = (int)(k % CONTACT_LIVE_LAG);
-    KMC_HIP(c, hipMemcpyAsync(c->c_live_host + slot, c->c_live.p, sizeof(int64_t),
-                              hipMemcpyDeviceToHost, c->stream));
+    if (c->c_rm_hi[0] < c->c_rm_lo[1]) {
+      contact_move_args m{};
+      m.src = contact_buf(c, c->c_buf);
+      m.dst = contact_buf(c, 1 - c->c_buf);
+      m.drift = c->c_vel > 0.0;
+      m.capacity = cap;
+      for (int side = 0; side < 2; ++side) {
+        m.rm_lo[side] = c->c_rm_lo[side];
+        m.rm_hi[side] = c->c_rm_hi[side];
+        m.count[side] = c->c_pop[side];
+        m.list_off[side] = c->c_list_off[side];
+        m.list_n[side] = c->c_list_n[side];
+      }
+      m.sites = c->c_sites.p;
+      m.t_now = c->c_time;
+      m.tile_kept = c->c_off.p;  // capacity + 1 entries: room for both tiles' counts
+      m.tile_first = c->c_off.p + scan_tmp_elems(bound);
+      m.base = c->c_base.p;
+      m.n_live = c->c_live.p;
+      m.next_id = c->c_next.p;
+      m.live_out = c->c_live_out.p + k;
+      m.live_host = c->c_live_host + slot;
+      m.err = c->c_err.p;
+      KMC_HIP(c, launch_contact_move(a, m, bound, c->stream));
+      c->c_buf = 1 - c->c_buf;
+    } else {
+      // two sections whose closed ranges share a site's y: contact n_seg may remove particles that
+      // contact 1 has just placed
+      int64_t n_side = bound;  // slots the live ones lie in: contact 1's injection may add some
+      for (int side = 0; side < 2; ++side) {
+        a.s = contact_buf(c, c->c_buf);
+        KMC_HIP(c, launch_contact_keep(a, n_side, c->c_rm_lo[side], c->c_rm_hi[side], c->c_keep.p,
+                                       c->stream));
+        KMC_HIP(c, exclusive_scan(c->c_keep.p, c->c_off.p, n_side, c->c_scan_tmp.p, c->stream));
+        KMC_HIP(c, launch_contact_compact(n_side, contact_buf(c, c->c_buf),
+                                          contact_buf(c, 1 - c->c_buf), c->c_keep.p, c->c_off.p,
+                                          c->stream));
+        c->c_buf = 1 - c->c_buf;
+        a.s = contact_buf(c, c->c_buf);
+        KMC_HIP(c, launch_contact_inject(a, c->c_off.p + n_side, c->c_pop[side],
+                                         c->c_sites.p + c->c_list_off[side], c->c_list_n[side],
+                                         c->c_next.p, c->c_time, c->c_live.p, c->stream));
+        n_side = std::min(cap, n_side + c->c_pop[side]);
+      }
+      KMC_HIP(c, hipMemcpyAsync(c->c_live_out.p + k, c->c_live.p, sizeof(int64_t),
+                                hipMemcpyDeviceToDevice, c->stream));
+      KMC_HIP(c, hipMemcpyAsync(c->c_live_host + slot, c->c_live.p, sizeof(int64_t),
+                                hipMemcpyDeviceToHost, c->stream));
+    }
     KMC_HIP(c, hipEventRecord(c->c_live_ev[slot], c->stream));
   }
   KMC_HIP(c, hipStreamSynchronize(c->stream));

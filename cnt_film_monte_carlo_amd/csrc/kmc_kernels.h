@@ -102,6 +102,25 @@ struct contact_args {
   const uint32_t* perm;     // thread j steps slot perm[j] (the sorted slots); null: slot j
 };
 
+// Repopulation of both contacts in one pass (k_contact_count, _offsets, _move).
+struct contact_move_args {
+  contact_slots src, dst;
+  int32_t drift;            // v > 0: heading, s_off and t_last move too
+  int64_t capacity;
+  double rm_lo[2], rm_hi[2];  // y ranges the contacts clear
+  int64_t count[2];         // new particles of each contact
+  const int32_t* sites;     // the contacts' site lists, at list_off, list_n long
+  int64_t list_off[2], list_n[2];
+  double t_now;
+  int64_t* tile_kept;       // per tile of slots: kept by both contacts (then its offset)
+  int64_t* tile_first;      // kept by contact 1 alone (its injection must fit beside them)
+  int64_t* base;            // [3]: kept, first new id, slots counted
+  int64_t* n_live;
+  uint64_t* next_id;
+  int64_t *live_out, *live_host;
+  int32_t* err;
+};
+
 struct trace_view {         // trace [n_trace][tr_max] (single network only)
   int64_t n_trace = 0, tr_max = 0;
   int32_t* tr_site = nullptr;
@@ -199,8 +218,8 @@ hipError_t launch_fill_blocks(int64_t n, const site_hdr* hdr, const double* cum,
 struct contact_key_layout {
   uint32_t lines;      // row lines of the film (the eighths split [0, lines))
   int32_t row_bits, chir_bits;
-  int32_t regions;     // 0: the key is the row line alone
-  uint32_t dead;
+  int32_t row_shift;   // the key holds a row's place in its eighth >> row_shift
+  uint32_t dead;       // the largest key
   int32_t key_bits;    // bits the radix sort looks at
 };
 // keys[i] = sort key of slot i (contact_key_layout), ids[i] = i
@@ -249,6 +268,9 @@ hipError_t launch_contact_keep(const contact_args& a, int64_t n, double y_lo, do
 hipError_t launch_contact_compact(int64_t capacity, const contact_slots& src,
                                   const contact_slots& dst, const uint32_t* keep,
                                   const int64_t* off, hipStream_t st);
+// both contacts' repopulation of slots [0, n), n >= *m.n_live; m.rm_* ranges disjoint
+hipError_t launch_contact_move(const contact_args& a, const contact_move_args& m, int64_t n,
+                               hipStream_t st);
 hipError_t launch_contact_inject(const contact_args& a, const int64_t* base, int64_t count,
                                  const int32_t* sites, int64_t n_sites, uint64_t* next_id,
                                  double t_now, int64_t* n_live, hipStream_t st);

@@ -2059,11 +2059,10 @@ __global__ __launch_bounds__(256) void k_contact_keys(int64_t capacity, const in
   if (e < *n_live) {
     const int32_t s = site[e];
     const uint32_t row = (uint32_t)roff[s];
-    k = row;
-    if (kl.regions) {
-      const uint32_t region = (uint32_t)((uint64_t)row * KMC_COUNT_COPIES / kl.lines);
-      k |= (region << (kl.chir_bits + kl.row_bits)) | ((uint32_t)chir[s] << kl.row_bits);
-    }
+    const uint32_t region = (uint32_t)((uint64_t)row * KMC_COUNT_COPIES / kl.lines);
+    const uint32_t first = (uint32_t)(((uint64_t)region * kl.lines) / KMC_COUNT_COPIES);
+    k = (region << (kl.chir_bits + kl.row_bits)) | ((uint32_t)chir[s] << kl.row_bits) |
+        ((row - first) >> kl.row_shift);
   }
   keys[e] = k;
   ids[e] = (uint32_t)e;
@@ -2215,20 +2214,13 @@ __global__ __launch_bounds__(256) void k_contact_compact(int64_t capacity, conta
   dst.t_last[o] = src.t_last[e];
 }
 
-// `count` new particles in slots *base + k on sites of `sites`, as the particle constructor
-// makes them (particle.h:49-52): a random site of the list (rand() % size), the first dwell
-// from the site (ff_time), then the heading (rand() % 2).  Ids continue from *next_id.
-__global__ __launch_bounds__(256) void k_contact_inject(contact_args a, const int64_t* base,
-                                                        int64_t count,
-                                                        const int32_t* __restrict__ sites,
-                                                        int64_t n_sites,
-                                                        const uint64_t* __restrict__ next_id,
-                                                        double t_now) {
+// A new particle in `slot` on a site of `sites`, as the particle constructor makes it
+// (particle.h:49-52): a random site of the list (rand() % size), the first dwell from the site
+// (ff_time), then the heading (rand() % 2).
+__device__ __forceinline__ void contact_new(const contact_args& a, int64_t slot, uint64_t id64,
+                                            const int32_t* __restrict__ sites, int64_t n_sites,
+                                            double t_now) {
 #pragma clang fp contract(off)
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= count) return;
-  const int64_t slot = *base + k;
-  const uint64_t id64 = *next_id + (uint64_t)k;
   if (slot >= a.capacity) {
     atomicOr(a.err, CONTACT_ERR_CAPACITY);
     return;
@@ -2252,12 +2244,134 @@ __global__ __launch_bounds__(256) void k_contact_inject(contact_args a, const in
   a.s.t_last[slot] = t_now;
 }
 
+// `count` new particles in slots *base + k; ids continue from *next_id.
+__global__ __launch_bounds__(256) void k_contact_inject(contact_args a, const int64_t* base,
+                                                        int64_t count,
+                                                        const int32_t* __restrict__ sites,
+                                                        int64_t n_sites,
+                                                        const uint64_t* __restrict__ next_id,
+                                                        double t_now) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < count) contact_new(a, *base + k, *next_id + (uint64_t)k, sites, n_sites, t_now);
+}
+
 __global__ void k_contact_finish(const int64_t* base, int64_t count, int64_t capacity,
                                  uint64_t* next_id, int64_t* n_live) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   const int64_t n = *base + count;
   *n_live = n < capacity ? n : capacity;
   *next_id += (uint64_t)count;
+}
+
+// Repopulation of both contacts (monte_carlo.h:443-491) in three launches: contact 1 loses the
+// particles whose y lies in its range and gets c_pop[0] new ones, then contact n_seg likewise; the
+// kept particles keep their order and the new ones follow them, contact 1's first.  With disjoint
+// ranges (checked by the caller) contact n_seg removes none of contact 1's new particles, so one
+// pass over the slots decides for both.  Tiles of SCAN_TILE slots: k_contact_count counts what a
+// tile keeps, k_contact_offsets scans the tiles, k_contact_move writes the other buffer.  The move
+// is bound by memory: 72 bytes a particle read and written, by lanes on consecutive slots (eight
+// consecutive slots to a lane, as in the scans: 72 us at 1 M particles, this way 16).  A pass per
+// contact took fourteen launches; a step of 1 M particles took ~110 us outside its sort and step
+// kernel, now 26.
+__device__ __forceinline__ bool in_contact(const contact_move_args& m, int side, double y) {
+  return y >= m.rm_lo[side] && y <= m.rm_hi[side];
+}
+
+__global__ __launch_bounds__(SCAN_THREADS) void k_contact_count(contact_move_args m) {
+  __shared__ int32_t s_kept, s_first;
+  if (threadIdx.x == 0) s_kept = s_first = 0;
+  __syncthreads();
+  const int64_t n = *m.n_live;
+  const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+  int32_t kept = 0, first = 0;  // kept by both contacts; by contact 1
+#pragma unroll
+  for (int i = 0; i < SCAN_ITEMS; ++i) {
+    const int64_t e = base + i * SCAN_THREADS;
+    const double y = e < n ? m.src.y[e] : 0.0;
+    const bool k0 = e < n && !in_contact(m, 0, y);
+    first += __popcll(__ballot(k0));
+    kept += __popcll(__ballot(k0 && !in_contact(m, 1, y)));
+  }
+  if ((threadIdx.x & 63u) == 0) {
+    atomicAdd(&s_kept, kept);
+    atomicAdd(&s_first, first);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    m.tile_kept[blockIdx.x] = s_kept;
+    m.tile_first[blockIdx.x] = s_first;
+  }
+}
+
+__global__ __launch_bounds__(SCAN_THREADS) void k_contact_offsets(contact_move_args m, int64_t n_tiles) {
+  __shared__ int64_t lds[SCAN_THREADS / 64];
+  int64_t kept = 0, first = 0;
+  for (int64_t base = 0; base < n_tiles; base += SCAN_THREADS) {
+    const int64_t i = base + threadIdx.x;
+    int64_t total;
+    const int64_t ex = block_exclusive_scan(i < n_tiles ? m.tile_kept[i] : 0, lds, &total);
+    if (i < n_tiles) m.tile_kept[i] = kept + ex;
+    kept += total;
+    (void)block_exclusive_scan(i < n_tiles ? m.tile_first[i] : 0, lds, &total);
+    first += total;
+  }
+  if (threadIdx.x != 0) return;
+  const int64_t live = kept + m.count[0] + m.count[1];
+  if (first + m.count[0] > m.capacity || live > m.capacity) atomicOr(m.err, CONTACT_ERR_CAPACITY);
+  m.base[0] = kept;
+  m.base[1] = (int64_t)*m.next_id;
+  m.base[2] = *m.n_live;  // the slots counted: k_contact_move looks at the same ones
+  *m.next_id += (uint64_t)(m.count[0] + m.count[1]);
+  *m.n_live = live < m.capacity ? live : m.capacity;
+  *m.live_out = *m.n_live;
+  *m.live_host = *m.n_live;  // pinned host memory
+}
+
+// Blocks [0, n_tiles): the kept particles; the rest: the new ones.
+__global__ __launch_bounds__(SCAN_THREADS) void k_contact_move(contact_args a, contact_move_args m,
+                                                               int64_t n_tiles) {
+#pragma clang fp contract(off)
+  __shared__ int32_t s_kept[SCAN_ITEMS * SCAN_THREADS / 64];
+  if ((int64_t)blockIdx.x < n_tiles) {
+    const int64_t n = m.base[2];
+    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint64_t keep[SCAN_ITEMS];
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) {
+      const int64_t e = base + i * SCAN_THREADS;
+      const double y = e < n ? m.src.y[e] : 0.0;
+      keep[i] = __ballot(e < n && !in_contact(m, 0, y) && !in_contact(m, 1, y));
+      if (lane == 0) s_kept[i * (SCAN_THREADS / 64) + wave] = __popcll(keep[i]);
+    }
+    __syncthreads();
+    int64_t o = m.tile_kept[blockIdx.x];
+    uint32_t before = 0;  // runs of 64 slots added to o
+#pragma unroll
+    for (int i = 0; i < SCAN_ITEMS; ++i) {
+      for (; before < i * (SCAN_THREADS / 64) + wave; ++before) o += s_kept[before];
+      if (!(keep[i] >> lane & 1u)) continue;
+      const int64_t e = base + i * SCAN_THREADS;
+      const int64_t to = o + __popcll(keep[i] & (((uint64_t)1 << lane) - 1u));
+      m.dst.site[to] = m.src.site[e];
+      m.dst.t_next[to] = m.src.t_next[e];
+      m.dst.hops[to] = m.src.hops[e];
+      m.dst.id[to] = m.src.id[e];
+      m.dst.y[to] = m.src.y[e];
+      if (m.drift) {
+        m.dst.heading[to] = m.src.heading[e];
+        m.dst.s_off[to] = m.src.s_off[e];
+        m.dst.t_last[to] = m.src.t_last[e];
+      }
+    }
+    return;
+  }
+  const int64_t k = ((int64_t)blockIdx.x - n_tiles) * blockDim.x + threadIdx.x;
+  if (k >= m.count[0] + m.count[1]) return;
+  const int side = k < m.count[0] ? 0 : 1;
+  a.s = m.dst;
+  contact_new(a, m.base[0] + k, (uint64_t)m.base[1] + (uint64_t)k, m.sites + m.list_off[side],
+              m.list_n[side], m.t_now);
 }
 
 static inline dim3 grid_for(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }
@@ -2548,6 +2662,22 @@ hipError_t launch_contact_compact(int64_t capacity, const contact_slots& src,
   if (capacity == 0) return hipSuccess;
   hipLaunchKernelGGL(k_contact_compact, grid_for(capacity), dim3(256), 0, st, capacity, src, dst,
                      keep, off);
+  return hipGetLastError();
+}
+
+hipError_t launch_contact_move(const contact_args& a, const contact_move_args& m, int64_t n,
+                               hipStream_t st) {
+  if (n < 0 || n > a.capacity || (m.count[0] > 0 && m.list_n[0] < 1) ||
+      (m.count[1] > 0 && m.list_n[1] < 1))
+    return hipErrorInvalidValue;
+  const int64_t n_tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+  const int64_t fresh = (m.count[0] + m.count[1] + SCAN_THREADS - 1) / SCAN_THREADS;
+  if (n_tiles > 0)
+    hipLaunchKernelGGL(k_contact_count, dim3((unsigned)n_tiles), dim3(SCAN_THREADS), 0, st, m);
+  hipLaunchKernelGGL(k_contact_offsets, dim3(1), dim3(SCAN_THREADS), 0, st, m, n_tiles);
+  if (n_tiles + fresh > 0)
+    hipLaunchKernelGGL(k_contact_move, dim3((unsigned)(n_tiles + fresh)), dim3(SCAN_THREADS), 0, st, a,
+                       m, n_tiles);
   return hipGetLastError();
 }
 
