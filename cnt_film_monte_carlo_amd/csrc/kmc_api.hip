@@ -133,7 +133,8 @@ struct kmc_ctx {
   // drift along the tubes (particle::fly): velocity [m/s], links as block lines, error word
   double velocity = 0.0;      // set by kmc_set_velocity
   double exc_velocity = 0.0;  // the velocity of the injected excitons (fixed by kmc_inject)
-  dbuf<uint2> d_links;
+  dbuf<uint4> d_fly_table;    // of this film's rows when fly_ok
+  bool fly_ok = false;
   dbuf<int32_t> d_fly_err;
 
   // excitons
@@ -336,7 +337,7 @@ net_view view_of(kmc_ctx* c) {
   v.site_count = c->d_site_count.p;
   v.count_stride = c->count_stride;
   v.velocity = c->exc_velocity;
-  v.links = c->d_links.p;
+  v.fly_table = c->d_fly_table.p;
   v.fly_err = c->d_fly_err.p;
   v.live = c->d_live.p;
   return v;
@@ -452,10 +453,22 @@ int pack_rows(kmc_ctx* c, const char* who = nullptr) {
   KMC_TRY(dalloc(c, c->d_src_roff, c->h_src.size()));
   KMC_HIP(c, launch_gather_offsets((int64_t)c->h_src.size(), c->d_src.p, c->d_roff.p, c->d_hdr.p,
                                    c->d_src_roff.p, c->stream));
-  KMC_TRY(dalloc(c, c->d_links, n));
-  KMC_HIP(c, launch_links(n, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p, c->d_hdr.p,
-                          c->d_links.p, c->stream));
+  c->fly_ok = false;
   KMC_HIP(c, hipStreamSynchronize(c->stream));
+  return KMC_OK;
+}
+
+// The legs of flights along the tubes: made when particles that drift are first placed on the rows.
+int fly_table(kmc_ctx* c) {
+  if (c->fly_ok) return KMC_OK;
+  double half[3];
+  for (int k = 0; k < 3; ++k)
+    half[k] = (c->cfg.periodic_mask & (1 << k)) ? 0.5 * c->cfg.period_len[k] : INFINITY;
+  KMC_TRY(dalloc(c, c->d_fly_table, 4 * (size_t)c->n_sites));
+  KMC_HIP(c, launch_fly_table(c->n_sites, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p,
+                              c->d_hdr.p, c->d_pos[0].p, c->d_pos[1].p, c->d_pos[2].p, half,
+                              c->d_fly_table.p, c->stream));
+  c->fly_ok = true;
   return KMC_OK;
 }
 
@@ -557,7 +570,7 @@ int kmc_destroy(kmc_ctx* c) {
   dfree(c->d_sel); dfree(c->d_mlp_flag); dfree(c->d_read);
   dfree(c->d_err); dfree(c->x_site); dfree(c->x_t); dfree(c->x_dx); dfree(c->x_dy);
   dfree(c->x_dz); dfree(c->x_hops); dfree(c->x_hash); dfree(c->x_drains); dfree(c->x_krec);
-  dfree(c->x_heading); dfree(c->x_soff); dfree(c->x_tlast); dfree(c->d_links); dfree(c->d_fly_err);
+  dfree(c->x_heading); dfree(c->x_soff); dfree(c->x_tlast); dfree(c->d_fly_table); dfree(c->d_fly_err);
   dfree(c->d_site_count); dfree(c->r_dx); dfree(c->r_dy); dfree(c->r_dz);
   dfree(c->d_reduced); dfree(c->r_drain); dfree(c->tr_site); dfree(c->tr_time); dfree(c->tr_n);
   dfree(c->d_min);
@@ -1119,7 +1132,10 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   c->n_exc = E;
   c->n_bins = c->bin0 = c->win_bins = 0;
   c->n_trace = 0;
-  if (c->velocity > 0.0) KMC_TRY(check_links(c, "kmc_inject"));
+  if (c->velocity > 0.0) {
+    KMC_TRY(check_links(c, "kmc_inject"));
+    KMC_TRY(fly_table(c));
+  }
   c->exc_velocity = c->velocity;
   KMC_HIP(c, launch_inject(excitons_of(c), c->d_blocks.p, c->d_src_roff.p,
                            (uint32_t)c->h_src.size(), c->cfg.seed, c->stream));
@@ -2178,6 +2194,7 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
     return fail(c, KMC_ERR_STATE, "kmc_contact_run: CSR not complete");
   if (n_steps == 0) return KMC_OK;
   KMC_HIP(c, hipSetDevice(c->cfg.device));
+  if (c->c_vel > 0.0) KMC_TRY(fly_table(c));
   const int64_t S = c->c_nseg;
   KMC_TRY(dalloc(c, c->c_pop_out, (size_t)n_steps * S));
   KMC_TRY(dalloc(c, c->c_cur_out, (size_t)n_steps * (S - 1)));

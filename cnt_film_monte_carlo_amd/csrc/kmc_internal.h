@@ -103,6 +103,7 @@ constexpr uint32_t EDGE_DRAIN_BIT = 0x80000000u;
 constexpr uint32_t ROW_UNITS = 8;  // 16-byte units per 128-byte line of the hop kernel's blocks
 // Same-tube links of the drift path: no link (tube end) and the bound on site passes per flight.
 constexpr uint32_t LINK_NONE = 0xFFFFFFFFu;
+constexpr uint32_t FLY_HEADING_BIT = 0x80000000u;  // beside a site index (< 2^31) in a flight leg
 constexpr uint32_t FLY_MAX_PASSES = 1u << 22;
 constexpr uint32_t EDGE_COL_MASK = 0x7FFFFFFFu;
 // Row word of the hop kernel (a target, a source, a link): first line of the site's block |

@@ -60,7 +60,7 @@ struct net_view {
   int64_t count_stride;
   // drift along the tubes (particle::fly), used when velocity > 0
   double velocity;
-  const uint2* links;       // per site: {left, right} block line | drain bit, or LINK_NONE
+  const uint4* fly_table;   // per site and heading: the leg a flight follows (k_fly_table)
   int32_t* fly_err;         // set when a flight exceeds FLY_MAX_PASSES site passes
   // excitons still able to hop at the end of a launch (not trapped, t <= t_max), summed per
   // wave; zeroed by the sort-key kernel ahead of every launch
@@ -252,9 +252,12 @@ hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bo
 bool hop_rows_pays(int64_t movable, int n_cu);
 hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
                            bool sample, bool trace, hipStream_t st);
-// links[i] = {line of left | drain bit, line of right | drain bit}, LINK_NONE for a tube end
-hipError_t launch_links(int64_t n, const int32_t* left, const int32_t* right, const uint8_t* flags,
-                        const int64_t* roff, const site_hdr* hdr, uint2* links, hipStream_t st);
+// table[2 (2 i + heading)], [.. + 1]: the leg of a flight at site i (scatterer::left/right,
+// scatterer.h:29-30; half_per as in net_view)
+hipError_t launch_fly_table(int64_t n, const int32_t* left, const int32_t* right,
+                            const uint8_t* flags, const int64_t* roff, const site_hdr* hdr,
+                            const double* px, const double* py, const double* pz,
+                            const double* half_per, uint4* table, hipStream_t st);
 hipError_t launch_hop_ens(const ens_args& a, bool count, bool sample, hipStream_t st);
 hipError_t launch_ens_keys(int64_t n, const net_view* nets, const uint16_t* exc_net,
                            const int64_t* ebase, uint64_t* keys, uint32_t* ids, uint32_t* live,

@@ -788,25 +788,6 @@ __global__ __launch_bounds__(256) void k_inject(exciton_arrays x, const uint4* _
   x.t_last[e] = 0.0;
 }
 
-// Same-tube links as block lines with the target's drain bit (the flight's view of
-// scatterer::left/right, scatterer.h:29-30).
-__global__ __launch_bounds__(256) void k_links(int64_t n, const int32_t* __restrict__ left,
-                                               const int32_t* __restrict__ right,
-                                               const uint8_t* __restrict__ flags,
-                                               const int64_t* __restrict__ roff,
-                                               const site_hdr* __restrict__ hdr,
-                                               uint2* __restrict__ links) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int32_t l = left[i], r = right[i];
-  uint2 o;
-  o.x = l < 0 ? LINK_NONE
-              : (row_word((uint32_t)roff[l], hdr[l].n) | ((flags[l] & 2u) ? EDGE_DRAIN_BIT : 0u));
-  o.y = r < 0 ? LINK_NONE
-              : (row_word((uint32_t)roff[r], hdr[r].n) | ((flags[r] & 2u) ? EDGE_DRAIN_BIT : 0u));
-  links[i] = o;
-}
-
 // ---------------------------------------------------------------------------------------------
 // Drift along the tube (particle::fly, src/monte_carlo/particle.cpp:9-54) for v > 0.  The
 // exciton sits s_off beyond its current site on the segment toward the next site along its
@@ -825,58 +806,90 @@ struct flight_state {
   uint64_t hs;        // visited-site hash
 };
 
-// Next site along the heading; a tube end reverses the heading (particle.cpp:18-37).
-__device__ __forceinline__ uint32_t fly_next(uint2 lk, uint32_t& heading) {
-  const uint32_t nx = heading ? (lk.y != LINK_NONE ? lk.y : lk.x) : (lk.x != LINK_NONE ? lk.x : lk.y);
-  heading = (nx == lk.y) ? 1u : 0u;
-  return nx;
+// One step along a tube: where the segment that a flight at a site follows under a heading leads.
+// 32 bytes at fly_table[2 (2 site + heading)], the tube end's turn (particle.cpp:18-37) and the
+// segment's length resolved beforehand.  A flight is a chain of dependent loads: with a leg its
+// first segment needs one load, issued at the hop and in flight while the dwell is drawn, and each
+// site passed one more; from the sites' links and row blocks it was three, a square root and a
+// second division (500 hops of 100,003 excitons at 2e5 m/s: 2.26 ms, with legs 1.75; loading the
+// next leg ahead of the comparison as well changed nothing).
+struct fly_leg {
+  uint32_t word;     // row word of the site it leads to | its drain bit; LINK_NONE: no links
+  uint32_t site;     // that site
+  uint32_t heading;  // the heading along the segment (1 = toward `right`)
+  double len;        // the segment's length [m]
+  float x, y, z;     // that site's FP32 position
+};
+
+__device__ __forceinline__ fly_leg load_leg(const net_view& v, uint32_t site, uint32_t heading) {
+  const uint4* b = v.fly_table + 2u * (2u * (size_t)site + heading);
+  const uint4 p = b[0], q = b[1];
+  return fly_leg{p.x, p.y & ~FLY_HEADING_BIT, p.y >> 31, __hiloint2double((int)p.w, (int)p.z),
+                 __uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z)};
 }
 
-__device__ __forceinline__ void fly_segment(const net_view& v, const flight_state& f, uint32_t Rn,
-                                            float& px, float& py, float& pz, double& sx,
-                                            double& sy, double& sz) {
+// The table, a thread per site and heading.
+__global__ __launch_bounds__(256) void k_fly_table(int64_t n, const int32_t* __restrict__ left,
+                                                   const int32_t* __restrict__ right,
+                                                   const uint8_t* __restrict__ flags,
+                                                   const int64_t* __restrict__ roff,
+                                                   const site_hdr* __restrict__ hdr,
+                                                   const double* __restrict__ px,
+                                                   const double* __restrict__ py,
+                                                   const double* __restrict__ pz, double hx, double hy,
+                                                   double hz, uint4* __restrict__ table) {
 #pragma clang fp contract(off)
-  const uint4 p = v.blocks[(size_t)ROW_UNITS * (Rn & TGT_LINE_MASK) + 7];
-  px = __uint_as_float(p.x);
-  py = __uint_as_float(p.y);
-  pz = __uint_as_float(p.z);
-  sx = min_image((double)px - (double)f.x, v.half_per[0]);
-  sy = min_image((double)py - (double)f.y, v.half_per[1]);
-  sz = min_image((double)pz - (double)f.z, v.half_per[2]);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= 2 * n) return;
+  const int64_t i = t >> 1;
+  const int32_t l = left[i], r = right[i];
+  // the heading's next site, else, at a tube end, the other one
+  const int32_t nx = (t & 1) ? (r >= 0 ? r : l) : (l >= 0 ? l : r);
+  uint4 a = make_uint4(LINK_NONE, 0u, 0u, 0u), b = make_uint4(0u, 0u, 0u, 0u);
+  if (nx >= 0) {
+    const float x = (float)px[nx], y = (float)py[nx], z = (float)pz[nx];
+    const double sx = min_image((double)x - (double)(float)px[i], hx);
+    const double sy = min_image((double)y - (double)(float)py[i], hy);
+    const double sz = min_image((double)z - (double)(float)pz[i], hz);
+    const double len = norm3(sx, sy, sz);
+    a = make_uint4(row_word((uint32_t)roff[nx], hdr[nx].n) | ((flags[nx] & 2u) ? EDGE_DRAIN_BIT : 0u),
+                   (uint32_t)nx | (nx == r ? FLY_HEADING_BIT : 0u), (uint32_t)__double2loint(len),
+                   (uint32_t)__double2hiint(len));
+    b = make_uint4(__float_as_uint(x), __float_as_uint(y), __float_as_uint(z), 0u);
+  }
+  table[2 * t] = a;
+  table[2 * t + 1] = b;
 }
 
-// Flight of duration tau.  A site reached on the way becomes the current site; a drain site
-// counts a drain and re-injects on a source site (draw of stream STREAM_FLY_DRAIN + j for the
+// Flight of duration tau; `leg` is the one at (f.site, f.heading) and follows them.  A site
+// reached on the way becomes the current site; a drain site counts a drain and re-injects on a source site (draw of stream STREAM_FLY_DRAIN + j for the
 // j-th drain of this flight, hop counter h), keeping the displacement, and the flight goes on
 // from there, as the reference's next 1 fs step would.  False when the flight would pass more
 // than FLY_MAX_PASSES sites (the state is then left where the bound stopped it).
-__device__ bool fly(const net_view& v, flight_state& f, double tau, uint32_t e, uint64_t h) {
+__device__ __forceinline__ bool fly(const net_view& v, flight_state& f, fly_leg& leg, double tau,
+                                    uint32_t e, uint64_t h) {
 #pragma clang fp contract(off)
-  uint2 lk = v.links[f.site];
-  if (lk.x == LINK_NONE && lk.y == LINK_NONE) return true;  // particle.cpp:11-12
   uint32_t j = 0;
   for (uint32_t pass = 0; pass < FLY_MAX_PASSES; ++pass) {
-    const uint32_t nx = fly_next(lk, f.heading);
-    const uint32_t Rn = nx & ~EDGE_DRAIN_BIT;
-    float px, py, pz;
-    double sx, sy, sz;
-    fly_segment(v, f, Rn, px, py, pz, sx, sy, sz);
-    const double len = norm3(sx, sy, sz);
-    const double dist = len - f.s;
-    if (!(dist / v.velocity < tau)) {  // stops on this segment (particle.cpp:46-49)
+    if (leg.word == LINK_NONE) return true;  // particle.cpp:11-12
+    f.heading = leg.heading;
+    const double dist = leg.len - f.s;
+    const double need = dist / v.velocity;
+    if (!(need < tau)) {  // stops on this segment (particle.cpp:46-49)
       f.s = f.s + v.velocity * tau;
       return true;
     }
-    tau = tau - dist / v.velocity;
-    f.dx = f.dx + sx;
-    f.dy = f.dy + sy;
-    f.dz = f.dz + sz;
+    tau = tau - need;
+    f.dx = f.dx + min_image((double)leg.x - (double)f.x, v.half_per[0]);
+    f.dy = f.dy + min_image((double)leg.y - (double)f.y, v.half_per[1]);
+    f.dz = f.dz + min_image((double)leg.z - (double)f.z, v.half_per[2]);
     f.s = 0.0;
-    f.R = Rn;
-    f.site = v.blocks[(size_t)ROW_UNITS * (Rn & TGT_LINE_MASK)].y;
-    f.x = px;
-    f.y = py;
-    f.z = pz;
+    const uint32_t nx = leg.word;
+    f.R = nx & ~EDGE_DRAIN_BIT;
+    f.site = leg.site;
+    f.x = leg.x;
+    f.y = leg.y;
+    f.z = leg.z;
     f.hs = (f.hs ^ ((uint64_t)f.site | (2ull << 32))) * FNV_PRIME;
     if (nx & EDGE_DRAIN_BIT) {
       ++f.nd;
@@ -891,27 +904,21 @@ __device__ bool fly(const net_view& v, flight_state& f, double tau, uint32_t e, 
       f.z = __uint_as_float(p.z);
       f.hs = (f.hs ^ ((uint64_t)f.site | (1ull << 32))) * FNV_PRIME;
     }
-    lk = v.links[f.site];
-    if (lk.x == LINK_NONE && lk.y == LINK_NONE) return true;
+    leg = load_leg(v, f.site, f.heading);
   }
-  return false;
+  return leg.word == LINK_NONE;
 }
 
 // Position of the exciton relative to its current site: s along the segment toward the next one.
-__device__ __forceinline__ void fly_offset(const net_view& v, const flight_state& f, double& ox,
-                                           double& oy, double& oz) {
+__device__ __forceinline__ void fly_offset(const net_view& v, const flight_state& f,
+                                           const fly_leg& leg, double& ox, double& oy, double& oz) {
 #pragma clang fp contract(off)
   ox = oy = oz = 0.0;
   if (!(f.s != 0.0)) return;
-  uint32_t hd = f.heading;
-  const uint32_t Rn = fly_next(v.links[f.site], hd) & ~EDGE_DRAIN_BIT;
-  float px, py, pz;
-  double sx, sy, sz;
-  fly_segment(v, f, Rn, px, py, pz, sx, sy, sz);
-  const double q = f.s / norm3(sx, sy, sz);
-  ox = sx * q;
-  oy = sy * q;
-  oz = sz * q;
+  const double q = f.s / leg.len;
+  ox = min_image((double)leg.x - (double)f.x, v.half_per[0]) * q;
+  oy = min_image((double)leg.y - (double)f.y, v.half_per[1]) * q;
+  oz = min_image((double)leg.z - (double)f.z, v.half_per[2]) * q;
 }
 
 // One exciton through its hop budget (event-driven form of particle::step,
@@ -936,6 +943,8 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
   const uint32_t R0 = (uint32_t)v.roff[v.x.site[e]];
   uint32_t R = row_word(R0, v.blocks[(size_t)ROW_UNITS * R0].x);
   row_regs row = load_row(v.blocks, R);
+  fly_leg leg{};
+  if (FLY) leg = load_leg(v, row.site, hd);
   const uint64_t h_end = h + hop_budget;
   const size_t E = v.x.n;
   count_cache cc;
@@ -950,12 +959,13 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
         const size_t r = (size_t)(k - (uint32_t)v.bin0) * E + e;
         if (FLY) {  // the flight from the last event up to tk
           flight_state g{R, row.site, row.x, row.y, row.z, so, hd, dx, dy, dz, nd, hs};
-          if (!fly(v, g, tk - tl, e, h)) {
+          fly_leg gl = leg;
+          if (!fly(v, g, gl, tk - tl, e, h)) {
             atomicOr(v.fly_err, 1);
             break;
           }
           double ox, oy, oz;
-          fly_offset(v, g, ox, oy, oz);
+          fly_offset(v, g, gl, ox, oy, oz);
           v.rec_dx[r] = g.dx + ox;
           v.rec_dy[r] = g.dy + oy;
           v.rec_dz[r] = g.dz + oz;
@@ -973,7 +983,7 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
       if (h >= h_end || !(t <= t_max) || !(t < INFINITY)) break;
       // fly through the dwell, then hop from the site reached (particle.cpp:62-75)
       flight_state g{R, row.site, row.x, row.y, row.z, so, hd, dx, dy, dz, nd, hs};
-      if (!fly(v, g, t - tl, e, h)) {
+      if (!fly(v, g, leg, t - tl, e, h)) {
         atomicOr(v.fly_err, 1);
         break;
       }
@@ -1018,6 +1028,8 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
     dy = dy + min_image((double)row.y - (double)sy, v.half_per[1]);
     dz = dz + min_image((double)row.z - (double)sz, v.half_per[2]);
     hs = (hs ^ (uint64_t)row.site) * FNV_PRIME;
+    // the flight's first leg, in flight while the dwell is drawn
+    if (FLY) leg = load_leg(v, row.site, hd);
     const uint32_t r = nonzero_draw1(w_dw, v.seed, e, h, STREAM_HOP_REDRAW);
     t = t + dwell_time(row.n, row.gamma, r);
     // drain: count current and re-inject, keeping displacement and dwell (kubo_step,
@@ -1027,6 +1039,7 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
       R = v.src_roff[r31(draw4(v.seed, e, h, STREAM_REINJECT).v[0]) % v.n_src];
       row = load_row(v.blocks, R);
       hs = (hs ^ ((uint64_t)row.site | (1ull << 32))) * FNV_PRIME;
+      if (FLY) leg = load_leg(v, row.site, hd);
     }
     if (FLY) {
       so = 0.0;
@@ -1988,10 +2001,11 @@ __global__ __launch_bounds__(256) void k_contact_fly(contact_args a) {
     double tl = a.s.t_last[e];
     flight_state g{R, row.site, row.x, row.y, row.z, a.s.s_off[e], (uint32_t)a.s.heading[e],
                    0.0, 0.0, 0.0, 0u, 0ull};
+    fly_leg leg = load_leg(a.fv, g.site, g.heading);
     uint64_t made = 0;
     hop_words hw;
     while (t <= a.t_end) {
-      if (!fly(a.fv, g, t - tl, id, h)) {
+      if (!fly(a.fv, g, leg, t - tl, id, h)) {
         atomicOr(a.err, CONTACT_ERR_FLY);
         break;
       }
@@ -2018,15 +2032,16 @@ __global__ __launch_bounds__(256) void k_contact_fly(contact_args a) {
       row = load_row(a.blocks, R);
       const uint32_t r = nonzero_draw1(w_dw, a.seed, id, h, STREAM_HOP_REDRAW);
       g = flight_state{R, row.site, row.x, row.y, row.z, 0.0, g.heading, 0.0, 0.0, 0.0, 0u, 0ull};
+      leg = load_leg(a.fv, g.site, g.heading);  // in flight while the dwell is drawn
       tl = t;
       t = t + dwell_time(row.n, row.gamma, r);
       ++h;
       ++made;
     }
-    if (!fly(a.fv, g, a.t_end - tl, id, h)) atomicOr(a.err, CONTACT_ERR_FLY);
+    if (!fly(a.fv, g, leg, a.t_end - tl, id, h)) atomicOr(a.err, CONTACT_ERR_FLY);
     tl = a.t_end;
     double ox, oy, oz;
-    fly_offset(a.fv, g, ox, oy, oz);
+    fly_offset(a.fv, g, leg, ox, oy, oz);
     const double y_new = a.py[g.site] + oy;
     a.s.site[e] = (int32_t)g.site;
     a.s.heading[e] = (uint8_t)g.heading;
@@ -2594,11 +2609,13 @@ hipError_t launch_mask_count(int64_t nnz, const uint8_t* cls, const uint8_t* mas
   return hipGetLastError();
 }
 
-hipError_t launch_links(int64_t n, const int32_t* left, const int32_t* right, const uint8_t* flags,
-                        const int64_t* roff, const site_hdr* hdr, uint2* links, hipStream_t st) {
+hipError_t launch_fly_table(int64_t n, const int32_t* left, const int32_t* right,
+                            const uint8_t* flags, const int64_t* roff, const site_hdr* hdr,
+                            const double* px, const double* py, const double* pz,
+                            const double* half_per, uint4* table, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_links, grid_for(n), dim3(256), 0, st, n, left, right, flags, roff, hdr,
-                     links);
+  hipLaunchKernelGGL(k_fly_table, grid_for(2 * n), dim3(256), 0, st, n, left, right, flags, roff, hdr,
+                     px, py, pz, half_per[0], half_per[1], half_per[2], table);
   return hipGetLastError();
 }
 
