@@ -464,7 +464,7 @@ int fly_table(kmc_ctx* c) {
   double half[3];
   for (int k = 0; k < 3; ++k)
     half[k] = (c->cfg.periodic_mask & (1 << k)) ? 0.5 * c->cfg.period_len[k] : INFINITY;
-  KMC_TRY(dalloc(c, c->d_fly_table, 4 * (size_t)c->n_sites));
+  KMC_TRY(dalloc(c, c->d_fly_table, 4 * (size_t)(c->n_units / ROW_UNITS)));
   KMC_HIP(c, launch_fly_table(c->n_sites, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p,
                               c->d_hdr.p, c->d_pos[0].p, c->d_pos[1].p, c->d_pos[2].p, half,
                               c->d_fly_table.p, c->stream));

@@ -60,7 +60,7 @@ struct net_view {
   int64_t count_stride;
   // drift along the tubes (particle::fly), used when velocity > 0
   double velocity;
-  const uint4* fly_table;   // per site and heading: the leg a flight follows (k_fly_table)
+  const uint4* fly_table;   // per block line and heading: the leg a flight follows (k_fly_table)
   int32_t* fly_err;         // set when a flight exceeds FLY_MAX_PASSES site passes
   // excitons still able to hop at the end of a launch (not trapped, t <= t_max), summed per
   // wave; zeroed by the sort-key kernel ahead of every launch
@@ -252,7 +252,7 @@ hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bo
 bool hop_rows_pays(int64_t movable, int n_cu);
 hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
                            bool sample, bool trace, hipStream_t st);
-// table[2 (2 i + heading)], [.. + 1]: the leg of a flight at site i (scatterer::left/right,
+// table[2 (2 roff[i] + heading)], [.. + 1]: the leg of a flight at site i (scatterer::left/right,
 // scatterer.h:29-30; half_per as in net_view)
 hipError_t launch_fly_table(int64_t n, const int32_t* left, const int32_t* right,
                             const uint8_t* flags, const int64_t* roff, const site_hdr* hdr,

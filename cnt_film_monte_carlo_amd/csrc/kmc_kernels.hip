@@ -807,12 +807,12 @@ struct flight_state {
 };
 
 // One step along a tube: where the segment that a flight at a site follows under a heading leads.
-// 32 bytes at fly_table[2 (2 site + heading)], the tube end's turn (particle.cpp:18-37) and the
-// segment's length resolved beforehand.  A flight is a chain of dependent loads: with a leg its
-// first segment needs one load, issued at the hop and in flight while the dwell is drawn, and each
-// site passed one more; from the sites' links and row blocks it was three, a square root and a
-// second division (500 hops of 100,003 excitons at 2e5 m/s: 2.26 ms, with legs 1.75; loading the
-// next leg ahead of the comparison as well changed nothing).
+// 32 bytes at fly_table[2 (2 line + heading)], line the first of the site's block, the tube end's
+// turn (particle.cpp:18-37) and the segment's length resolved beforehand.  A flight is a chain of
+// dependent loads: with a leg its first segment needs one load, issued at the hop and in flight
+// while the dwell is drawn, and each site passed one more; from the sites' links and row blocks it
+// was three, a square root and a second division (500 hops of 100,003 excitons at 2e5 m/s: 2.26 ms,
+// with legs 1.75; loading the next leg ahead of the comparison as well changed nothing).
 struct fly_leg {
   uint32_t word;     // row word of the site it leads to | its drain bit; LINK_NONE: no links
   uint32_t site;     // that site
@@ -821,11 +821,18 @@ struct fly_leg {
   float x, y, z;     // that site's FP32 position
 };
 
-__device__ __forceinline__ fly_leg load_leg(const net_view& v, uint32_t site, uint32_t heading) {
-  const uint4* b = v.fly_table + 2u * (2u * (size_t)site + heading);
-  const uint4 p = b[0], q = b[1];
+__device__ __forceinline__ const uint4* leg_of(const net_view& v, uint32_t W, uint32_t heading) {
+  return v.fly_table + 2u * (2u * (size_t)(W & TGT_LINE_MASK) + heading);
+}
+
+__device__ __forceinline__ fly_leg leg_from_units(const uint4& p, const uint4& q) {
   return fly_leg{p.x, p.y & ~FLY_HEADING_BIT, p.y >> 31, __hiloint2double((int)p.w, (int)p.z),
                  __uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z)};
+}
+
+__device__ __forceinline__ fly_leg load_leg(const net_view& v, uint32_t W, uint32_t heading) {
+  const uint4* b = leg_of(v, W, heading);
+  return leg_from_units(b[0], b[1]);
 }
 
 // The table, a thread per site and heading.
@@ -857,14 +864,15 @@ __global__ __launch_bounds__(256) void k_fly_table(int64_t n, const int32_t* __r
                    (uint32_t)__double2hiint(len));
     b = make_uint4(__float_as_uint(x), __float_as_uint(y), __float_as_uint(z), 0u);
   }
-  table[2 * t] = a;
-  table[2 * t + 1] = b;
+  uint4* o = table + 2 * (2 * roff[i] + (t & 1));
+  o[0] = a;
+  o[1] = b;
 }
 
-// Flight of duration tau; `leg` is the one at (f.site, f.heading) and follows them.  A site
-// reached on the way becomes the current site; a drain site counts a drain and re-injects on a source site (draw of stream STREAM_FLY_DRAIN + j for the
-// j-th drain of this flight, hop counter h), keeping the displacement, and the flight goes on
-// from there, as the reference's next 1 fs step would.  False when the flight would pass more
+// Flight of duration tau; `leg` is the one at (f.R, f.heading) and follows them.  A site reached on
+// the way becomes the current site; a drain site counts a drain and re-injects on a source site
+// (draw of stream STREAM_FLY_DRAIN + j for the j-th drain of this flight, hop counter h), keeping
+// the displacement, and the flight goes on from there, as the reference's next 1 fs step would.  False when the flight would pass more
 // than FLY_MAX_PASSES sites (the state is then left where the bound stopped it).
 __device__ __forceinline__ bool fly(const net_view& v, flight_state& f, fly_leg& leg, double tau,
                                     uint32_t e, uint64_t h) {
@@ -904,7 +912,7 @@ __device__ __forceinline__ bool fly(const net_view& v, flight_state& f, fly_leg&
       f.z = __uint_as_float(p.z);
       f.hs = (f.hs ^ ((uint64_t)f.site | (1ull << 32))) * FNV_PRIME;
     }
-    leg = load_leg(v, f.site, f.heading);
+    leg = load_leg(v, f.R, f.heading);
   }
   return leg.word == LINK_NONE;
 }
@@ -921,157 +929,6 @@ __device__ __forceinline__ void fly_offset(const net_view& v, const flight_state
   oz = min_image((double)leg.z - (double)f.z, v.half_per[2]) * q;
 }
 
-// One exciton through its hop budget (event-driven form of particle::step,
-// src/monte_carlo/particle.cpp:57-80; FLY adds the drift of particle::fly for v > 0).  v holds everything of the exciton's network;
-// it is uniform across the wave, so its fields live in scalar registers.
-// Returns whether a further launch could move the exciton (t <= t_max, a dwell pending).
-template <bool COUNT, bool SAMPLE, bool TRACE, bool FLY = false>
-__device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint64_t hop_budget,
-                                            double t_max, const trace_view& tv) {
-#pragma clang fp contract(off)
-  double t = v.x.t_next[e];
-  double tl = FLY ? v.x.t_last[e] : 0.0;
-  double so = FLY ? v.x.s_off[e] : 0.0;
-  uint32_t hd = FLY ? (uint32_t)v.x.heading[e] : 0u;
-  uint64_t h = v.x.hops[e];
-  double dx = v.x.dx[e], dy = v.x.dy[e], dz = v.x.dz[e];
-  uint32_t nd = v.x.drains[e];
-  uint64_t hs = v.x.hash[e];
-  uint32_t k = SAMPLE ? v.x.k_rec[e] : 0u;
-  int64_t tr = 0;
-  if (TRACE && e < tv.n_trace) tr = tv.tr_n[e];
-  const uint32_t R0 = (uint32_t)v.roff[v.x.site[e]];
-  uint32_t R = row_word(R0, v.blocks[(size_t)ROW_UNITS * R0].x);
-  row_regs row = load_row(v.blocks, R);
-  fly_leg leg{};
-  if (FLY) leg = load_leg(v, row.site, hd);
-  const uint64_t h_end = h + hop_budget;
-  const size_t E = v.x.n;
-  count_cache cc;
-  hop_words hw;
-  uint32_t* cbase = COUNT ? v.site_count + (size_t)xcd_id() * v.count_stride : nullptr;
-
-  while (true) {
-    if (SAMPLE) {
-      while (k < (uint32_t)v.n_bins) {
-        const double tk = (double)(k + 1u) * v.dt_sample;
-        if (!(tk < t)) break;
-        const size_t r = (size_t)(k - (uint32_t)v.bin0) * E + e;
-        if (FLY) {  // the flight from the last event up to tk
-          flight_state g{R, row.site, row.x, row.y, row.z, so, hd, dx, dy, dz, nd, hs};
-          fly_leg gl = leg;
-          if (!fly(v, g, gl, tk - tl, e, h)) {
-            atomicOr(v.fly_err, 1);
-            break;
-          }
-          double ox, oy, oz;
-          fly_offset(v, g, gl, ox, oy, oz);
-          v.rec_dx[r] = g.dx + ox;
-          v.rec_dy[r] = g.dy + oy;
-          v.rec_dz[r] = g.dz + oz;
-          v.rec_drain[r] = g.nd;
-        } else {
-          v.rec_dx[r] = dx;
-          v.rec_dy[r] = dy;
-          v.rec_dz[r] = dz;
-          v.rec_drain[r] = nd;
-        }
-        ++k;
-      }
-    }
-    if (FLY) {
-      if (h >= h_end || !(t <= t_max) || !(t < INFINITY)) break;
-      // fly through the dwell, then hop from the site reached (particle.cpp:62-75)
-      flight_state g{R, row.site, row.x, row.y, row.z, so, hd, dx, dy, dz, nd, hs};
-      if (!fly(v, g, leg, t - tl, e, h)) {
-        atomicOr(v.fly_err, 1);
-        break;
-      }
-      if (g.R != R) {
-        R = g.R;
-        row = load_row(v.blocks, R);
-      }
-      so = g.s;
-      hd = g.heading;
-      dx = g.dx;
-      dy = g.dy;
-      dz = g.dz;
-      nd = g.nd;
-      hs = g.hs;
-      if (trapped(row.n, row.gamma)) {
-        // no rates here: the event leaves the exciton in place (scatterer.cpp:14-15) and no
-        // dwell ends again; it counts as a hop so that later flights draw on fresh counters
-        tl = t;
-        t = INFINITY;
-        ++h;
-        hw.have = false;
-        continue;
-      }
-    } else if (h >= h_end || trapped(row.n, row.gamma) || !(t <= t_max)) {
-      break;
-    }
-
-    // event selection (scatterer::update_state, scatterer.cpp:17-30)
-    uint32_t w_sel, w_dw;
-    hw.get(v.seed, e, h, w_sel, w_dw);
-    const double dice = div_rand_max(row.gamma * (double)r31(w_sel));
-    const uint32_t idx = select_entry(v.blocks, R, row.c, row.n, dice);
-    const uint32_t tg = target_of(v.blocks, R, row, idx);
-    if (COUNT) cc.add(count_slot(R & TGT_LINE_MASK, v.count_stride), cbase);
-    const float sx = row.x, sy = row.y, sz = row.z;
-    const double t_hop = t;
-
-    // dwell at the new site (particle.cpp:183 -> ff_time)
-    R = tg & ~EDGE_DRAIN_BIT;
-    row = load_row(v.blocks, R);
-    dx = dx + min_image((double)row.x - (double)sx, v.half_per[0]);
-    dy = dy + min_image((double)row.y - (double)sy, v.half_per[1]);
-    dz = dz + min_image((double)row.z - (double)sz, v.half_per[2]);
-    hs = (hs ^ (uint64_t)row.site) * FNV_PRIME;
-    // the flight's first leg, in flight while the dwell is drawn
-    if (FLY) leg = load_leg(v, row.site, hd);
-    const uint32_t r = nonzero_draw1(w_dw, v.seed, e, h, STREAM_HOP_REDRAW);
-    t = t + dwell_time(row.n, row.gamma, r);
-    // drain: count current and re-inject, keeping displacement and dwell (kubo_step,
-    // src/monte_carlo/monte_carlo.cpp:330-336)
-    if (tg & EDGE_DRAIN_BIT) {
-      ++nd;
-      R = v.src_roff[r31(draw4(v.seed, e, h, STREAM_REINJECT).v[0]) % v.n_src];
-      row = load_row(v.blocks, R);
-      hs = (hs ^ ((uint64_t)row.site | (1ull << 32))) * FNV_PRIME;
-      if (FLY) leg = load_leg(v, row.site, hd);
-    }
-    if (FLY) {
-      so = 0.0;
-      tl = t_hop;
-    }
-    if (TRACE && e < tv.n_trace && tr < tv.tr_max) {
-      tv.tr_site[(size_t)e * tv.tr_max + tr] = (int32_t)row.site;
-      tv.tr_time[(size_t)e * tv.tr_max + tr] = t_hop;
-      ++tr;
-    }
-    ++h;
-  }
-  if (COUNT) cc.flush(cbase);
-
-  v.x.site[e] = (int32_t)row.site;
-  v.x.t_next[e] = t;
-  v.x.hops[e] = h;
-  v.x.dx[e] = dx;
-  v.x.dy[e] = dy;
-  v.x.dz[e] = dz;
-  v.x.drains[e] = nd;
-  v.x.hash[e] = hs;
-  if (SAMPLE) v.x.k_rec[e] = k;
-  if (TRACE && e < tv.n_trace) tv.tr_n[e] = tr;
-  if (FLY) {
-    v.x.s_off[e] = so;
-    v.x.t_last[e] = tl;
-    v.x.heading[e] = (uint8_t)hd;
-    return t <= t_max && t < INFINITY;
-  }
-  return !trapped(row.n, row.gamma) && t <= t_max;
-}
 
 // The hop loop of one wave (v = 0), built around the cooperative row load: every lane takes part
 // in every row load, so the loop runs until no lane of the wave can hop; a lane without an
@@ -1084,7 +941,7 @@ __device__ __forceinline__ bool hop_exciton(const net_view& v, uint32_t e, uint6
 //       MSD records fall due, and
 //   (C) the hop selected in (A) happens if the exciton's clock allows it (t <= t_max), else the
 //       exciton stops at this site and the issued load is simply not used.
-// Every exciton's arithmetic and its order are those of hop_exciton (and of the oracle); only
+// Every exciton's arithmetic and its order are those of the oracle; only
 // the selection is computed before the clock test that decides whether it is used.  A drain
 // target's header and position are gathered by the lanes concerned.
 // COUNT: departures from the block lines [win_base, win_base + COUNT_WINDOW_LINES) are counted
@@ -1281,6 +1138,300 @@ __device__ __forceinline__ void hop_wave(const net_view& v, uint32_t e, bool val
   v.x.hash[e] = hs;
   if (SAMPLE) v.x.k_rec[e] = k;
   if (TRACE && e < tv.n_trace) tv.tr_n[e] = tr;
+}
+
+// The hops of one wave's excitons (event-driven form of particle::step,
+// src/monte_carlo/particle.cpp:57-80) with drift along the tubes for v > 0, built like hop_wave.
+// Below ~100,000 excitons the chain of one iteration bounds the kernel (~330 vector and ~210 scalar
+// instructions), above it their issue; so the next row's load goes out before the dwell, the records
+// and the flight are computed: on a guess whether the flight ends on its leg (the dwell in single
+// precision), or exactly when the flight's time is known already.  The guess decides only which row
+// is loaded; where it is wrong the lane spends an iteration on loading the right one.  An iteration
+// takes a lane one site on, by a hop or along the tube, so lanes in a long flight hold back no others.
+// `c` is the view's copy in LDS, for what few iterations need: as kernel arguments those pointers
+// would hold scalar registers throughout (~100 were spilled to lanes of vector registers).
+// 1,000 hops on 50,051 sites at 2e5 m/s, with counts and records / without, in ms: 100,003 excitons
+// 3.27 / 2.49, 1 M 22.7 / 13.3; a lane with its own gathers through flight and hop 3.65 / 2.96 and
+// 27.5 / 18.9.  Three waves per SIMD instead of two spill 45 registers with counts and records:
+// 4.93 and 32.9.
+template <bool COUNT, bool SAMPLE, bool TRACE>
+__device__ __forceinline__ void hop_wave_fly(const net_view& v, uint32_t e, bool valid,
+                                             uint64_t hop_budget, double t_max,
+                                             const trace_view& tv, uint4* lds_wave, uint32_t lane,
+                                             uint32_t* win, uint32_t win_base, const net_view& c) {
+#pragma clang fp contract(off)
+  double t = INFINITY, tl = 0.0, so = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
+  uint64_t h = 0, hs = 0;
+  uint32_t hd = 0, nd = 0, k = 0, W = 0;
+  int64_t tr = 0;
+  if (valid) {
+    t = c.x.t_next[e];
+    tl = c.x.t_last[e];
+    so = c.x.s_off[e];
+    hd = (uint32_t)c.x.heading[e];
+    h = c.x.hops[e];
+    dx = c.x.dx[e];
+    dy = c.x.dy[e];
+    dz = c.x.dz[e];
+    nd = c.x.drains[e];
+    hs = c.x.hash[e];
+    if (SAMPLE) k = c.x.k_rec[e];
+    if (TRACE && e < tv.n_trace) tr = tv.tr_n[e];
+    const uint32_t R0 = (uint32_t)c.roff[c.x.site[e]];
+    W = row_word(R0, v.blocks[(size_t)ROW_UNITS * R0].x);
+  }
+  const uint64_t h_end = h + hop_budget;
+  double t_rec = INFINITY;
+  if (SAMPLE && k < (uint32_t)v.n_bins) t_rec = (double)(k + 1u) * v.dt_sample;
+  bool active = valid;
+  uint32_t site_now = 0;       // when stopped: the site it stopped at
+  bool pend = false;           // a hop into this site is to be finished
+  uint32_t r_dw = 0;           // its dwell draw
+  float px = 0.f, py = 0.f, pz = 0.f;  // position of the site it left
+  bool flown = false;          // on a flight whose remaining time is tau
+  bool reload = false;         // the row on its way is not the lane's: W is to be loaded
+  double tau = 0.0;
+  uint32_t passes = 0, fly_drains = 0;  // sites and drains passed on the flight
+  // the state before the flight, restored when it exceeds the pass bound
+  double so0 = 0.0, dx0 = 0.0, dy0 = 0.0, dz0 = 0.0;
+  uint64_t hs0 = 0;
+  uint32_t hd0 = 0, nd0 = 0, site0 = 0;
+  hop_words hw;
+  count_cache cc;
+  uint32_t* cbase = COUNT ? v.site_count + (size_t)xcd_id() * v.count_stride : nullptr;
+  uint32_t count_line = COUNT_NONE;  // counted at the top of the next iteration, as in hop_wave
+  auto count_departure = [&]() {
+    const uint32_t off = count_line - win_base;
+    if (off < COUNT_WINDOW_LINES) window_count(win, off, count_line, cbase, v.count_stride);
+    else cc.add(count_slot(count_line, v.count_stride), cbase);
+    count_line = COUNT_NONE;
+  };
+
+  coop_issue(v.blocks, W, lds_wave, lane);
+  // the next leg as loaded: unpacked only after the row has arrived, or the wave would wait for it
+  // where it is issued
+  const uint4* at = leg_of(v, W, hd);
+  uint4 leg_p = at[0], leg_q = at[1];
+  while (true) {
+    const coop_row row = coop_finish(lds_wave, lane);
+    const fly_leg leg = leg_from_units(leg_p, leg_q);
+    if (COUNT && count_line != COUNT_NONE) count_departure();
+    // (A) where the lane goes next, guessed, and the load of that row: the hop from this site if
+    // the flight through the dwell is taken to end on its leg, else the leg's site
+    const bool on = active && !reload;
+    const bool linked = leg.word != LINK_NONE;  // particle.cpp:11-12
+    double need = 0.0;
+    bool stay = true;
+    if (on && linked) {
+      need = (leg.len - so) / v.velocity;
+      if (flown) {
+        stay = !(need < tau);
+      } else {
+        // the dwell in single precision: a wrong guess costs an iteration, nothing else
+        const float guess = pend ? -__log2f((float)r_dw * 0x1p-31f) * 0.6931472f / (float)row.gamma
+                                 : (float)(t - tl);
+        stay = !((float)need < guess);
+      }
+    }
+    uint32_t tg = 0, r_next = 0, W_next = W;
+    const bool can = on && stay && h < h_end && !trapped(row.n, row.gamma);
+    if (can) {
+      // event selection (scatterer::update_state, scatterer.cpp:17-30)
+      uint32_t w_sel, w_dw;
+      hw.get(v.seed, e, h, w_sel, w_dw);
+      const double dice = div_rand_max(row.gamma * (double)r31(w_sel));
+      const uint32_t idx = select_entry(v.blocks, W, row.c, row.n, dice);
+      tg = idx < ROW_INLINE ? target_lds(lds_wave, lane, idx) : target_wide(v.blocks, W, row.n, idx);
+      r_next = nonzero_draw1(w_dw, v.seed, e, h, STREAM_HOP_REDRAW);
+      W_next = tg & ~EDGE_DRAIN_BIT;
+      if (tg & EDGE_DRAIN_BIT) {
+        W_next = c.src_roff[r31(draw4(v.seed, e, h, STREAM_REINJECT).v[0]) % c.n_src];
+      }
+    } else if (on && !stay) {
+      W_next = leg.word & ~EDGE_DRAIN_BIT;
+      if (leg.word & EDGE_DRAIN_BIT) {
+        W_next = c.src_roff[r31(draw4(v.seed, e, h, STREAM_FLY_DRAIN + fly_drains).v[0]) % c.n_src];
+      }
+    }
+    const uint32_t hd_next = on && linked ? leg.heading : hd;
+    // a lane whose exciton has stopped loads block line 0, which every such lane shares
+    coop_issue(v.blocks, active ? W_next : 0u, lds_wave, lane);
+    at = leg_of(v, active ? W_next : 0u, hd_next);
+    leg_p = at[0];
+    leg_q = at[1];
+    reload = false;
+    // (B) the hop into this site finishes: dwell at the new site (particle.cpp:183 -> ff_time)
+    if (pend && on) {
+      dx = dx + min_image((double)row.x - (double)px, v.half_per[0]);
+      dy = dy + min_image((double)row.y - (double)py, v.half_per[1]);
+      dz = dz + min_image((double)row.z - (double)pz, v.half_per[2]);
+      hs = (hs ^ (uint64_t)row.site) * FNV_PRIME;
+      if (TRACE && e < tv.n_trace && tr < tv.tr_max) {
+        tv.tr_site[(size_t)e * tv.tr_max + tr] = (int32_t)row.site;
+        tv.tr_time[(size_t)e * tv.tr_max + tr] = t;
+        ++tr;
+      }
+      t = t + dwell_time(row.n, row.gamma, r_dw);
+      pend = false;
+    }
+    if (on && !flown) {
+      if (SAMPLE) {
+        while (t_rec < t) {  // the flight from the last event up to t_rec
+          const double tau_r = t_rec - tl;
+          double gx = dx, gy = dy, gz = dz;
+          uint32_t gd = nd;
+          if (!linked || !(need < tau_r)) {
+            const double s_r = linked ? so + v.velocity * tau_r : so;
+            if (s_r != 0.0) {
+              const double q = s_r / leg.len;
+              gx = dx + min_image((double)leg.x - (double)row.x, v.half_per[0]) * q;
+              gy = dy + min_image((double)leg.y - (double)row.y, v.half_per[1]) * q;
+              gz = dz + min_image((double)leg.z - (double)row.z, v.half_per[2]) * q;
+            }
+          } else {
+            flight_state g{W, row.site, row.x, row.y, row.z, so, hd, dx, dy, dz, nd, hs};
+            fly_leg gl = leg;
+            net_view fv = v;
+            fv.src_roff = c.src_roff;
+            fv.n_src = c.n_src;
+            if (!fly(fv, g, gl, tau_r, e, h)) {
+              atomicOr(c.fly_err, 1);
+              break;
+            }
+            double ox, oy, oz;
+            fly_offset(c, g, gl, ox, oy, oz);
+            gx = g.dx + ox;
+            gy = g.dy + oy;
+            gz = g.dz + oz;
+            gd = g.nd;
+          }
+          const size_t r = (size_t)(k - (uint32_t)c.bin0) * c.x.n + e;
+          c.rec_dx[r] = gx;
+          c.rec_dy[r] = gy;
+          c.rec_dz[r] = gz;
+          c.rec_drain[r] = gd;
+          ++k;
+          t_rec = k < (uint32_t)c.n_bins ? (double)(k + 1u) * c.dt_sample : INFINITY;
+        }
+      }
+      if (h >= h_end || !(t <= t_max) || !(t < INFINITY)) {
+        active = false;
+        site_now = row.site;
+      } else {
+        // fly through the dwell, then hop from the site reached (particle.cpp:62-75)
+        tau = t - tl;
+        so0 = so;
+        dx0 = dx;
+        dy0 = dy;
+        dz0 = dz;
+        hs0 = hs;
+        hd0 = hd;
+        nd0 = nd;
+        site0 = row.site;
+      }
+    }
+    // (C) what (A) guessed, if it holds; otherwise the row again, with the flight's time known
+    if (on && active) {
+      if (linked && passes == FLY_MAX_PASSES) {
+        atomicOr(c.fly_err, 1);
+        so = so0;
+        dx = dx0;
+        dy = dy0;
+        dz = dz0;
+        hs = hs0;
+        hd = hd0;
+        nd = nd0;
+        site_now = site0;
+        active = false;
+      } else if (linked && stay == (need < tau)) {
+        flown = reload = true;
+      } else if (!stay) {  // passes the leg's site
+        tau = tau - need;
+        dx = dx + min_image((double)leg.x - (double)row.x, v.half_per[0]);
+        dy = dy + min_image((double)leg.y - (double)row.y, v.half_per[1]);
+        dz = dz + min_image((double)leg.z - (double)row.z, v.half_per[2]);
+        so = 0.0;
+        hs = (hs ^ ((uint64_t)leg.site | (2ull << 32))) * FNV_PRIME;
+        if (leg.word & EDGE_DRAIN_BIT) {
+          ++nd;
+          ++fly_drains;
+          const uint32_t src_site = v.blocks[(size_t)ROW_UNITS * (W_next & TGT_LINE_MASK)].y;
+          hs = (hs ^ ((uint64_t)src_site | (1ull << 32))) * FNV_PRIME;
+        }
+        ++passes;
+        flown = true;
+        hd = hd_next;
+        W = W_next;
+      } else {  // ends on this segment (particle.cpp:46-49)
+        if (linked) so = so + v.velocity * tau;
+        hd = hd_next;
+        flown = false;
+        passes = fly_drains = 0u;
+        if (!can) {
+          // no rates here: the event leaves the exciton in place (scatterer.cpp:14-15) and no dwell
+          // ends again; it counts as a hop so that later flights draw on fresh counters
+          tl = t;
+          t = INFINITY;
+          ++h;
+          hw.have = false;
+        } else {
+          if (COUNT) count_line = W & TGT_LINE_MASK;
+          so = 0.0;
+          tl = t;
+          if (tg & EDGE_DRAIN_BIT) {
+            // drain: the dwell drawn at the drain site, then re-injection keeping displacement and
+            // dwell (kubo_step, src/monte_carlo/monte_carlo.cpp:330-336)
+            const uint4* bd = v.blocks + (size_t)ROW_UNITS * (tg & TGT_LINE_MASK);
+            const uint4 hdr = bd[0], pd = bd[7];
+            dx = dx + min_image((double)__uint_as_float(pd.x) - (double)row.x, v.half_per[0]);
+            dy = dy + min_image((double)__uint_as_float(pd.y) - (double)row.y, v.half_per[1]);
+            dz = dz + min_image((double)__uint_as_float(pd.z) - (double)row.z, v.half_per[2]);
+            hs = (hs ^ (uint64_t)hdr.y) * FNV_PRIME;
+            ++nd;
+            const uint32_t src_site = v.blocks[(size_t)ROW_UNITS * (W_next & TGT_LINE_MASK)].y;
+            hs = (hs ^ ((uint64_t)src_site | (1ull << 32))) * FNV_PRIME;
+            if (TRACE && e < tv.n_trace && tr < tv.tr_max) {
+              tv.tr_site[(size_t)e * tv.tr_max + tr] = (int32_t)src_site;
+              tv.tr_time[(size_t)e * tv.tr_max + tr] = t;
+              ++tr;
+            }
+            t = t + dwell_time(hdr.x, __hiloint2double((int)hdr.w, (int)hdr.z), r_next);
+          } else {
+            pend = true;
+            r_dw = r_next;
+            px = row.x;
+            py = row.y;
+            pz = row.z;
+          }
+          ++h;
+          W = W_next;
+        }
+      }
+    }
+    if (__ballot(active) == 0) break;
+  }
+  // the last issued load lands in this wave's LDS rows: wait for it before the wave moves on
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (COUNT && count_line != COUNT_NONE) count_departure();
+  if (COUNT) cc.flush(cbase);
+  if (uint32_t* live = c.live) {
+    const uint64_t b = __ballot(valid && t <= t_max && t < INFINITY);
+    if (lane == 0u && b != 0ull) atomicAdd(live, (uint32_t)__popcll(b));
+  }
+  if (!valid) return;
+  c.x.site[e] = (int32_t)site_now;
+  c.x.t_next[e] = t;
+  c.x.hops[e] = h;
+  c.x.dx[e] = dx;
+  c.x.dy[e] = dy;
+  c.x.dz[e] = dz;
+  c.x.drains[e] = nd;
+  c.x.hash[e] = hs;
+  if (SAMPLE) c.x.k_rec[e] = k;
+  if (TRACE && e < tv.n_trace) tv.tr_n[e] = tr;
+  c.x.s_off[e] = so;
+  c.x.t_last[e] = tl;
+  c.x.heading[e] = (uint8_t)hd;
 }
 
 // Position of this thread in the sorted exciton order.  Workgroups are dealt to the XCDs in turn,
@@ -1714,16 +1865,33 @@ __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
 
 // The same with drift along the tubes (v > 0).
 template <bool COUNT, bool SAMPLE, bool TRACE>
-__global__ __launch_bounds__(256) void k_hop_fly(hop_args a) {
-  const uint32_t pos = xcd_position();
-  bool live = false;
-  if (pos < a.v.x.n) {
-    const uint32_t e = a.perm ? a.perm[pos] : pos;
-    live = hop_exciton<COUNT, SAMPLE, TRACE, true>(a.v, e, a.hop_budget, a.t_max, a.tv);
+__global__ __launch_bounds__(256, 2) void k_hop_fly(hop_args a) {
+  __shared__ uint4 rows[4 * 64 * ROW_UNITS];  // 8 KB of staged rows per wave
+  __shared__ uint32_t win[COUNT_WINDOW_WORDS]; // 8 KB: the workgroup's departure-count window
+  const uint32_t pos = xcd_position(), lane = threadIdx.x & 63u, n = (uint32_t)a.v.x.n;
+  const bool valid = pos < n;
+  const bool wave_live = __builtin_amdgcn_readfirstlane(pos - lane) < n;
+  const uint32_t e = valid ? (a.perm ? a.perm[pos] : pos) : 0u;
+  uint4* lds_wave = rows + 64u * ROW_UNITS * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ net_view cold;
+  if (threadIdx.x == 0) cold = a.v;
+  uint32_t base = 0u;
+  if constexpr (COUNT) {
+    for (uint32_t i = threadIdx.x; i < COUNT_WINDOW_WORDS; i += blockDim.x) win[i] = 0u;
+    const uint32_t p0 = pos - threadIdx.x;
+    if (p0 < n) {
+      const uint32_t L0 = (uint32_t)a.v.roff[a.v.x.site[a.perm ? a.perm[p0] : p0]];
+      base = L0 > COUNT_WINDOW_LINES / 2 ? L0 - COUNT_WINDOW_LINES / 2 : 0u;
+    }
   }
-  if (a.v.live) {
-    const uint64_t b = __ballot(live);
-    if ((threadIdx.x & 63u) == 0u && b != 0ull) atomicAdd(a.v.live, (uint32_t)__popcll(b));
+  __syncthreads();
+  if (wave_live)
+    hop_wave_fly<COUNT, SAMPLE, TRACE>(a.v, e, valid, a.hop_budget, a.t_max, a.tv, lds_wave, lane, win,
+                                       base, cold);
+  if constexpr (COUNT) {
+    __syncthreads();
+    window_flush(win, base, a.v.site_count + (size_t)xcd_id() * a.v.count_stride,
+                 a.v.count_stride);
   }
 }
 
@@ -2001,7 +2169,7 @@ __global__ __launch_bounds__(256) void k_contact_fly(contact_args a) {
     double tl = a.s.t_last[e];
     flight_state g{R, row.site, row.x, row.y, row.z, a.s.s_off[e], (uint32_t)a.s.heading[e],
                    0.0, 0.0, 0.0, 0u, 0ull};
-    fly_leg leg = load_leg(a.fv, g.site, g.heading);
+    fly_leg leg = load_leg(a.fv, R, g.heading);
     uint64_t made = 0;
     hop_words hw;
     while (t <= a.t_end) {
@@ -2032,7 +2200,7 @@ __global__ __launch_bounds__(256) void k_contact_fly(contact_args a) {
       row = load_row(a.blocks, R);
       const uint32_t r = nonzero_draw1(w_dw, a.seed, id, h, STREAM_HOP_REDRAW);
       g = flight_state{R, row.site, row.x, row.y, row.z, 0.0, g.heading, 0.0, 0.0, 0.0, 0u, 0ull};
-      leg = load_leg(a.fv, g.site, g.heading);  // in flight while the dwell is drawn
+      leg = load_leg(a.fv, R, g.heading);  // in flight while the dwell is drawn
       tl = t;
       t = t + dwell_time(row.n, row.gamma, r);
       ++h;
