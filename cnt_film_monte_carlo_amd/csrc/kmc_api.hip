@@ -458,20 +458,6 @@ int pack_rows(kmc_ctx* c, const char* who = nullptr) {
   return KMC_OK;
 }
 
-// The legs of flights along the tubes: made when particles that drift are first placed on the rows.
-int fly_table(kmc_ctx* c) {
-  if (c->fly_ok) return KMC_OK;
-  double half[3];
-  for (int k = 0; k < 3; ++k)
-    half[k] = (c->cfg.periodic_mask & (1 << k)) ? 0.5 * c->cfg.period_len[k] : INFINITY;
-  KMC_TRY(dalloc(c, c->d_fly_table, 4 * (size_t)(c->n_units / ROW_UNITS)));
-  KMC_HIP(c, launch_fly_table(c->n_sites, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p,
-                              c->d_hdr.p, c->d_pos[0].p, c->d_pos[1].p, c->d_pos[2].p, half,
-                              c->d_fly_table.p, c->stream));
-  c->fly_ok = true;
-  return KMC_OK;
-}
-
 // Every same-tube link must have a nonzero length in the FP32 positions a flight uses (a flight
 // over a zero-length segment would pass sites without using time).
 int check_links(kmc_ctx* c, const char* what) {
@@ -496,6 +482,26 @@ int check_links(kmc_ctx* c, const char* what) {
                                              " coincide");
     }
   }
+  return KMC_OK;
+}
+
+// The legs of flights along the tubes, made when particles that drift are first placed on a film's
+// rows.  The kernel that measures every link also finds those check_links refuses (a loop over the
+// sites here took 0.5 ms per 50,000 of them, at every injection).
+int fly_table(kmc_ctx* c, const char* what) {
+  if (c->fly_ok) return KMC_OK;
+  double half[3];
+  for (int k = 0; k < 3; ++k)
+    half[k] = (c->cfg.periodic_mask & (1 << k)) ? 0.5 * c->cfg.period_len[k] : INFINITY;
+  KMC_TRY(dalloc(c, c->d_fly_table, 4 * (size_t)(c->n_units / ROW_UNITS)));
+  KMC_HIP(c, hipMemsetAsync(c->d_fly_err.p, 0, sizeof(int32_t), c->stream));
+  KMC_HIP(c, launch_fly_table(c->n_sites, c->d_left.p, c->d_right.p, c->d_flags.p, c->d_roff.p,
+                              c->d_hdr.p, c->d_pos[0].p, c->d_pos[1].p, c->d_pos[2].p, half,
+                              c->d_fly_table.p, c->d_fly_err.p, c->stream));
+  int32_t bad = 0;
+  KMC_TRY(copy_out(c, &bad, c->d_fly_err.p, sizeof(int32_t)));
+  if (bad) KMC_TRY(check_links(c, what));  // names the sites
+  c->fly_ok = true;
   return KMC_OK;
 }
 
@@ -1132,10 +1138,7 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   c->n_exc = E;
   c->n_bins = c->bin0 = c->win_bins = 0;
   c->n_trace = 0;
-  if (c->velocity > 0.0) {
-    KMC_TRY(check_links(c, "kmc_inject"));
-    KMC_TRY(fly_table(c));
-  }
+  if (c->velocity > 0.0) KMC_TRY(fly_table(c, "kmc_inject"));
   c->exc_velocity = c->velocity;
   KMC_HIP(c, launch_inject(excitons_of(c), c->d_blocks.p, c->d_src_roff.p,
                            (uint32_t)c->h_src.size(), c->cfg.seed, c->stream));
@@ -2055,7 +2058,7 @@ int kmc_contact_init(kmc_ctx* c, int32_t n_seg, int64_t c1_pop, int64_t c2_pop, 
     return fail(c, KMC_ERR_ARG, "kmc_contact_init: need populations >= 0, 0 < capacity < 2^31");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   if (c->velocity > 0.0) {
-    KMC_TRY(check_links(c, who));
+    KMC_TRY(fly_table(c, who));
     for (uint8_t f : c->h_flags)
       if (f & KMC_SITE_DRAIN)
         return fail(c, KMC_ERR_STATE, "kmc_contact_init: with velocity > 0 a flight would "
@@ -2194,7 +2197,7 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
     return fail(c, KMC_ERR_STATE, "kmc_contact_run: CSR not complete");
   if (n_steps == 0) return KMC_OK;
   KMC_HIP(c, hipSetDevice(c->cfg.device));
-  if (c->c_vel > 0.0) KMC_TRY(fly_table(c));
+  if (c->c_vel > 0.0) KMC_TRY(fly_table(c, who));
   const int64_t S = c->c_nseg;
   KMC_TRY(dalloc(c, c->c_pop_out, (size_t)n_steps * S));
   KMC_TRY(dalloc(c, c->c_cur_out, (size_t)n_steps * (S - 1)));

@@ -253,11 +253,11 @@ bool hop_rows_pays(int64_t movable, int n_cu);
 hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
                            bool sample, bool trace, hipStream_t st);
 // table[2 (2 roff[i] + heading)], [.. + 1]: the leg of a flight at site i (scatterer::left/right,
-// scatterer.h:29-30; half_per as in net_view)
+// scatterer.h:29-30; half_per as in net_view); *bad is set where a link has no length
 hipError_t launch_fly_table(int64_t n, const int32_t* left, const int32_t* right,
                             const uint8_t* flags, const int64_t* roff, const site_hdr* hdr,
                             const double* px, const double* py, const double* pz,
-                            const double* half_per, uint4* table, hipStream_t st);
+                            const double* half_per, uint4* table, int32_t* bad, hipStream_t st);
 hipError_t launch_hop_ens(const ens_args& a, bool count, bool sample, hipStream_t st);
 hipError_t launch_ens_keys(int64_t n, const net_view* nets, const uint16_t* exc_net,
                            const int64_t* ebase, uint64_t* keys, uint32_t* ids, uint32_t* live,

@@ -844,7 +844,8 @@ __global__ __launch_bounds__(256) void k_fly_table(int64_t n, const int32_t* __r
                                                    const double* __restrict__ px,
                                                    const double* __restrict__ py,
                                                    const double* __restrict__ pz, double hx, double hy,
-                                                   double hz, uint4* __restrict__ table) {
+                                                   double hz, uint4* __restrict__ table,
+                                                   int32_t* __restrict__ bad) {
 #pragma clang fp contract(off)
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= 2 * n) return;
@@ -859,6 +860,7 @@ __global__ __launch_bounds__(256) void k_fly_table(int64_t n, const int32_t* __r
     const double sy = min_image((double)y - (double)(float)py[i], hy);
     const double sz = min_image((double)z - (double)(float)pz[i], hz);
     const double len = norm3(sx, sy, sz);
+    if (!(len > 0.0)) *bad = 1;  // a flight would pass sites without using time
     a = make_uint4(row_word((uint32_t)roff[nx], hdr[nx].n) | ((flags[nx] & 2u) ? EDGE_DRAIN_BIT : 0u),
                    (uint32_t)nx | (nx == r ? FLY_HEADING_BIT : 0u), (uint32_t)__double2loint(len),
                    (uint32_t)__double2hiint(len));
@@ -2780,10 +2782,10 @@ hipError_t launch_mask_count(int64_t nnz, const uint8_t* cls, const uint8_t* mas
 hipError_t launch_fly_table(int64_t n, const int32_t* left, const int32_t* right,
                             const uint8_t* flags, const int64_t* roff, const site_hdr* hdr,
                             const double* px, const double* py, const double* pz,
-                            const double* half_per, uint4* table, hipStream_t st) {
+                            const double* half_per, uint4* table, int32_t* bad, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_fly_table, grid_for(2 * n), dim3(256), 0, st, n, left, right, flags, roff, hdr,
-                     px, py, pz, half_per[0], half_per[1], half_per[2], table);
+                     px, py, pz, half_per[0], half_per[1], half_per[2], table, bad);
   return hipGetLastError();
 }
 
