@@ -2064,7 +2064,9 @@ __global__ __launch_bounds__(256) void k_fold_counts(int64_t n_lines, int64_t st
 
 // =============================================================================================
 // (d) MSD / current reduction: block (k, b) reduces bin k over exciton batch b in a fixed
-//     order (per-thread strided sums, wavefront shuffle tree, LDS across waves).
+//     order (per-thread strided sums, wavefront shuffle tree, LDS across waves).  Bound by memory,
+//     with a workgroup per bin and batch: each thread has the records of REDUCE_AHEAD excitons in
+//     flight (16 M excitons, 8 bins, 32 batches: 0.62 ms, 2.36 with one).
 // =============================================================================================
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -2072,21 +2074,37 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+constexpr int REDUCE_AHEAD = 8;
+
 __global__ __launch_bounds__(256) void k_reduce_samples(reduce_args a) {
   __shared__ double lds[5][4];
   const int k = blockIdx.x, b = blockIdx.y;
   const int64_t E = a.n_exc;
   const int64_t e0 = (int64_t)b * E / a.n_batches, e1 = (int64_t)(b + 1) * E / a.n_batches;
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-    if ((uint32_t)(a.bin0 + k) < a.k_rec[e]) {
+  const uint32_t bin = (uint32_t)(a.bin0 + k);
+  for (int64_t base = e0 + threadIdx.x; base < e1; base += REDUCE_AHEAD * blockDim.x) {
+    double x[REDUCE_AHEAD], y[REDUCE_AHEAD], z[REDUCE_AHEAD];
+    uint32_t n[REDUCE_AHEAD], nd[REDUCE_AHEAD];
+#pragma unroll
+    for (int i = 0; i < REDUCE_AHEAD; ++i) {
+      const int64_t e = base + i * blockDim.x < e1 ? base + i * blockDim.x : base;
       const size_t r = (size_t)k * E + e;
-      const double x = a.rec_dx[r], y = a.rec_dy[r], z = a.rec_dz[r];
-      acc[0] += 1.0;
-      acc[1] += x * x;
-      acc[2] += y * y;
-      acc[3] += z * z;
-      acc[4] += (double)a.rec_drain[r];
+      n[i] = a.k_rec[e];
+      x[i] = a.rec_dx[r];
+      y[i] = a.rec_dy[r];
+      z[i] = a.rec_dz[r];
+      nd[i] = a.rec_drain[r];
+    }
+#pragma unroll
+    for (int i = 0; i < REDUCE_AHEAD; ++i) {
+      if (base + i * blockDim.x < e1 && bin < n[i]) {
+        acc[0] += 1.0;
+        acc[1] += x[i] * x[i];
+        acc[2] += y[i] * y[i];
+        acc[3] += z[i] * z[i];
+        acc[4] += (double)nd[i];
+      }
     }
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
