@@ -307,12 +307,14 @@ static inline int32_t window_bins(const kmc_ctx* c) {
 }
 
 // Zeroes the first nrec records (a window's worth).
-static int clear_records(kmc_ctx* c, size_t nrec) {
-  if (nrec == 0) return KMC_OK;
-  KMC_HIP(c, hipMemsetAsync(c->r_dx.p, 0, nrec * sizeof(double), c->stream));
-  KMC_HIP(c, hipMemsetAsync(c->r_dy.p, 0, nrec * sizeof(double), c->stream));
-  KMC_HIP(c, hipMemsetAsync(c->r_dz.p, 0, nrec * sizeof(double), c->stream));
-  KMC_HIP(c, hipMemsetAsync(c->r_drain.p, 0, nrec * sizeof(uint32_t), c->stream));
+static int clear_records(kmc_ctx* c, size_t nrec, bool k_rec) {
+  clear_args a;
+  if (k_rec) a.add(c->x_krec.p, c->n_exc * sizeof(uint32_t));
+  a.add(c->r_dx.p, nrec * sizeof(double));
+  a.add(c->r_dy.p, nrec * sizeof(double));
+  a.add(c->r_dz.p, nrec * sizeof(double));
+  a.add(c->r_drain.p, nrec * sizeof(uint32_t));
+  KMC_HIP(c, launch_clear(a, c->stream));
   return KMC_OK;
 }
 
@@ -1127,13 +1129,14 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   const int64_t n_lines = c->n_units / ROW_UNITS;  // counters per block line
   c->count_stride = (n_lines + COUNT_ALIGN - 1) / COUNT_ALIGN * COUNT_ALIGN;
   KMC_TRY(dalloc(c, c->d_site_count, (size_t)KMC_COUNT_COPIES * c->count_stride));
-  KMC_HIP(c, hipMemsetAsync(c->d_site_count.p, 0, c->d_site_count.n * sizeof(uint32_t),
-                            c->stream));
   KMC_TRY(dalloc(c, c->d_counts64, c->n_sites));
-  KMC_HIP(c, hipMemsetAsync(c->d_counts64.p, 0, c->n_sites * sizeof(uint64_t), c->stream));
-  c->count_pending = 0;
   KMC_TRY(dalloc(c, c->d_live, 3));
-  KMC_HIP(c, hipMemsetAsync(c->d_live.p, 0, 3 * sizeof(uint32_t), c->stream));
+  clear_args clear;
+  clear.add(c->d_site_count.p, (size_t)KMC_COUNT_COPIES * c->count_stride * sizeof(uint32_t));
+  clear.add(c->d_counts64.p, c->n_sites * sizeof(uint64_t));
+  clear.add(c->d_live.p, 3 * sizeof(uint32_t));
+  KMC_HIP(c, launch_clear(clear, c->stream));
+  c->count_pending = 0;
   c->run_launches = 0;
   c->n_exc = E;
   c->n_bins = c->bin0 = c->win_bins = 0;
@@ -1163,8 +1166,7 @@ static int set_samples(kmc_ctx* c, int32_t n_bins, double t_sample_max, int32_t 
   KMC_TRY(dalloc(c, c->r_dy, nrec));
   KMC_TRY(dalloc(c, c->r_dz, nrec));
   KMC_TRY(dalloc(c, c->r_drain, nrec));
-  KMC_HIP(c, hipMemsetAsync(c->x_krec.p, 0, c->n_exc * sizeof(uint32_t), c->stream));
-  KMC_TRY(clear_records(c, nrec));
+  KMC_TRY(clear_records(c, nrec, true));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
   c->n_bins = n_bins;
   c->bin0 = 0;
@@ -1218,7 +1220,7 @@ int kmc_next_sample_window(kmc_ctx* c) {
                     " samples up to the window's end (run to t >= " +
                     std::to_string(c->t_sample_max * end / c->n_bins) + " s first)");
   c->bin0 = end;
-  KMC_TRY(clear_records(c, (size_t)c->win_bins * c->n_exc));
+  KMC_TRY(clear_records(c, (size_t)c->win_bins * c->n_exc, false));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
   return KMC_OK;
 }

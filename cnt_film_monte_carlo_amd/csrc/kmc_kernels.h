@@ -188,6 +188,17 @@ hipError_t launch_interleave3(int64_t n, const double* x, const double* y, const
                               double* out, hipStream_t st);
 hipError_t launch_finish_pair_rates(int64_t n, const double* rates, const csr_arrays& out,
                                     int32_t* err, hipStream_t st);
+// Arrays of 32-bit words to zero, each on a 16-byte boundary.
+struct clear_args {
+  int n = 0;
+  void* p[5];
+  size_t words[5];
+  void add(void* q, size_t bytes) {
+    p[n] = q;
+    words[n++] = bytes / 4;
+  }
+};
+hipError_t launch_clear(const clear_args& a, hipStream_t st);
 hipError_t launch_inject(const exciton_arrays& x, const uint4* blocks, const uint32_t* src_roff,
                          uint32_t n_src, uint64_t seed, hipStream_t st);
 hipError_t launch_block_sizes(int64_t n, const site_hdr* hdr, const int32_t* order, uint32_t* lines,

@@ -2651,6 +2651,34 @@ hipError_t launch_unpack_rows(int64_t n, const site_hdr* hdr, int64_t* row, doub
   return hipGetLastError();
 }
 
+// Zeroes several arrays in one launch, 16 bytes a lane.  A new run on a small film is a handful of
+// arrays of a few kilobytes, where every launch costs ~4 us of host time and ~3 on the device
+// (1,000 excitons on 5,000 sites: an injection 21 us with a memset per array, 17 with this; a
+// sampling grid 23 and 13).
+__global__ __launch_bounds__(256) void k_clear(clear_args a) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+  for (int k = 0; k < a.n; ++k) {
+    uint32_t* p = static_cast<uint32_t*>(a.p[k]);
+    const size_t words = a.words[k], quads = words / 4;
+    for (size_t i = t; i < quads; i += step)
+      reinterpret_cast<uint4*>(p)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (t < words % 4) p[4 * quads + t] = 0u;
+  }
+}
+
+hipError_t launch_clear(const clear_args& a, hipStream_t st) {
+  size_t most = 0;
+  for (int k = 0; k < a.n; ++k) {
+    if ((uintptr_t)a.p[k] % 16 != 0) return hipErrorInvalidValue;
+    most = std::max(most, a.words[k]);
+  }
+  if (most == 0) return hipSuccess;
+  // up to 4,096 workgroups: beyond them a lane takes several pieces
+  const size_t groups = std::min<size_t>((most / 4 + 255) / 256 + 1, 4096);
+  hipLaunchKernelGGL(k_clear, dim3((unsigned)groups), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_interleave3(int64_t n, const double* x, const double* y, const double* z,
                               double* out, hipStream_t st) {
   if (n == 0) return hipSuccess;
