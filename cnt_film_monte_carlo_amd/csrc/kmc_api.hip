@@ -192,8 +192,9 @@ struct kmc_ctx {
   dbuf<uint64_t> c_next;
   dbuf<int32_t> c_err, c_pop_out, c_cur_out;
   dbuf<uint64_t> c_made;                  // hops made since kmc_contact_init
-  dbuf<uint32_t> c_skeys, c_sids;         // [2 capacity] slot sort (contact_key_layout_of): keys, ids
-  dbuf<uint8_t> c_sort_tmp;
+  // the slots' order (contact_key_layout_of): keys, the live slots in order, counts and cursors
+  dbuf<uint8_t> c_skeys;
+  dbuf<uint32_t> c_sids, c_bins;
   double c_step_ms = 0.0;                 // device time of the step kernels since then
   std::vector<hipEvent_t> c_ev;           // CONTACT_EV_PAIRS (start, stop) pairs, reused
   std::vector<char> c_ev_busy;            // pair recorded and not yet read
@@ -584,7 +585,7 @@ int kmc_destroy(kmc_ctx* c) {
   dfree(c->d_min);
   dfree(c->c_sites); dfree(c->c_keep); dfree(c->c_off); dfree(c->c_scan_tmp); dfree(c->c_live); dfree(c->c_base);
   dfree(c->c_live_out); dfree(c->c_next); dfree(c->c_err); dfree(c->c_pop_out); dfree(c->c_cur_out);
-  dfree(c->c_made); dfree(c->c_skeys); dfree(c->c_sids); dfree(c->c_sort_tmp);
+  dfree(c->c_made); dfree(c->c_skeys); dfree(c->c_sids); dfree(c->c_bins);
   for (hipEvent_t e : c->c_ev)
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : c->c_live_ev)
@@ -1968,31 +1969,27 @@ contact_slots contact_buf(kmc_ctx* c, int b) {
 // The order in which a step's threads take the live slots.  Slots sort by the eighth of the film
 // their site lies in (the eighths of the sorted slots go to the eight XCDs, so each XCD's L2
 // serves one compact region), then by the site's chirality, then by the site's row in the eighth,
-// to as many of the row's leading bits as the sort's last 8-bit pass has left.  The chirality sets
-// the rates a particle meets along its tube, so the particles of one wave make similar numbers of
-// hops in a step and fewer of its lanes idle while its last particle hops.  Finer rows gain
-// nothing: with 1 M particles on 625k sites of three chiralities the sort and the step kernel take
-// 73 + 655 us with 8 key bits, 124 + 685 with 16 and 178 + 687 with all 28; with one chirality
-// the kernel takes 6.5 ms at 8 bits, 6.9 at 11 and 7.0 at 16.
-// Dead slots follow the live ones in the sort's input and have the largest key, so its stability
-// leaves them last.
+// to as many of the row's leading bits as eight bits have left.  The chirality sets the rates a particle meets along its tube, so the particles of
+// one wave make similar numbers of hops in a step and fewer of its lanes idle while its last
+// particle hops.  Finer rows gain nothing: with 1 M particles on 625k sites of three chiralities
+// the step kernel takes 655 us with 8 key bits, 685 with 16 and 687 with all 28; with one
+// chirality 6.5 ms at 8 bits, 6.9 at 11 and 7.0 at 16.
 contact_key_layout contact_key_layout_of(const kmc_ctx* c, uint32_t lines) {
   const auto bits = [](uint32_t v) {  // bits that hold the values [0, v]
     int b = 1;
     while (b < 32 && (v >> b) != 0) ++b;
     return b;
   };
-  static_assert(KMC_COUNT_COPIES == 8, "three key bits hold the eighth");
+  static_assert(KMC_COUNT_COPIES == 8 && MAX_CHIR <= 32 && ORDER_BINS == 256,
+                "three key bits hold the eighth, up to five the chirality");
   contact_key_layout kl{};
   kl.lines = lines;
   uint8_t top = 0;
   for (const uint8_t ch : c->h_chir) top = std::max(top, ch);
   kl.chir_bits = top ? bits(top) : 0;
   const int row_bits = bits(lines / KMC_COUNT_COPIES + 1u);  // an eighth starts at a rounded line
-  kl.row_bits = std::min(row_bits, (3 + kl.chir_bits + 7) / 8 * 8 - (3 + kl.chir_bits));
+  kl.row_bits = std::min(row_bits, 5 - kl.chir_bits);
   kl.row_shift = row_bits - kl.row_bits;
-  kl.key_bits = 3 + kl.chir_bits + kl.row_bits;
-  kl.dead = (1u << kl.key_bits) - 1u;
   return kl;
 }
 
@@ -2209,19 +2206,17 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
   // errors are this call's: a hop cap reached leaves every particle consistent (the one that
   // stopped continues in the next step), so a retry with a larger cap may go on
   KMC_HIP(c, hipMemsetAsync(c->c_err.p, 0, sizeof(int32_t), c->stream));
-  // each step's threads take the live slots in the order of contact_key_layout_of (a radix sort;
-  // dead slots sort last): draws are keyed by particle id and hop count, so the order changes no
-  // result
+  // each step's threads take the live slots in the order of contact_key_layout_of: draws are keyed
+  // by particle id and hop count, so the order changes no result
   const int64_t cap = c->c_cap;
   const contact_key_layout kl = contact_key_layout_of(c, (uint32_t)(c->n_units / ROW_UNITS));
-  const int key_bits = kl.key_bits;
-  KMC_TRY(dalloc(c, c->c_skeys, 2 * (size_t)cap));
-  KMC_TRY(dalloc(c, c->c_sids, 2 * (size_t)cap));
-  size_t sort_need = 0;
-  KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(nullptr, sort_need, c->c_skeys.p,
-                                                c->c_skeys.p + cap, c->c_sids.p, c->c_sids.p + cap,
-                                                (int)cap, 0, key_bits, c->stream));
-  KMC_TRY(dalloc(c, c->c_sort_tmp, std::max<size_t>(sort_need, 1)));
+  KMC_TRY(dalloc(c, c->c_skeys, (size_t)cap));
+  KMC_TRY(dalloc(c, c->c_sids, (size_t)cap));
+  KMC_TRY(dalloc(c, c->c_bins, 2 * ORDER_BINS));
+  clear_args clear;
+  clear.add(c->c_bins.p, 2 * ORDER_BINS * sizeof(uint32_t));
+  KMC_HIP(c, launch_clear(clear, c->stream));
+  const contact_order order{c->c_skeys.p, c->c_bins.p, c->c_bins.p + ORDER_BINS, c->c_sids.p};
   // Step k covers the slots [0, bound): at most the live count, which a step raises by at most
   // the two contacts' injections.  The count is read exactly here, then after every step into
   // pinned memory, and step k uses the one after step k - CONTACT_LIVE_LAG.
@@ -2245,15 +2240,9 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
     a.max_hops = max_hops_per_step;
     a.pop = c->c_pop_out.p + k * S;
     a.cur = c->c_cur_out.p + k * (S - 1);
-    KMC_HIP(c, launch_contact_keys(bound, c->c_live.p, c->c_site[c->c_buf].p, c->d_roff.p,
-                                   c->d_chir.p, kl, c->c_skeys.p, c->c_sids.p, c->stream));
-    size_t have = c->c_sort_tmp.n;
-    if (bound > 0)
-      KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(c->c_sort_tmp.p, have, c->c_skeys.p,
-                                                    c->c_skeys.p + cap, c->c_sids.p,
-                                                    c->c_sids.p + cap, (int)bound, 0, key_bits,
-                                                    c->stream));
-    a.perm = c->c_sids.p + cap;
+    KMC_HIP(c, launch_contact_order(bound, c->c_live.p, c->c_site[c->c_buf].p, c->d_roff.p,
+                                    c->d_chir.p, kl, order, c->stream));
+    a.perm = order.perm;
     const int q = (int)(k % CONTACT_EV_PAIRS);
     KMC_TRY(contact_read_pair(c, q));
     KMC_HIP(c, hipEventRecord(c->c_ev[2 * q], c->stream));
@@ -2282,6 +2271,8 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
       m.tile_kept = c->c_off.p;  // capacity + 1 entries: room for both tiles' counts
       m.tile_first = c->c_off.p + scan_tmp_elems(bound);
       m.base = c->c_base.p;
+      m.order_count = order.count;
+      m.order_cursor = order.cursor;
       m.n_live = c->c_live.p;
       m.next_id = c->c_next.p;
       m.live_out = c->c_live_out.p + k;
@@ -2292,6 +2283,7 @@ int kmc_contact_run(kmc_ctx* c, double dt, int64_t n_steps, uint64_t max_hops_pe
     } else {
       // two sections whose closed ranges share a site's y: contact n_seg may remove particles that
       // contact 1 has just placed
+      KMC_HIP(c, launch_clear(clear, c->stream));  // for the next step's order
       int64_t n_side = bound;  // slots the live ones lie in: contact 1's injection may add some
       for (int side = 0; side < 2; ++side) {
         a.s = contact_buf(c, c->c_buf);

@@ -97,7 +97,7 @@ struct contact_args {
   int32_t* pop;             // [n_seg] particles per section after the step
   int32_t* cur;             // [n_seg - 1] net crossings of each interface during the step
   int32_t* err;             // CONTACT_ERR_* bits
-  net_view fv;              // v > 0: links, periods, velocity and blocks for the flights
+  net_view fv;              // v > 0: legs, periods, velocity and blocks for the flights
   unsigned long long* hops_made;  // hops made in contact mode so far (all particles)
   const uint32_t* perm;     // thread j steps slot perm[j] (the sorted slots); null: slot j
 };
@@ -115,6 +115,7 @@ struct contact_move_args {
   int64_t* tile_kept;       // per tile of slots: kept by both contacts (then its offset)
   int64_t* tile_first;      // kept by contact 1 alone (its injection must fit beside them)
   int64_t* base;            // [3]: kept, first new id, slots counted
+  uint32_t *order_count, *order_cursor;  // contact_order's, zeroed here
   int64_t* n_live;
   uint64_t* next_id;
   int64_t *live_out, *live_host;
@@ -223,21 +224,24 @@ hipError_t launch_exciton_keys(int64_t n, const int32_t* site, const int64_t* ro
 hipError_t launch_fill_blocks(int64_t n, const site_hdr* hdr, const double* cum,
                               const edge_rec* edge, const int64_t* roff, const double* px,
                               const double* py, const double* pz, uint4* blocks, hipStream_t st);
-// Sort key of a live contact slot: with `regions`, (eighth of the film by row line, chirality of
-// the site, row line) in bit fields [row_bits + chir_bits, +3], [row_bits, +chir_bits], [0,
-// row_bits); without, the row line alone.  Dead slots key `dead`, which sorts last.
+// Key of a live contact slot: (eighth of the film by row line, chirality of the site, row line) in
+// bit fields [row_bits + chir_bits, +3], [row_bits, +chir_bits], [0, row_bits), below ORDER_BINS.
+constexpr int ORDER_BINS = 256;
 struct contact_key_layout {
   uint32_t lines;      // row lines of the film (the eighths split [0, lines))
-  int32_t row_bits, chir_bits;
-  int32_t row_shift;   // the key holds a row's place in its eighth >> row_shift
-  uint32_t dead;       // the largest key
-  int32_t key_bits;    // bits the radix sort looks at
+  int32_t chir_bits;
+  int32_t row_bits, row_shift;  // the key holds a row's place in its eighth >> row_shift
 };
-// keys[i] = sort key of slot i (contact_key_layout), ids[i] = i
-hipError_t launch_contact_keys(int64_t capacity, const int64_t* n_live, const int32_t* site,
-                               const int64_t* roff, const uint8_t* chir,
-                               const contact_key_layout& kl, uint32_t* keys, uint32_t* ids,
-                               hipStream_t st);
+struct contact_order {
+  uint8_t* key;                 // of every slot
+  uint32_t *count, *cursor;     // [ORDER_BINS] zeroed: slots of a key, places taken
+  uint32_t* perm;               // the live slots in order
+};
+// o.perm = slots [0, *n_live) in the order of their keys; n >= *n_live
+hipError_t launch_contact_order(int64_t n, const int64_t* n_live, const int32_t* site,
+                                const int64_t* roff, const uint8_t* chir,
+                                const contact_key_layout& kl, const contact_order& o,
+                                hipStream_t st);
 // keys[i] = Morton code of site i's cell, ids[i] = i (block placement order, after a sort)
 hipError_t launch_morton_keys(int64_t n, const int32_t* cell_of, int32_t nx, int32_t ny,
                               uint64_t* keys, int32_t* ids, hipStream_t st);

@@ -47,3 +47,32 @@ def test_contact_repopulation_edges(kmc, orc, nw, n_seg, c1, c2, v):
     np.testing.assert_allclose(p["t_next"], ref["t_next"], rtol=1e-12)
     assert ctx.contact_stats()[0] == ref["hops_made"]
     ctx.close()
+
+
+@pytest.mark.parametrize("n_chir", [2, 3, 9, 16])
+def test_contact_order_keys(kmc, orc, nw, n_chir):
+    """The slots' order with one to four key bits for the chirality, 16 being the most a film has
+    (one rate for all pairs, 15 nm cutoff): every particle as the oracle's."""
+    print(f"[gpu-contact-move] {n_chir} chiralities", file=sys.stderr, flush=True)
+    w = nw.film_small()
+    net = nw.build_network(w)
+    net["flags"] = np.zeros(net["n"], np.uint8)
+    net["chirality"] = ((np.arange(net["n"]) // 20) % n_chir).astype(np.uint8)
+    tab = ([0.0], [0.0], [0.0], [0.0], np.full(n_chir * n_chir, 1e12))
+    ctx = kmc.Context(kmc.Config(cutoff=w.cutoff, min_distance=0.4 * NM, seed=43))
+    ctx.set_sites(net["x"], net["y"], net["z"], net["ox"], net["oy"], net["oz"], net["left"],
+                  net["right"], net["chirality"], net["flags"])
+    ctx.set_rate_table(*tab)
+    ctx.build_cells()
+    ctx.build_rates(kmc.RATE_TABLE)
+    ctx.contact_init(5, 900, 100, 8000)
+    pop, cur, live = ctx.contact_run(2e-12, 4)
+    onet = orc.Net(net, w.cutoff, 0.4 * NM)
+    onet.set_table(*[np.asarray(t, float) for t in tab])
+    ref = orc.contact(net, onet.csr(0), 43, 5, 900, 100, 8000, 2e-12, 4)
+    assert np.array_equal(pop, ref["population"]) and np.array_equal(cur, ref["crossings"])
+    assert np.array_equal(live, ref["n_live"]) and ref["hops_made"] > 1000
+    p = ctx.contact_particles()
+    for k in ("id", "site", "hops"):
+        assert np.array_equal(p[k], ref[k]), k
+    ctx.close()
