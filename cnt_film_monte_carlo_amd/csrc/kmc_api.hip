@@ -149,8 +149,9 @@ struct kmc_ctx {
   dbuf<uint64_t> d_counts64;    // running 64-bit totals the copies are folded into
   int64_t count_stride = 0;
   uint64_t count_pending = 0;   // bound on any copy's count since the last fold
-  dbuf<uint32_t> d_live;        // [0] excitons able to hop after the last launch; [1], [2] the
-                                // excitons not idle at a launch's start, used alternately
+  // LIVE_WORDS counts, by launch parity: [0], [1] the excitons able to hop after a launch; [2], [3]
+  // those not idle at its start
+  dbuf<uint32_t> d_live;
   int64_t run_launches = 0;     // hop launches of the last kmc_run
   // hop-kernel timing of a timed kmc_run: one (start, stop) event pair per launch
   std::vector<hipEvent_t> hop_ev;
@@ -210,6 +211,7 @@ constexpr int CONTACT_EV_PAIRS = 64;
 // the live count after step k - CONTACT_LIVE_LAG bounds the slots step k's sort, step and
 // compaction cover; the host waits for it only that many steps back
 constexpr int CONTACT_LIVE_LAG = 2;
+constexpr int LIVE_WORDS = 4;
 
 // Sites or pairs that a read-back rearranges on the device at a time, 16 bytes each in d_read.
 constexpr int64_t READ_CHUNK = (int64_t)1 << 20;
@@ -1131,11 +1133,11 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   c->count_stride = (n_lines + COUNT_ALIGN - 1) / COUNT_ALIGN * COUNT_ALIGN;
   KMC_TRY(dalloc(c, c->d_site_count, (size_t)KMC_COUNT_COPIES * c->count_stride));
   KMC_TRY(dalloc(c, c->d_counts64, c->n_sites));
-  KMC_TRY(dalloc(c, c->d_live, 3));
+  KMC_TRY(dalloc(c, c->d_live, LIVE_WORDS));
   clear_args clear;
   clear.add(c->d_site_count.p, (size_t)KMC_COUNT_COPIES * c->count_stride * sizeof(uint32_t));
   clear.add(c->d_counts64.p, c->n_sites * sizeof(uint64_t));
-  clear.add(c->d_live.p, 3 * sizeof(uint32_t));
+  clear.add(c->d_live.p, LIVE_WORDS * sizeof(uint32_t));
   KMC_HIP(c, launch_clear(clear, c->stream));
   c->count_pending = 0;
   c->run_launches = 0;
@@ -1305,12 +1307,32 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
     it.k_rec = sample ? c->x_krec.p : nullptr;
     it.n_bins = a.v.n_bins;
     it.dt_sample = a.v.dt_sample;
-    KMC_HIP(c, hipMemsetAsync(c->d_live.p + 1, 0, 2 * sizeof(uint32_t), c->stream));
+    KMC_HIP(c, hipMemsetAsync(c->d_live.p + 2, 0, 2 * sizeof(uint32_t), c->stream));
   }
   const int64_t step = chunk > 0 ? chunk : std::max<int64_t>(hops, 1);
   int64_t done = 0, launches = 0;
   int64_t movable = E;  // an upper bound on the excitons a launch can move (the last live count)
+  // and on those it looks at: the ones not idle where the idle are left out, else all of them,
+  // trapped ones too.  An idle exciton stays idle, so a count bounds the later launches'.
+  int64_t walked = E;
   do {
+    const int parity = (int)(launches & 1);
+    if (leave_idle) {
+      it.alive = c->d_live.p + 2 + parity;
+      it.alive_next = c->d_live.p + 3 - parity;
+      a.n_alive = it.alive;
+    }
+    a.v.live = c->d_live.p + parity;
+    KMC_HIP(c, launch_exciton_keys(E, c->x_site.p, c->d_roff.p, it, c->d_keys.p, c->d_ids.p,
+                                   a.v.live, c->stream));
+    if (launches > 0 && live_check_due(launches)) {
+      uint32_t n[LIVE_WORDS];
+      KMC_TRY(copy_out(c, n, c->d_live.p, sizeof(n)));
+      const int64_t live = n[1 - parity];
+      if (live == 0) break;
+      movable = std::min(movable, live);
+      if (leave_idle) walked = std::min<int64_t>(walked, n[2 + parity]);
+    }
     int64_t len = step;
     if (chunk > 0 && movable * TAIL_FRACTION <= E && step <= INT64_MAX / TAIL_STRETCH)
       len = step * TAIL_STRETCH;
@@ -1322,13 +1344,6 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
       if (c->count_pending + add > COUNT_COPY_MAX) KMC_TRY(fold_counts(c, c->stream));
       c->count_pending += add;
     }
-    if (leave_idle) {
-      it.alive = c->d_live.p + 1 + (launches & 1);
-      it.alive_next = c->d_live.p + 1 + ((launches + 1) & 1);
-      a.n_alive = it.alive;
-    }
-    KMC_HIP(c, launch_exciton_keys(E, c->x_site.p, c->d_roff.p, it, c->d_keys.p, c->d_ids.p,
-                                   c->d_live.p, c->stream));
     size_t have = c->sort_tmp_bytes;
     KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(c->d_sort_tmp.p, have, c->d_keys.p,
                                                   c->d_keys.p + E, c->d_ids.p, c->d_ids.p + E,
@@ -1342,20 +1357,14 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
       }
       KMC_HIP(c, hipEventRecord(c->hop_ev[2 * launches], c->stream));
     }
-    if (!fly && hop_rows_pays(movable, c->n_cu))
-      KMC_HIP(c, launch_hop_rows(a, movable, (uint32_t)(c->n_units / ROW_UNITS), c->n_cu, count,
+    if (!fly && hop_rows_pays(walked, c->n_cu))
+      KMC_HIP(c, launch_hop_rows(a, walked, (uint32_t)(c->n_units / ROW_UNITS), c->n_cu, count,
                                  sample, trace, c->stream));
     else
       KMC_HIP(c, launch_hop(a, count, sample, trace, fly, c->stream));
     if (c->time_hops) KMC_HIP(c, hipEventRecord(c->hop_ev[2 * launches + 1], c->stream));
     done += sub;
     ++launches;
-    if (done < hops && live_check_due(launches)) {
-      uint32_t live = 0;
-      KMC_TRY(copy_out(c, &live, c->d_live.p, sizeof(uint32_t)));
-      if (live == 0u) break;
-      movable = std::min<int64_t>(movable, (int64_t)live);
-    }
   } while (done < hops);
   c->run_launches = launches;
   if (c->time_hops) {
@@ -1480,9 +1489,9 @@ int kmc_get_run_stats(kmc_ctx* c, int64_t* launches, int64_t* live_excitons) {
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   if (launches) *launches = c->run_launches;
   if (live_excitons) {
-    uint32_t live = 0;
-    KMC_TRY(copy_out(c, &live, c->d_live.p, sizeof(uint32_t)));
-    *live_excitons = c->run_launches > 0 ? (int64_t)live : -1;
+    uint32_t live[2] = {0, 0};
+    KMC_TRY(copy_out(c, live, c->d_live.p, sizeof(live)));
+    *live_excitons = c->run_launches > 0 ? (int64_t)live[(c->run_launches - 1) & 1] : -1;
   }
   return KMC_OK;
 }

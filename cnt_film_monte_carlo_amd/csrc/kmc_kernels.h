@@ -262,10 +262,11 @@ hipError_t launch_mask_count(int64_t nnz, const uint8_t* cls, const uint8_t* mas
                              hipStream_t st);
 hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bool fly,
                       hipStream_t st);
-// The hop loop for launches of few excitons (k_hop_rows).  `movable`, the excitons expected to
-// move, decides and sizes the grid; any number is handled.  n_lines = block lines of the film.
-bool hop_rows_pays(int64_t movable, int n_cu);
-hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
+// The hop loop for launches of few excitons (k_hop_rows).  `walked`, the positions of the order that
+// the launch looks at (movable or not), decides and sizes the grid; *n_alive, or v.x.n where that is
+// null, may not exceed it.  n_lines = block lines of the film.
+bool hop_rows_pays(int64_t walked, int n_cu);
+hipError_t launch_hop_rows(hop_args a, int64_t walked, uint32_t n_lines, int n_cu, bool count,
                            bool sample, bool trace, hipStream_t st);
 // table[2 (2 roff[i] + heading)], [.. + 1]: the leg of a flight at site i (scatterer::left/right,
 // scatterer.h:29-30; half_per as in net_view); *bad is set where a link has no length

@@ -1819,10 +1819,10 @@ __device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool val
   if (TRACE && e < tv.n_trace) tv.tr_n[e] = tr;
 }
 
-// Positions as in k_hop, blockDim.x / 16 excitons to a workgroup; the workgroups of an XCD walk
-// its eighth of the order.  The departure counts of the lines around the workgroup's first
-// exciton -- all lines of a small film -- go to a window of 32-bit LDS counters (a launch's hops
-// cannot wrap one: at most 2^32 departures per copy), the others to the XCD's copy.
+// Positions as in k_hop, blockDim.x / 16 excitons to a workgroup; the workgroups of an XCD take its
+// eighth of the order.  The departure counts of the lines around the workgroup's first exciton --
+// all lines of a small film -- go to a window of 32-bit LDS counters (a launch's hops cannot wrap
+// one: at most 2^32 departures per copy), the others to the XCD's copy.
 template <bool COUNT, bool SAMPLE, bool TRACE>
 __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   extern __shared__ uint4 rows_lds[];
@@ -1834,33 +1834,30 @@ __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   const uint32_t groups = (n + per_group - 1u) / per_group;
   const uint32_t per_xcd = (groups + KMC_COUNT_COPIES - 1u) / KMC_COUNT_COPIES;
   const uint32_t lane = threadIdx.x & 63u;
-  for (uint32_t rank = blockIdx.x / KMC_COUNT_COPIES; rank < per_xcd;
-       rank += gridDim.x / KMC_COUNT_COPIES) {
-    const uint32_t p0 = ((blockIdx.x % KMC_COUNT_COPIES) * per_xcd + rank) * per_group;
-    if (p0 >= n) break;
-    const uint32_t pos = p0 + (threadIdx.x >> 4);
-    const bool valid = pos < n;
-    const uint32_t e = valid ? (a.perm ? a.perm[pos] : pos) : 0u;
-    uint32_t base = 0u;
-    if constexpr (COUNT) {
-      for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) win[i] = 0u;
-      if (a.win_lines < a.n_lines) {
-        const uint32_t L0 = (uint32_t)a.v.roff[a.v.x.site[a.perm ? a.perm[p0] : p0]];
-        base = L0 > a.win_lines / 2u ? L0 - a.win_lines / 2u : 0u;
-        base = min(base, a.n_lines - a.win_lines);
-      }
-      __syncthreads();
+  const uint32_t rank = blockIdx.x / KMC_COUNT_COPIES;
+  const uint32_t p0 = ((blockIdx.x % KMC_COUNT_COPIES) * per_xcd + rank) * per_group;
+  if (rank >= per_xcd || p0 >= n) return;
+  const uint32_t pos = p0 + (threadIdx.x >> 4);
+  const bool valid = pos < n;
+  const uint32_t e = valid ? (a.perm ? a.perm[pos] : pos) : 0u;
+  uint32_t base = 0u;
+  if constexpr (COUNT) {
+    for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) win[i] = 0u;
+    if (a.win_lines < a.n_lines) {
+      const uint32_t L0 = (uint32_t)a.v.roff[a.v.x.site[a.perm ? a.perm[p0] : p0]];
+      base = L0 > a.win_lines / 2u ? L0 - a.win_lines / 2u : 0u;
+      base = min(base, a.n_lines - a.win_lines);
     }
-    hop_rows<COUNT, SAMPLE, TRACE>(a.v, e, valid, a.hop_budget, a.t_max, a.tv, s, lane, win, base,
-                                   a.win_lines);
-    if constexpr (COUNT) {
-      __syncthreads();
-      uint32_t* cbase = a.v.site_count + (size_t)xcd_id() * a.v.count_stride;
-      for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) {
-        const uint32_t cnt = win[i];
-        if (cnt) atomicAdd(cbase + count_slot(base + i, a.v.count_stride), cnt);
-      }
-      __syncthreads();
+    __syncthreads();
+  }
+  hop_rows<COUNT, SAMPLE, TRACE>(a.v, e, valid, a.hop_budget, a.t_max, a.tv, s, lane, win, base,
+                                 a.win_lines);
+  if constexpr (COUNT) {
+    __syncthreads();
+    uint32_t* cbase = a.v.site_count + (size_t)xcd_id() * a.v.count_stride;
+    for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) {
+      const uint32_t cnt = win[i];
+      if (cnt) atomicAdd(cbase + count_slot(base + i, a.v.count_stride), cnt);
     }
   }
 }
@@ -2008,13 +2005,13 @@ constexpr int64_t CU_LDS = 160 * 1024;
 // A row of lanes per exciton pays up to 128 excitons per CU: 1,250 hops on 76,543 sites take
 // 0.72 / 0.94 / 1.53 / 1.91 / 3.3 ms at 1,000 / 16,384 / 24,576 / 32,768 / 50,000 excitons (a wave
 // round per 16,384), k_hop's lane per exciton 1.93 / 2.03 / 2.07 / 2.10 / 2.14 ms.
-bool hop_rows_pays(int64_t movable, int n_cu) { return movable <= (int64_t)128 * n_cu; }
+bool hop_rows_pays(int64_t walked, int n_cu) { return walked <= (int64_t)128 * n_cu; }
 
-hipError_t launch_hop_rows(hop_args a, int64_t movable, uint32_t n_lines, int n_cu, bool count,
+hipError_t launch_hop_rows(hop_args a, int64_t walked, uint32_t n_lines, int n_cu, bool count,
                            bool sample, bool trace, hipStream_t st) {
   int bs = 64;
-  while (bs < 256 && movable * 16 > (int64_t)bs * n_cu) bs *= 2;
-  const int64_t groups = (movable * 16 + bs - 1) / bs;
+  while (bs < 256 && walked * 16 > (int64_t)bs * n_cu) bs *= 2;
+  const int64_t groups = (walked * 16 + bs - 1) / bs;
   const int64_t grid = (groups + KMC_COUNT_COPIES - 1) / KMC_COUNT_COPIES * KMC_COUNT_COPIES;
   // the window takes what the workgroups that share a CU leave of its LDS
   const int64_t share = CU_LDS / std::max<int64_t>(1, std::min<int64_t>(8, (grid + n_cu - 1) / n_cu)) - 1024;
