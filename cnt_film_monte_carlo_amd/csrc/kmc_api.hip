@@ -149,8 +149,8 @@ struct kmc_ctx {
   dbuf<uint64_t> d_counts64;    // running 64-bit totals the copies are folded into
   int64_t count_stride = 0;
   uint64_t count_pending = 0;   // bound on any copy's count since the last fold
-  // LIVE_WORDS counts, by launch parity: [0], [1] the excitons able to hop after a launch; [2], [3]
-  // those not idle at its start
+  // by launch parity p: at LIVE_HALF p the excitons able to hop after a launch, in LIVE_SLOTS words;
+  // at 2 LIVE_HALF + p those not idle at its start
   dbuf<uint32_t> d_live;
   int64_t run_launches = 0;     // hop launches of the last kmc_run
   // hop-kernel timing of a timed kmc_run: one (start, stop) event pair per launch
@@ -211,7 +211,7 @@ constexpr int CONTACT_EV_PAIRS = 64;
 // the live count after step k - CONTACT_LIVE_LAG bounds the slots step k's sort, step and
 // compaction cover; the host waits for it only that many steps back
 constexpr int CONTACT_LIVE_LAG = 2;
-constexpr int LIVE_WORDS = 4;
+constexpr int LIVE_HALF = LIVE_SLOTS * LIVE_STRIDE, LIVE_WORDS = 2 * LIVE_HALF + 2;
 
 // Sites or pairs that a read-back rearranges on the device at a time, 16 bytes each in d_read.
 constexpr int64_t READ_CHUNK = (int64_t)1 << 20;
@@ -1268,6 +1268,12 @@ static inline bool live_check_due(int64_t launches) {
   return (launches & (launches - 1)) == 0 || launches % LIVE_CHECK_EVERY == 0;
 }
 
+static int64_t live_sum(const uint32_t* half) {
+  int64_t n = 0;
+  for (int k = 0; k < LIVE_SLOTS; ++k) n += half[k * LIVE_STRIDE];
+  return n;
+}
+
 static int fold_counts(kmc_ctx* c, hipStream_t st) {
   KMC_HIP(c, launch_fold_counts(c->n_units / ROW_UNITS, c->count_stride, c->d_blocks.p,
                                 c->d_site_count.p, c->d_counts64.p, st));
@@ -1307,7 +1313,7 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
     it.k_rec = sample ? c->x_krec.p : nullptr;
     it.n_bins = a.v.n_bins;
     it.dt_sample = a.v.dt_sample;
-    KMC_HIP(c, hipMemsetAsync(c->d_live.p + 2, 0, 2 * sizeof(uint32_t), c->stream));
+    KMC_HIP(c, hipMemsetAsync(c->d_live.p + 2 * LIVE_HALF, 0, 2 * sizeof(uint32_t), c->stream));
   }
   const int64_t step = chunk > 0 ? chunk : std::max<int64_t>(hops, 1);
   int64_t done = 0, launches = 0;
@@ -1318,20 +1324,20 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
   do {
     const int parity = (int)(launches & 1);
     if (leave_idle) {
-      it.alive = c->d_live.p + 2 + parity;
-      it.alive_next = c->d_live.p + 3 - parity;
+      it.alive = c->d_live.p + 2 * LIVE_HALF + parity;
+      it.alive_next = c->d_live.p + 2 * LIVE_HALF + 1 - parity;
       a.n_alive = it.alive;
     }
-    a.v.live = c->d_live.p + parity;
+    a.v.live = c->d_live.p + parity * LIVE_HALF;
     KMC_HIP(c, launch_exciton_keys(E, c->x_site.p, c->d_roff.p, it, c->d_keys.p, c->d_ids.p,
                                    a.v.live, c->stream));
     if (launches > 0 && live_check_due(launches)) {
       uint32_t n[LIVE_WORDS];
       KMC_TRY(copy_out(c, n, c->d_live.p, sizeof(n)));
-      const int64_t live = n[1 - parity];
+      const int64_t live = live_sum(n + (1 - parity) * LIVE_HALF);
       if (live == 0) break;
       movable = std::min(movable, live);
-      if (leave_idle) walked = std::min<int64_t>(walked, n[2 + parity]);
+      if (leave_idle) walked = std::min<int64_t>(walked, n[2 * LIVE_HALF + parity]);
     }
     int64_t len = step;
     if (chunk > 0 && movable * TAIL_FRACTION <= E && step <= INT64_MAX / TAIL_STRETCH)
@@ -1489,9 +1495,9 @@ int kmc_get_run_stats(kmc_ctx* c, int64_t* launches, int64_t* live_excitons) {
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   if (launches) *launches = c->run_launches;
   if (live_excitons) {
-    uint32_t live[2] = {0, 0};
-    KMC_TRY(copy_out(c, live, c->d_live.p, sizeof(live)));
-    *live_excitons = c->run_launches > 0 ? (int64_t)live[(c->run_launches - 1) & 1] : -1;
+    uint32_t n[LIVE_HALF];
+    KMC_TRY(copy_out(c, n, c->d_live.p + ((c->run_launches + 1) & 1) * LIVE_HALF, sizeof(n)));
+    *live_excitons = c->run_launches > 0 ? live_sum(n) : -1;
   }
   return KMC_OK;
 }

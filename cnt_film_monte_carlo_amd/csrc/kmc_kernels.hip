@@ -467,10 +467,8 @@ __global__ __launch_bounds__(256) void k_exciton_keys(int64_t n, const int32_t* 
                                                       uint32_t* __restrict__ live) {
 #pragma clang fp contract(off)
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e == 0) {
-    if (live) *live = 0u;
-    if (it.alive_next) *it.alive_next = 0u;
-  }
+  if (e < LIVE_SLOTS) live[e * LIVE_STRIDE] = 0u;
+  if (e == 0 && it.alive_next) *it.alive_next = 0u;
   bool alive = false;
   if (e < n) {
     uint32_t key = (uint32_t)roff[site[e]];
@@ -1804,7 +1802,9 @@ __device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool val
   if (v.live) {
     // excitons that a further launch could move (the budget aside)
     const uint64_t b = __ballot(valid && l == 0u && !trapped(n, gamma) && t <= t_max);
-    if (lane == 0u && b != 0ull) atomicAdd(v.live, (uint32_t)__popcll(b));
+    // 8,192 waves ending together, one after another on one word, took 80 us of a launch
+    if (lane == 0u && b != 0ull)
+      atomicAdd(v.live + (blockIdx.x % LIVE_SLOTS) * LIVE_STRIDE, (uint32_t)__popcll(b));
   }
   if (!valid || l != 0u) return;
   v.x.site[e] = (int32_t)site;
