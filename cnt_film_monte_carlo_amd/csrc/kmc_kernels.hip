@@ -1823,6 +1823,8 @@ __device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool val
 // eighth of the order.  The departure counts of the lines around the workgroup's first exciton --
 // all lines of a small film -- go to a window of 32-bit LDS counters (a launch's hops cannot wrap
 // one: at most 2^32 departures per copy), the others to the XCD's copy.
+constexpr uint32_t WIN_AHEAD = 8;  // 16-byte pieces of the window that a thread clears or reads at once
+
 template <bool COUNT, bool SAMPLE, bool TRACE>
 __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   extern __shared__ uint4 rows_lds[];
@@ -1834,6 +1836,7 @@ __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   const uint32_t groups = (n + per_group - 1u) / per_group;
   const uint32_t per_xcd = (groups + KMC_COUNT_COPIES - 1u) / KMC_COUNT_COPIES;
   const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t quads = (a.win_lines + 3u) / 4u;  // of the window, in whole 16 bytes
   const uint32_t rank = blockIdx.x / KMC_COUNT_COPIES;
   const uint32_t p0 = ((blockIdx.x % KMC_COUNT_COPIES) * per_xcd + rank) * per_group;
   if (rank >= per_xcd || p0 >= n) return;
@@ -1842,7 +1845,10 @@ __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   const uint32_t e = valid ? (a.perm ? a.perm[pos] : pos) : 0u;
   uint32_t base = 0u;
   if constexpr (COUNT) {
-    for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) win[i] = 0u;
+    for (uint32_t i = threadIdx.x; i < quads; i += WIN_AHEAD * blockDim.x)
+#pragma unroll
+      for (uint32_t k = 0; k < WIN_AHEAD; ++k)
+        reinterpret_cast<uint4*>(win)[min(i + k * blockDim.x, quads - 1u)] = make_uint4(0u, 0u, 0u, 0u);
     if (a.win_lines < a.n_lines) {
       const uint32_t L0 = (uint32_t)a.v.roff[a.v.x.site[a.perm ? a.perm[p0] : p0]];
       base = L0 > a.win_lines / 2u ? L0 - a.win_lines / 2u : 0u;
@@ -1855,9 +1861,23 @@ __global__ __launch_bounds__(256, 4) void k_hop_rows(hop_args a) {
   if constexpr (COUNT) {
     __syncthreads();
     uint32_t* cbase = a.v.site_count + (size_t)xcd_id() * a.v.count_stride;
-    for (uint32_t i = threadIdx.x; i < a.win_lines; i += blockDim.x) {
-      const uint32_t cnt = win[i];
-      if (cnt) atomicAdd(cbase + count_slot(base + i, a.v.count_stride), cnt);
+    for (uint32_t i = threadIdx.x; i < quads; i += WIN_AHEAD * blockDim.x) {
+      uint4 q[WIN_AHEAD];
+      uint32_t any = 0u;
+#pragma unroll
+      for (uint32_t k = 0; k < WIN_AHEAD; ++k) {
+        q[k] = reinterpret_cast<const uint4*>(win)[min(i + k * blockDim.x, quads - 1u)];
+        any |= q[k].x | q[k].y | q[k].z | q[k].w;
+      }
+      if (any == 0u) continue;
+#pragma unroll
+      for (uint32_t k = 0; k < WIN_AHEAD; ++k) {
+        const uint32_t at = i + k * blockDim.x, cnt[4] = {q[k].x, q[k].y, q[k].z, q[k].w};
+        if (at >= quads) break;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j)
+          if (cnt[j]) atomicAdd(cbase + count_slot(base + 4u * at + j, a.v.count_stride), cnt[j]);
+      }
     }
   }
 }
@@ -2013,12 +2033,17 @@ hipError_t launch_hop_rows(hop_args a, int64_t walked, uint32_t n_lines, int n_c
   while (bs < 256 && walked * 16 > (int64_t)bs * n_cu) bs *= 2;
   const int64_t groups = (walked * 16 + bs - 1) / bs;
   const int64_t grid = (groups + KMC_COUNT_COPIES - 1) / KMC_COUNT_COPIES * KMC_COUNT_COPIES;
-  // the window takes what the workgroups that share a CU leave of its LDS
+  // the window takes what the workgroups that share a CU leave of its LDS, but no more than a
+  // launch's hops pay for: a thread clears and flushes four lines at a time, one such turn per hop
+  // (one hop of one exciton on 300,000 sites: 56 us of clearing and flushing 39,000 lines one at a
+  // time by a single wave, as against a hop kernel of 5)
+  const int64_t paid = 4 * (int64_t)std::min<uint64_t>(a.hop_budget, 1u << 20) * bs;
   const int64_t share = CU_LDS / std::max<int64_t>(1, std::min<int64_t>(8, (grid + n_cu - 1) / n_cu)) - 1024;
   const int64_t batches = (int64_t)(bs / 64) * (int64_t)sizeof(batch_lds);
   a.n_lines = n_lines;
-  a.win_lines = count ? (uint32_t)std::max<int64_t>(0, std::min<int64_t>(n_lines, (share - batches) / 4)) : 0u;
-  const size_t lds = (size_t)(batches + 4ll * a.win_lines);
+  const int64_t fits = std::max<int64_t>(0, (share - batches) / 16 * 4);
+  a.win_lines = count ? (uint32_t)std::min<int64_t>({n_lines, fits, paid}) : 0u;
+  const size_t lds = (size_t)(batches + 16ll * ((a.win_lines + 3) / 4));
 #define KMC_ROWS_CASE(C, S, T)                                                                 \
   if (count == C && sample == S && trace == T) {                                               \
     hipLaunchKernelGGL((k_hop_rows<C, S, T>), dim3((unsigned)grid), dim3(bs), lds, st, a);     \

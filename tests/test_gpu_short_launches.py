@@ -1,5 +1,6 @@
 """Launches of a hop or a few with few excitons: the row-of-lanes kernel's fixed costs (the count of
-excitons that can still move) against the lane-per-exciton kernel that one more exciton takes."""
+excitons that can still move, the window of departure counts) against launches without them, and the
+window's edges against the oracle."""
 import sys
 
 import numpy as np
@@ -40,3 +41,37 @@ def test_many_waves_ending_together(film):
     say(f"one hop of {line} excitons {rows:.1f} us, of one more {lanes:.1f} us")
     assert rows <= 3 * lanes
     assert film.run_stats() == (1, line + 1)
+
+
+def test_window_of_a_short_launch(kmc, nw):
+    """Departure counts of one hop on a film of far more lines than a window holds."""
+    w = nw.film_large()
+    w.net.n_tubes = 1500
+    ctx = nw.make_context(w, nw.build_network(w), seed=5)
+    ctx.set_rate_table(*nw.forster_tables(3))
+    ctx.build_cells()
+    ctx.build_rates(kmc.RATE_TABLE)
+    with_counts, without = (_hop_us(ctx, 1, 1, c) for c in (True, False))
+    say(f"one hop of one exciton on {ctx.n_sites} sites, with counts {with_counts:.1f} us, "
+        f"without {without:.1f} us")
+    ctx.close()
+    assert with_counts <= 3 * without
+
+
+@pytest.mark.parametrize("n_exc,hops", [(1, 1), (2, 3), (5, 1), (9, 2), (300, 1), (4100, 2), (16400, 5)])
+def test_short_launches_match_oracle(kmc, orc, film, nw, n_exc, hops):
+    """Windows of 4 lines per thread and hop, from 256 lines up to the film's."""
+    say(f"{n_exc} excitons, calls of {hops} hops")
+    ctx = film
+    ctx.inject(n_exc)
+    csr = ctx.get_csr()
+    flags = nw.build_network(nw.film_small())["flags"]
+    ox = orc.Excitons(csr, flags, seed=61, n_excitons=n_exc)
+    for _ in range(3):
+        ctx.run(hops)
+        ox.run(hops)
+    g = ctx.get_excitons()
+    for k, o in (("site", ox.site), ("hops", ox.hops), ("hash", ox.hash), ("drains", ox.drains),
+                 ("disp", ox.dsp)):
+        assert np.array_equal(g[k], o), k
+    assert np.array_equal(ctx.get_hop_counts(), ox.site_count)
