@@ -149,8 +149,8 @@ struct kmc_ctx {
   dbuf<uint64_t> d_counts64;    // running 64-bit totals the copies are folded into
   int64_t count_stride = 0;
   uint64_t count_pending = 0;   // bound on any copy's count since the last fold
-  // by launch parity p: at LIVE_HALF p the excitons able to hop after a launch, in LIVE_SLOTS words;
-  // at 2 LIVE_HALF + p those not idle at its start
+  // the counts of excitons after the last launch (net_view::live), then at LIVE_ALIVE two words,
+  // used alternately: those not idle at a launch's start
   dbuf<uint32_t> d_live;
   int64_t run_launches = 0;     // hop launches of the last kmc_run
   // hop-kernel timing of a timed kmc_run: one (start, stop) event pair per launch
@@ -211,7 +211,7 @@ constexpr int CONTACT_EV_PAIRS = 64;
 // the live count after step k - CONTACT_LIVE_LAG bounds the slots step k's sort, step and
 // compaction cover; the host waits for it only that many steps back
 constexpr int CONTACT_LIVE_LAG = 2;
-constexpr int LIVE_HALF = LIVE_SLOTS * LIVE_STRIDE, LIVE_WORDS = 2 * LIVE_HALF + 2;
+constexpr int LIVE_ALIVE = LIVE_SLOTS * LIVE_STRIDE, LIVE_WORDS = LIVE_ALIVE + 2;
 
 // Sites or pairs that a read-back rearranges on the device at a time, 16 bytes each in d_read.
 constexpr int64_t READ_CHUNK = (int64_t)1 << 20;
@@ -1268,10 +1268,15 @@ static inline bool live_check_due(int64_t launches) {
   return (launches & (launches - 1)) == 0 || launches % LIVE_CHECK_EVERY == 0;
 }
 
-static int64_t live_sum(const uint32_t* half) {
-  int64_t n = 0;
-  for (int k = 0; k < LIVE_SLOTS; ++k) n += half[k * LIVE_STRIDE];
-  return n;
+static int read_live(kmc_ctx* c, int64_t* live, int64_t* stuck) {
+  uint32_t n[LIVE_ALIVE];
+  KMC_TRY(copy_out(c, n, c->d_live.p, sizeof(n)));
+  *live = *stuck = 0;
+  for (int k = 0; k < LIVE_SLOTS; ++k) {
+    *live += n[k * LIVE_STRIDE];
+    *stuck += n[k * LIVE_STRIDE + 1];
+  }
+  return KMC_OK;
 }
 
 static int fold_counts(kmc_ctx* c, hipStream_t st) {
@@ -1313,32 +1318,15 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
     it.k_rec = sample ? c->x_krec.p : nullptr;
     it.n_bins = a.v.n_bins;
     it.dt_sample = a.v.dt_sample;
-    KMC_HIP(c, hipMemsetAsync(c->d_live.p + 2 * LIVE_HALF, 0, 2 * sizeof(uint32_t), c->stream));
+    KMC_HIP(c, hipMemsetAsync(c->d_live.p + LIVE_ALIVE, 0, 2 * sizeof(uint32_t), c->stream));
   }
   const int64_t step = chunk > 0 ? chunk : std::max<int64_t>(hops, 1);
   int64_t done = 0, launches = 0;
   int64_t movable = E;  // an upper bound on the excitons a launch can move (the last live count)
-  // and on those it looks at: the ones not idle where the idle are left out, else all of them,
-  // trapped ones too.  An idle exciton stays idle, so a count bounds the later launches'.
+  // and on those it looks at: the movable and the trapped whose clock is not past t_max where the
+  // idle are left out (an idle exciton stays idle), else all
   int64_t walked = E;
   do {
-    const int parity = (int)(launches & 1);
-    if (leave_idle) {
-      it.alive = c->d_live.p + 2 * LIVE_HALF + parity;
-      it.alive_next = c->d_live.p + 2 * LIVE_HALF + 1 - parity;
-      a.n_alive = it.alive;
-    }
-    a.v.live = c->d_live.p + parity * LIVE_HALF;
-    KMC_HIP(c, launch_exciton_keys(E, c->x_site.p, c->d_roff.p, it, c->d_keys.p, c->d_ids.p,
-                                   a.v.live, c->stream));
-    if (launches > 0 && live_check_due(launches)) {
-      uint32_t n[LIVE_WORDS];
-      KMC_TRY(copy_out(c, n, c->d_live.p, sizeof(n)));
-      const int64_t live = live_sum(n + (1 - parity) * LIVE_HALF);
-      if (live == 0) break;
-      movable = std::min(movable, live);
-      if (leave_idle) walked = std::min<int64_t>(walked, n[2 * LIVE_HALF + parity]);
-    }
     int64_t len = step;
     if (chunk > 0 && movable * TAIL_FRACTION <= E && step <= INT64_MAX / TAIL_STRETCH)
       len = step * TAIL_STRETCH;
@@ -1350,6 +1338,13 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
       if (c->count_pending + add > COUNT_COPY_MAX) KMC_TRY(fold_counts(c, c->stream));
       c->count_pending += add;
     }
+    if (leave_idle) {
+      it.alive = c->d_live.p + LIVE_ALIVE + (launches & 1);
+      it.alive_next = c->d_live.p + LIVE_ALIVE + ((launches + 1) & 1);
+      a.n_alive = it.alive;
+    }
+    KMC_HIP(c, launch_exciton_keys(E, c->x_site.p, c->d_roff.p, it, c->d_keys.p, c->d_ids.p,
+                                   c->d_live.p, c->stream));
     size_t have = c->sort_tmp_bytes;
     KMC_HIP(c, hipcub::DeviceRadixSort::SortPairs(c->d_sort_tmp.p, have, c->d_keys.p,
                                                   c->d_keys.p + E, c->d_ids.p, c->d_ids.p + E,
@@ -1371,6 +1366,13 @@ static int run_hops(kmc_ctx* c, hop_args a, int64_t hops, int64_t chunk, bool co
     if (c->time_hops) KMC_HIP(c, hipEventRecord(c->hop_ev[2 * launches + 1], c->stream));
     done += sub;
     ++launches;
+    if (done < hops && live_check_due(launches)) {
+      int64_t live = 0, stuck = 0;
+      KMC_TRY(read_live(c, &live, &stuck));
+      if (live == 0) break;
+      movable = std::min(movable, live);
+      if (leave_idle) walked = std::min(walked, live + stuck);
+    }
   } while (done < hops);
   c->run_launches = launches;
   if (c->time_hops) {
@@ -1495,9 +1497,9 @@ int kmc_get_run_stats(kmc_ctx* c, int64_t* launches, int64_t* live_excitons) {
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   if (launches) *launches = c->run_launches;
   if (live_excitons) {
-    uint32_t n[LIVE_HALF];
-    KMC_TRY(copy_out(c, n, c->d_live.p + ((c->run_launches + 1) & 1) * LIVE_HALF, sizeof(n)));
-    *live_excitons = c->run_launches > 0 ? live_sum(n) : -1;
+    int64_t live = 0, stuck = 0;
+    KMC_TRY(read_live(c, &live, &stuck));
+    *live_excitons = c->run_launches > 0 ? live : -1;
   }
   return KMC_OK;
 }
@@ -1650,7 +1652,8 @@ struct kmc_ensemble {
   size_t sort_bytes = 0;
   int end_bit = 33;
   int64_t resort_hops = 625;
-  uint32_t* d_live = nullptr;    // excitons of all members able to hop after the last launch
+  uint32_t* d_live = nullptr;    // excitons of all members able to hop after the last launch, and
+                                 // those only trapped
   int64_t max_exc = 0;           // the largest member (bounds a launch's count per slot)
 };
 
@@ -1866,8 +1869,8 @@ int kmc_ensemble_create(int32_t n_networks, kmc_ctx* const* networks, kmc_ensemb
                                            m->d_ids, m->d_ids + ne, (int)ne, 0, m->end_bit,
                                            m->stream);
   if (e == hipSuccess) e = hipMalloc(&m->d_sort_tmp, std::max<size_t>(m->sort_bytes, 1));
-  if (e == hipSuccess) e = hipMalloc((void**)&m->d_live, sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemsetAsync(m->d_live, 0, sizeof(uint32_t), m->stream);
+  if (e == hipSuccess) e = hipMalloc((void**)&m->d_live, 2 * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMemsetAsync(m->d_live, 0, 2 * sizeof(uint32_t), m->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->d_wave_net, wave_net.data(), wave_net.size() * 2, hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->d_exc_net, exc_net.data(), exc_net.size() * 2, hipMemcpyHostToDevice, m->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(m->d_pbase, pbase.data(), n_networks * 8, hipMemcpyHostToDevice, m->stream);

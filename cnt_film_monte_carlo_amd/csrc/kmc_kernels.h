@@ -62,9 +62,9 @@ struct net_view {
   double velocity;
   const uint4* fly_table;   // per block line and heading: the leg a flight follows (k_fly_table)
   int32_t* fly_err;         // set when a flight exceeds FLY_MAX_PASSES site passes
-  // excitons still able to hop at the end of a launch (not trapped, t <= t_max), summed per
-  // wave; zeroed by the sort-key kernel ahead of every launch.  k_hop_rows spreads it over
-  // LIVE_SLOTS words, the other kernels use the first
+  // excitons still able to hop at the end of a launch (not trapped, t <= t_max), and in the next
+  // word those only trapped (v = 0), summed per wave; zeroed by the sort-key kernel ahead of every
+  // launch.  k_hop_rows spreads them over LIVE_SLOTS pairs of words, the other kernels use the first
   uint32_t* live;
 };
 
@@ -217,10 +217,10 @@ struct idle_test {
   uint32_t* alive;        // += the excitons not idle (zero on entry)
   uint32_t* alive_next;   // set to zero for the next launch
 };
-// Words of a live count and their distance: a cache line each.
+// Pairs of words of the live counts and their distance: a cache line each.
 constexpr int LIVE_SLOTS = 32, LIVE_STRIDE = 32;
 // keys[e] = first line of exciton e's block (idle excitons: 0xFFFFFFFF, after every line),
-// ids[e] = e; the LIVE_SLOTS words of live (the next launch's count) = 0
+// ids[e] = e; the LIVE_SLOTS pairs of live (the next launch's counts) = 0
 hipError_t launch_exciton_keys(int64_t n, const int32_t* site, const int64_t* roff,
                                const idle_test& it, uint32_t* keys, uint32_t* ids, uint32_t* live,
                                hipStream_t st);

@@ -467,7 +467,7 @@ __global__ __launch_bounds__(256) void k_exciton_keys(int64_t n, const int32_t* 
                                                       uint32_t* __restrict__ live) {
 #pragma clang fp contract(off)
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < LIVE_SLOTS) live[e * LIVE_STRIDE] = 0u;
+  if (e < LIVE_SLOTS) live[e * LIVE_STRIDE] = live[e * LIVE_STRIDE + 1] = 0u;
   if (e == 0 && it.alive_next) *it.alive_next = 0u;
   bool alive = false;
   if (e < n) {
@@ -930,6 +930,13 @@ __device__ __forceinline__ void fly_offset(const net_view& v, const flight_state
 }
 
 
+// Adds a wave's excitons to the counts at the end of a launch: b those that a further launch could
+// move, due those with t <= t_max.
+__device__ __forceinline__ void add_live(uint32_t* live, uint64_t b, uint64_t due) {
+  if (b != 0ull) atomicAdd(live, (uint32_t)__popcll(b));
+  if (due != b) atomicAdd(live + 1, (uint32_t)__popcll(due & ~b));
+}
+
 // The hop loop of one wave (v = 0), built around the cooperative row load: every lane takes part
 // in every row load, so the loop runs until no lane of the wave can hop; a lane without an
 // exciton (valid false) or whose exciton has stopped keeps loading some row.  Each iteration
@@ -1124,8 +1131,8 @@ __device__ __forceinline__ void hop_wave(const net_view& v, uint32_t e, bool val
   if (COUNT) cc.flush(cbase);
   if (v.live) {
     // excitons that a further launch could move (the budget aside)
-    const uint64_t b = __ballot(valid && live);
-    if (lane == 0u && b != 0ull) atomicAdd(v.live, (uint32_t)__popcll(b));
+    const uint64_t b = __ballot(valid && live), due = __ballot(valid && t <= t_max);
+    if (lane == 0u) add_live(v.live, b, due);
   }
   if (!valid) return;
   v.x.site[e] = (int32_t)site_now;
@@ -1801,10 +1808,9 @@ __device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool val
   }
   if (v.live) {
     // excitons that a further launch could move (the budget aside)
-    const uint64_t b = __ballot(valid && l == 0u && !trapped(n, gamma) && t <= t_max);
+    const uint64_t due = __ballot(valid && l == 0u && t <= t_max), b = due & __ballot(!trapped(n, gamma));
     // 8,192 waves ending together, one after another on one word, took 80 us of a launch
-    if (lane == 0u && b != 0ull)
-      atomicAdd(v.live + (blockIdx.x % LIVE_SLOTS) * LIVE_STRIDE, (uint32_t)__popcll(b));
+    if (lane == 0u) add_live(v.live + (blockIdx.x % LIVE_SLOTS) * LIVE_STRIDE, b, due);
   }
   if (!valid || l != 0u) return;
   v.x.site[e] = (int32_t)site;
@@ -1978,7 +1984,7 @@ __global__ __launch_bounds__(256) void k_ens_keys(int64_t n, const net_view* __r
                                                   uint32_t* __restrict__ ids,
                                                   uint32_t* __restrict__ live) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g == 0 && live) *live = 0u;
+  if (g == 0 && live) live[0] = live[1] = 0u;
   if (g >= n) return;
   const uint32_t k = exc_net[g];
   const net_view& v = nets[k];
