@@ -1826,9 +1826,9 @@ __device__ __forceinline__ void hop_rows(const net_view& v, uint32_t e, bool val
 }
 
 // Positions as in k_hop, blockDim.x / 16 excitons to a workgroup; the workgroups of an XCD take its
-// eighth of the order.  The departure counts of the lines around the workgroup's first exciton --
-// all lines of a small film -- go to a window of 32-bit LDS counters (a launch's hops cannot wrap
-// one: at most 2^32 departures per copy), the others to the XCD's copy.
+// eighth of the order.  The departure counts of the lines around the workgroup's first exciton go
+// to a window of 32-bit LDS counters (a launch's hops cannot wrap one: at most 2^32 departures per
+// copy), the others to the XCD's copy.
 constexpr uint32_t WIN_AHEAD = 8;  // 16-byte pieces of the window that a thread clears or reads at once
 
 template <bool COUNT, bool SAMPLE, bool TRACE>
@@ -2041,9 +2041,10 @@ hipError_t launch_hop_rows(hop_args a, int64_t walked, uint32_t n_lines, int n_c
   const int64_t grid = (groups + KMC_COUNT_COPIES - 1) / KMC_COUNT_COPIES * KMC_COUNT_COPIES;
   // the window takes what the workgroups that share a CU leave of its LDS, but no more than a
   // launch's hops pay for: a thread clears and flushes four lines at a time, one such turn per hop
-  // (one hop of one exciton on 300,000 sites: 56 us of clearing and flushing 39,000 lines one at a
-  // time by a single wave, as against a hop kernel of 5)
-  const int64_t paid = 4 * (int64_t)std::min<uint64_t>(a.hop_budget, 1u << 20) * bs;
+  // and 16 at most (one hop of one exciton on 300,000 sites: 56 us of clearing and flushing 39,000
+  // lines by a single wave, as against a hop kernel of 5; 1,000 excitons' 2,500 hops there 1.69 ms
+  // with 4,096 lines for that wave, 1.86 with 39,000)
+  const int64_t paid = 4 * (int64_t)std::min<uint64_t>(a.hop_budget, 16u) * bs;
   const int64_t share = CU_LDS / std::max<int64_t>(1, std::min<int64_t>(8, (grid + n_cu - 1) / n_cu)) - 1024;
   const int64_t batches = (int64_t)(bs / 64) * (int64_t)sizeof(batch_lds);
   a.n_lines = n_lines;

@@ -26,11 +26,12 @@ def film(kmc, nw):
     ctx.close()
 
 
-def _hop_us(ctx, excitons, hops, count):
+def _hop_us(ctx, excitons, hops, count, t_step=np.inf):
+    """Best hop-kernel time of a call of so many hops, or up to the next of a row of times."""
     ctx.inject(excitons)
     best = np.inf
-    for _ in range(12):
-        ctx.run(hops, count_sites=count)
+    for k in range(12):
+        ctx.run(hops, t_max=(k + 1) * t_step, count_sites=count)
         best = min(best, 1e3 * ctx.hop_time())
     return best
 
@@ -43,17 +44,18 @@ def test_many_waves_ending_together(film):
     assert film.run_stats() == (1, line + 1)
 
 
-def test_window_of_a_short_launch(kmc, nw):
-    """Departure counts of one hop on a film of far more lines than a window holds."""
+@pytest.mark.parametrize("n_exc,hops,t_step", [(1, 1, np.inf), (200, 1 << 40, 5e-9)])
+def test_window_of_a_short_launch(kmc, nw, n_exc, hops, t_step):
+    """Departure counts of a hop or a few on a film of far more lines than a window holds."""
     w = nw.film_large()
     w.net.n_tubes = 1500
     ctx = nw.make_context(w, nw.build_network(w), seed=5)
     ctx.set_rate_table(*nw.forster_tables(3))
     ctx.build_cells()
     ctx.build_rates(kmc.RATE_TABLE)
-    with_counts, without = (_hop_us(ctx, 1, 1, c) for c in (True, False))
-    say(f"one hop of one exciton on {ctx.n_sites} sites, with counts {with_counts:.1f} us, "
-        f"without {without:.1f} us")
+    with_counts, without = (_hop_us(ctx, n_exc, hops, c, t_step) for c in (True, False))
+    say(f"{n_exc} excitons on {ctx.n_sites} sites, {hops} hops or {t_step} s, with counts "
+        f"{with_counts:.1f} us, without {without:.1f} us")
     ctx.close()
     assert with_counts <= 3 * without
 
