@@ -1,6 +1,6 @@
 """Launches of a hop or a few with few excitons: the row-of-lanes kernel's fixed costs (the count of
-excitons that can still move, the window of departure counts) against launches without them, and the
-window's edges against the oracle."""
+excitons that can still move, the window of departure counts, a batch of 16 hops) against launches
+without them, and the edges of window and batch against the oracle."""
 import sys
 
 import numpy as np
@@ -77,3 +77,43 @@ def test_short_launches_match_oracle(kmc, orc, film, nw, n_exc, hops):
                  ("disp", ox.dsp)):
         assert np.array_equal(g[k], o), k
     assert np.array_equal(ctx.get_hop_counts(), ox.site_count)
+
+
+def test_a_hop_costs_less_than_a_batch(film):
+    one, batch = (_hop_us(film, 64, h, False) for h in (1, 16))
+    say(f"64 excitons: one hop {one:.1f} us, a batch of 16 {batch:.1f} us")
+    assert one <= 0.7 * batch
+
+
+@pytest.mark.parametrize("n_exc", [1, 6, 1030, 20000])
+@pytest.mark.parametrize("dwells", [0.3, 2.0, 4.5, 9.0])
+def test_short_times_match_oracle(kmc, orc, film, nw, n_exc, dwells):
+    """Runs up to times about as long as the first batch's four hops, with records and trace."""
+    say(f"{n_exc} excitons up to {dwells} dwells at a time")
+    ctx = film
+    ctx.inject(n_exc)
+    csr = ctx.get_csr()
+    ox = orc.Excitons(csr, nw.build_network(nw.film_small())["flags"], seed=61, n_excitons=n_exc)
+    step = dwells / float(np.mean(csr["gamma"]))
+    nt = min(n_exc, 50)
+    for q in (ctx, ox):
+        q.set_samples(5, 4 * step)
+        q.set_trace(nt, 200)
+    for k in range(4):
+        ctx.run(1 << 40, t_max=(k + 1) * step)
+        ox.run(1 << 40, t_max=(k + 1) * step)
+    g = ctx.get_excitons()
+    for k, o in (("site", ox.site), ("hops", ox.hops), ("hash", ox.hash), ("drains", ox.drains),
+                 ("disp", ox.dsp)):
+        assert np.array_equal(g[k], o), k
+    np.testing.assert_allclose(g["t_next"], ox.t_next, rtol=1e-12, atol=0)
+    assert np.array_equal(ctx.get_hop_counts(), ox.site_count)
+    s = ctx.get_samples()
+    assert np.array_equal(s["n_recorded"], ox.k_rec)
+    made = np.arange(5)[:, None] < ox.k_rec[None, :]
+    assert np.array_equal(s["disp"][made], ox.rec_disp[made])
+    tr = ctx.get_trace()
+    n_hops = np.minimum(ox.hops[:nt].astype(np.int64), 200)
+    assert np.array_equal(tr["n_hops"], n_hops)
+    kept = np.arange(200)[None, :] < n_hops[:, None]
+    assert np.array_equal(tr["sites"][kept], ox.tr_site[:nt][kept])
