@@ -41,6 +41,7 @@ constexpr int GEOM_BATCH = 65536;  // geometries per launch (one workgroup each)
 // kernel.
 constexpr int64_t SPLIT_BELOW = 4096;
 constexpr size_t PART_CAP = size_t(1) << 21;
+constexpr int MAX_HALF = 8;   // pairs of acceptor cells that the cell loop is unrolled for, at most
 constexpr int DONORS = 64;    // donor atoms per chunk: one per lane, the same in the four waves
 
 struct ex_state {
@@ -213,17 +214,17 @@ __device__ __forceinline__ double wave_sum4(const double2 (&v)[4], uint32_t lane
 //    centre times exp(+-i k_b m): their inverse distances enter as sum and difference, with one
 //    FMA each per k_b, and the centre's phase is applied once per atom.
 // Per atom pair at NK = 2 (the momenta 0, +-1, +-2) that is ~16 issue slots (4 of them the
-// hardware root) against 28 for the plain sum over atoms and momenta: 27,951 geometries of
-// (8,6) -> (7,5) at 300 K take 63.3 -> 39.5 ms
-// (the nine tables of three chiralities 1,416 -> 791 ms), one geometry 0.27 -> 0.036 ms.  Errors
-// against an 80-bit evaluation of the same sum stay at rounding, 2e-16 to 4e-16 on average.
+// hardware root) against 28 for the plain sum over atoms and momenta: with tubes of ten cells,
+// 27,951 geometries of (8,6) -> (7,5) at 300 K take 63.3 -> 39.5 ms (the nine tables of three
+// chiralities 1,416 -> 791 ms), one geometry 0.27 -> 0.036 ms.  Errors against an 80-bit evaluation
+// of the same sum stay at rounding, 2e-16 to 4e-16 on average.
 //
 // Donor atoms go in chunks of 64, one per lane; the four waves take a quarter of the unit cell's
 // atoms each and add their sums through LDS.  The chunk's share of J_ab = sum_i u_a(i) W_b(i) is
 // then summed over the lanes, four terms at a time, the waves taking turns.  Split launches run
 // one chunk per workgroup and leave its share in part[] for k_exact_finish, which adds the chunks
 // in the same order, so both launch shapes give the same bits.
-template <int NK, int HALF>
+template <int NK, int HALF, bool ODD>
 __global__ __launch_bounds__(256) void k_exact_rate(exact_args a, const double* __restrict__ rec,
                                                     const double* __restrict__ cell,
                                                     const int32_t* __restrict__ term_a,
@@ -278,20 +279,20 @@ __global__ __launch_bounds__(256) void k_exact_rate(exact_args a, const double* 
           }
         };
         if constexpr (HALF > 0) {
-          // read again for every atom (scalar loads that hit the cache): kept over the loop, the
-          // table would spill from scalar to vector registers
+          // read again for every atom (scalar loads that hit the cache) where the table, kept over
+          // the loop, would spill from scalar to vector registers
           int t = 0;
-          if constexpr (NK > 2) asm volatile("" : "+s"(t));
+          if constexpr (HALF * CS > 25) asm volatile("" : "+s"(t));
 #pragma unroll
           for (int p = 0; p < HALF; ++p) pair_of_cells(cell + t + p * CS);
         } else {
           for (int p = 0; p < a.half; ++p) pair_of_cells(cell + p * CS);
-          if (a.odd) {
-            const double r = rsqrt_f64(fma(dy, dy, across));
-            z0 += r;
+        }
+        if (HALF > 0 ? ODD : a.odd != 0) {
+          const double r = rsqrt_f64(fma(dy, dy, across));
+          z0 += r;
 #pragma unroll
-            for (int b = 0; b < NK; ++b) cs[b] += r;
-          }
+          for (int b = 0; b < NK; ++b) cs[b] += r;
         }
         w[0] += z0;
 #pragma unroll
@@ -385,14 +386,24 @@ __global__ void k_zero_rates(int64_t n, const int64_t* sel, double* out) {
   if (g < n) out[sel ? sel[g] : g] = 0.0;
 }
 
-// One pass over at most MAXK nonzero |k_b| (and k_b = 0).  Tubes of 10 unit cells, the length
-// every table of the reference is made for, take the unrolled cell loop.
-template <int NK>
+// One pass over at most MAXK nonzero |k_b| (and k_b = 0).  The kernel is made for every number of
+// acceptor cells up to 2 MAX_HALF + 1, its cell loop unrolled: 6 to 16 % less time than the loop, the
+// more the shorter the tube and the more momenta (8,000 geometries of (7,5) -> (9,7) at 300 K with 4,
+// 9, 10 and 17 cells 6.5 -> 5.6, 39.5 -> 34.1, 51.8 -> 45.2 and 236 -> 217 ms); longer tubes, of which
+// the loop is a small part, take the loop.
+template <int NK, int HALF, bool ODD>
+void launch_cells(const exact_args& a, dim3 g, hipStream_t st) {
+  hipLaunchKernelGGL((k_exact_rate<NK, HALF, ODD>), g, dim3(256), 0, st, a, a.rec, a.cell, a.term_a,
+                     a.term_b);
+}
+
+template <int NK, int HALF = 1>
 void launch_width(const exact_args& a, dim3 g, hipStream_t st) {
-  if (a.half == 5 && !a.odd)
-    hipLaunchKernelGGL((k_exact_rate<NK, 5>), g, dim3(256), 0, st, a, a.rec, a.cell, a.term_a, a.term_b);
-  else
-    hipLaunchKernelGGL((k_exact_rate<NK, 0>), g, dim3(256), 0, st, a, a.rec, a.cell, a.term_a, a.term_b);
+  if constexpr (HALF <= MAX_HALF) {
+    if (a.half != HALF) return launch_width<NK, HALF + 1>(a, g, st);
+    return a.odd ? launch_cells<NK, HALF, true>(a, g, st) : launch_cells<NK, HALF, false>(a, g, st);
+  }
+  launch_cells<NK, 0, false>(a, g, st);
 }
 
 hipError_t launch_pass(const exact_args& a, hipStream_t st) {
