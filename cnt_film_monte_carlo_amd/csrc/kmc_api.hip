@@ -1140,6 +1140,11 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   if (c->h_src.empty()) return fail(c, KMC_ERR_STATE, "kmc_inject: no source (injection) sites");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   const int64_t E = n_excitons;
+  // before anything changes: an injection that is refused leaves the excitons as they were
+  if (c->velocity > 0.0) KMC_TRY(fly_table(c, "kmc_inject"));
+  c->n_exc = 0;  // one that fails later leaves none
+  c->n_bins = c->bin0 = c->win_bins = 0;
+  c->n_trace = 0;
   KMC_TRY(dalloc(c, c->x_site, E));
   KMC_TRY(dalloc(c, c->x_t, E));
   KMC_TRY(dalloc(c, c->x_dx, E));
@@ -1164,14 +1169,13 @@ int kmc_inject(kmc_ctx* c, int64_t n_excitons) {
   KMC_HIP(c, launch_clear(clear, c->stream));
   c->count_pending = 0;
   c->run_launches = 0;
-  c->n_exc = E;
-  c->n_bins = c->bin0 = c->win_bins = 0;
-  c->n_trace = 0;
-  if (c->velocity > 0.0) KMC_TRY(fly_table(c, "kmc_inject"));
   c->exc_velocity = c->velocity;
-  KMC_HIP(c, launch_inject(excitons_of(c), c->d_blocks.p, c->d_src_roff.p,
-                           (uint32_t)c->h_src.size(), c->cfg.seed, c->stream));
+  exciton_arrays x = excitons_of(c);
+  x.n = E;
+  KMC_HIP(c, launch_inject(x, c->d_blocks.p, c->d_src_roff.p, (uint32_t)c->h_src.size(), c->cfg.seed,
+                           c->stream));
   KMC_HIP(c, hipStreamSynchronize(c->stream));
+  c->n_exc = E;
   return KMC_OK;
 }
 
