@@ -654,6 +654,12 @@ int mfail(int code, const std::string& m) {
   g_mlp_err = m;
   return code;
 }
+// The runtime's own record of the error is cleared: the next call's launches would report it again.
+int hip_mfail(hipError_t e, const char* who) {
+  (void)hipGetLastError();
+  return mfail(e == hipErrorNoDevice ? KMC_ERR_NODEVICE : KMC_ERR_HIP,
+               std::string(who) + ": " + hipGetErrorString(e));
+}
 
 }  // namespace
 
@@ -690,9 +696,7 @@ namespace {
 #define MLP_HIP(call)                                                                      \
   do {                                                                                     \
     const hipError_t e_ = (call);                                                          \
-    if (e_ != hipSuccess)                                                                  \
-      return mfail(e_ == hipErrorNoDevice ? KMC_ERR_NODEVICE : KMC_ERR_HIP,                \
-                   std::string(__func__) + ": " + hipGetErrorString(e_));                  \
+    if (e_ != hipSuccess) return hip_mfail(e_, __func__);                                  \
   } while (0)
 
 template <typename T>
@@ -707,9 +711,9 @@ int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 int ensure_cap(kmc_mlp* m, int64_t rows) {
   rows = round_up(std::max<int64_t>(rows, 128), 128);
   if (rows <= m->cap) return KMC_OK;
+  m->cap = 0;  // until all of it has grown
   MLP_HIP(grow(&m->X, rows * IN));
   MLP_HIP(grow(&m->tgt, rows));
-  m->cap = 0;
   MLP_HIP(grow(&m->XT, rows * IN));
   MLP_HIP(grow(&m->HT, rows * WD * NH));
   MLP_HIP(grow(&m->DT, rows * WD * NH));
@@ -836,6 +840,7 @@ hipError_t launch_infer(const infer_args& a, int n_cu, hipStream_t st) {
 int stage_geometry(kmc_mlp* m, int64_t n, const double* th, const double* z, const double* a1,
                    const double* a2) {
   if (n > m->geo_cap) {
+    m->geo_cap = 0;  // until all of it has grown
     MLP_HIP(grow(&m->d_geo, 4 * n));
     MLP_HIP(grow(&m->d_rate, n));
     MLP_HIP(grow(&m->d_flag, n));
@@ -952,7 +957,7 @@ int kmc_mlp_create(int32_t device, const kmc_mlp_domain* dom, kmc_mlp** out) {
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {
     kmc_mlp_destroy(m);
-    return mfail(KMC_ERR_HIP, std::string("kmc_mlp_create: ") + hipGetErrorString(e));
+    return hip_mfail(e, "kmc_mlp_create");
   }
   *out = m;
   return KMC_OK;
@@ -1207,7 +1212,7 @@ int kmc_mlp_train(kmc_mlp* m, int64_t n, const float* feat, const float* targets
   if (h_lp) (void)hipHostFree(h_lp);
   for (hipEvent_t ev : {done[0], done[1], uploaded})
     if (ev) (void)hipEventDestroy(ev);
-  if (e != hipSuccess) return mfail(KMC_ERR_HIP, std::string("kmc_mlp_train: ") + hipGetErrorString(e));
+  if (e != hipSuccess) return hip_mfail(e, "kmc_mlp_train");
   if (elapsed_ms)
     *elapsed_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return KMC_OK;
