@@ -225,6 +225,7 @@ int fail(kmc_ctx* c, int code, const std::string& msg) {
 }
 
 int hip_fail(kmc_ctx* c, hipError_t e, const char* where) {
+  (void)hipGetLastError();  // the next call's launches would report it again
   std::string m = std::string(where) + ": " + hipGetErrorString(e);
   return fail(c, KMC_ERR_HIP, m);
 }
@@ -250,6 +251,7 @@ int dalloc(kmc_ctx* c, dbuf<T>& b, size_t n) {
   hipError_t e = hipMalloc((void**)&b.p, n * sizeof(T));
   if (e != hipSuccess) {
     b.p = nullptr;
+    (void)hipGetLastError();
     return fail(c, KMC_ERR_ALLOC, "hipMalloc of " + std::to_string(n * sizeof(T)) +
                                       " bytes failed: " + hipGetErrorString(e));
   }
@@ -1192,6 +1194,7 @@ static int set_samples(kmc_ctx* c, int32_t n_bins, double t_sample_max, int32_t 
     return fail(c, KMC_ERR_ARG, std::string(who) + ": need 1 <= window_bins <= n_bins");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
   const size_t nrec = (size_t)(n_bins > 0 ? window : 0) * c->n_exc;
+  c->n_bins = c->bin0 = c->win_bins = 0;  // no grid, should one not fit
   KMC_TRY(dalloc(c, c->r_dx, nrec));
   KMC_TRY(dalloc(c, c->r_dy, nrec));
   KMC_TRY(dalloc(c, c->r_dz, nrec));
@@ -1261,6 +1264,7 @@ int kmc_set_trace(kmc_ctx* c, int64_t n_trace, int64_t max_hops) {
   if (n_trace < 0 || max_hops < 0 || n_trace > c->n_exc)
     return fail(c, KMC_ERR_ARG, "kmc_set_trace: need 0 <= n_trace <= n_excitons, max_hops >= 0");
   KMC_HIP(c, hipSetDevice(c->cfg.device));
+  c->n_trace = 0;  // no trace, should one not fit
   KMC_TRY(dalloc(c, c->tr_site, (size_t)n_trace * max_hops));
   KMC_TRY(dalloc(c, c->tr_time, (size_t)n_trace * max_hops));
   KMC_TRY(dalloc(c, c->tr_n, n_trace));
@@ -1905,6 +1909,7 @@ int kmc_ensemble_create(int32_t n_networks, kmc_ctx* const* networks, kmc_ensemb
   if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
   if (e != hipSuccess) {
     kmc_ensemble_destroy(m);
+    (void)hipGetLastError();
     return efail(KMC_ERR_HIP, std::string("kmc_ensemble_create: ") + hipGetErrorString(e));
   }
   *out = m;
@@ -2160,6 +2165,7 @@ int kmc_contact_init(kmc_ctx* c, int32_t n_seg, int64_t c1_pop, int64_t c2_pop, 
     return fail(c, KMC_ERR_ARG, "kmc_contact_init: a contact holding particles has no sites");
   if (total > capacity || c1_pop + c2_pop > capacity)
     return fail(c, KMC_ERR_CAPACITY, "kmc_contact_init: capacity below the populations");
+  c->c_on = false;  // until all of it stands
   c->c_nseg = n_seg;
   c->c_pop[0] = c1_pop;
   c->c_pop[1] = c2_pop;

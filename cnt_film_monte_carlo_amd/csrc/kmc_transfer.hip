@@ -432,6 +432,7 @@ hipError_t launch_pass(const exact_args& a, hipStream_t st) {
 
 thread_local std::string g_tr_err;
 int tfail(int code, const std::string& m) {
+  if (code == KMC_ERR_HIP) (void)hipGetLastError();  // the next call's launches would report it again
   g_tr_err = m;
   return code;
 }
