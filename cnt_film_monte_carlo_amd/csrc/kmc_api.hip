@@ -130,7 +130,7 @@ struct kmc_ctx {
   dbuf<int64_t> d_cls_start, d_sel;
   dbuf<uint8_t> d_mlp_flag;  // surrogate flags of the last surrogate build
   dbuf<uint8_t> d_read;      // read-backs: the caller's layout of one chunk
-  // drift along the tubes (particle::fly): velocity [m/s], links as block lines, error word
+  // drift along the tubes (particle::fly): velocity [m/s], the flights' legs, error word
   double velocity = 0.0;      // set by kmc_set_velocity
   double exc_velocity = 0.0;  // the velocity of the injected excitons (fixed by kmc_inject)
   dbuf<uint4> d_fly_table;    // of this film's rows when fly_ok
@@ -2019,11 +2019,12 @@ contact_slots contact_buf(kmc_ctx* c, int b) {
 // The order in which a step's threads take the live slots.  Slots sort by the eighth of the film
 // their site lies in (the eighths of the sorted slots go to the eight XCDs, so each XCD's L2
 // serves one compact region), then by the site's chirality, then by the site's row in the eighth,
-// to as many of the row's leading bits as eight bits have left.  The chirality sets the rates a particle meets along its tube, so the particles of
-// one wave make similar numbers of hops in a step and fewer of its lanes idle while its last
-// particle hops.  Finer rows gain nothing: with 1 M particles on 625k sites of three chiralities
-// the step kernel takes 655 us with 8 key bits, 685 with 16 and 687 with all 28; with one
-// chirality 6.5 ms at 8 bits, 6.9 at 11 and 7.0 at 16.
+// to as many of the row's leading bits as eight bits have left.  The chirality sets the rates a
+// particle meets along its tube, so the particles of one wave make similar numbers of hops in a
+// step and fewer of its lanes idle while its last particle hops.  Finer rows gain nothing: with 1 M
+// particles on 625k sites of three chiralities the step kernel takes 640 us for 40 mean dwells and
+// 1,385 us for 100 with 8 key bits, 682 and 1,444 with all 28 (one chirality 610 and 1,280, 652 and
+// 1,347), and the same 6.73 ms for 547 hops a particle.
 contact_key_layout contact_key_layout_of(const kmc_ctx* c, uint32_t lines) {
   const auto bits = [](uint32_t v) {  // bits that hold the values [0, v]
     int b = 1;

@@ -872,8 +872,9 @@ __global__ __launch_bounds__(256) void k_fly_table(int64_t n, const int32_t* __r
 // Flight of duration tau; `leg` is the one at (f.R, f.heading) and follows them.  A site reached on
 // the way becomes the current site; a drain site counts a drain and re-injects on a source site
 // (draw of stream STREAM_FLY_DRAIN + j for the j-th drain of this flight, hop counter h), keeping
-// the displacement, and the flight goes on from there, as the reference's next 1 fs step would.  False when the flight would pass more
-// than FLY_MAX_PASSES sites (the state is then left where the bound stopped it).
+// the displacement, and the flight goes on from there, as the reference's next 1 fs step would.
+// False when the flight would pass more than FLY_MAX_PASSES sites (the state is then left where the
+// bound stopped it).
 __device__ __forceinline__ bool fly(const net_view& v, flight_state& f, fly_leg& leg, double tau,
                                     uint32_t e, uint64_t h) {
 #pragma clang fp contract(off)
@@ -928,7 +929,6 @@ __device__ __forceinline__ void fly_offset(const net_view& v, const flight_state
   oy = min_image((double)leg.y - (double)f.y, v.half_per[1]) * q;
   oz = min_image((double)leg.z - (double)f.z, v.half_per[2]) * q;
 }
-
 
 // Adds a wave's excitons to the counts at the end of a launch: b those that a further launch could
 // move, due those with t <= t_max.
@@ -1505,12 +1505,12 @@ __global__ __launch_bounds__(256, 4) void k_hop(hop_args a) {
 // Few excitons (k_hop_rows).  With less than a wave per SIMD, k_hop's iteration takes its own
 // latency: LDS round trips, lane exchanges, ten Philox rounds and a logarithm one after another
 // in a single wave, ~3,500 cycles per hop, of which the row load itself is hidden; the chip is
-// idle.  What bounds this form is the same chain, shortened: ~1,300 cycles per hop, a quarter of
-// them the row's L2 latency (1,000 excitons on 5,000 sites, 1,250 hops: 2.19 -> 0.74 ms; 16,384
-// excitons on 76,543 sites: 2.03 -> 0.94 ms).  Each
-// exciton has a row of 16 lanes, four excitons to a wave.  The lanes hold the exciton's 128-byte
-// block line between them (8 bytes each), so a selection is a comparison per lane and a count of
-// the ballot's bits, with DPP row broadcasts instead of LDS staging.  Only the chain that leads
+// idle.  What bounds this form is the same chain, shortened: ~1,100 cycles per hop, a quarter of
+// them the row's L2 latency (76,543 sites, 1,250 hops with counts: 1,000 excitons 1.86 -> 0.57 ms,
+// 16,384 excitons 1.92 -> 0.84 ms).  Each exciton has a row of 16 lanes, four excitons to a wave.
+// The lanes hold the exciton's 128-byte block line between them (8 bytes each), so a selection is a
+// comparison per lane and a count of the ballot's bits, with DPP row broadcasts instead of LDS
+// staging.  Only the chain that leads
 // from row to row runs hop by hop; a batch of ROW_BATCH = 16 hops then has its draws, dwells and
 // displacements computed side by side, lane j for hop j, and folded into the exciton's sums in
 // hop order (the operations and their order are those of hop_wave, so are the bits).  Hops
@@ -2040,9 +2040,10 @@ hipError_t launch_hop(const hop_args& a, bool count, bool sample, bool trace, bo
 
 constexpr int64_t CU_LDS = 160 * 1024;
 
-// A row of lanes per exciton pays up to 128 excitons per CU: 1,250 hops on 76,543 sites take
-// 0.72 / 0.94 / 1.53 / 1.91 / 3.3 ms at 1,000 / 16,384 / 24,576 / 32,768 / 50,000 excitons (a wave
-// round per 16,384), k_hop's lane per exciton 1.93 / 2.03 / 2.07 / 2.10 / 2.14 ms.
+// A row of lanes per exciton pays up to 128 excitons per CU, two rounds of its waves: 1,250 hops with
+// counts on 76,543 sites take 0.57 / 0.84 / 1.42 / 1.81 ms at 1,000 / 16,384 / 24,576 / 32,768
+// excitons, k_hop's lane per exciton 1.86 / 1.92 / 1.96 / 1.94 ms; at 32,768 on 5,000 sites 1.75 and
+// 2.05, on 50,000 1.74 and 1.94, on 624,739 1.79 and 2.12.
 bool hop_rows_pays(int64_t walked, int n_cu) { return walked <= (int64_t)128 * n_cu; }
 
 hipError_t launch_hop_rows(hop_args a, int64_t walked, uint32_t n_lines, int n_cu, bool count,
@@ -2323,7 +2324,7 @@ __global__ __launch_bounds__(256) void k_contact_fly(contact_args a) {
 // The order in which a step takes the live slots: by contact_key, ORDER_BINS values, in two
 // launches over tiles of SCAN_TILE slots.  k_contact_keys counts every key's slots, k_contact_order
 // gives each tile its places behind the counts of the keys below.  Slots of one key stand in no
-// particular order (it changes no result).  At 1 M slots the pair takes 30 us, a library radix sort
+// particular order (it changes no result).  At 1 M slots the pair takes 35 us, a library radix sort
 // of the same 8-bit keys with their kernel 75; at 52,000 slots 15 us for 43 (seven launches).
 __global__ __launch_bounds__(SCAN_THREADS) void k_contact_keys(const int64_t* n_live,
                                                                const int32_t* __restrict__ site,
