@@ -30,7 +30,7 @@ def _hop_us(ctx, excitons, hops, count, t_step=np.inf):
     """Best hop-kernel time of a call of so many hops, or up to the next of a row of times."""
     ctx.inject(excitons)
     best = np.inf
-    for k in range(12):
+    for k in range(40):
         ctx.run(hops, t_max=(k + 1) * t_step, count_sites=count)
         best = min(best, 1e3 * ctx.hop_time())
     return best
